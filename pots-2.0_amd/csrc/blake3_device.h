@@ -125,4 +125,81 @@ __device__ __forceinline__ void b3_parent_cv(const uint32_t l[8], const uint32_t
   b3_compress_cv(iv, m, 0, 64, B3_PARENT | flags, out);
 }
 
+// ---- one compression on four lanes -----------------------------------------------------------
+//
+// A quad of consecutive lanes holds the state by columns: lane q has v[q], v[4+q], v[8+q] and
+// v[12+q], so a round's four column G's are one G on every lane, and its four diagonal G's one
+// more after lanes pass b, c and d round the quad (DPP moves on the VALU). A lane issues about
+// 250 VALU instructions per compression against 690 with one lane per compression: a third of
+// the time when the work is a few chunks or nodes whose latency counts, a third more issue
+// in total, so wide work keeps a lane each.
+//
+// The quad's 16 message words lie in LDS; each lane reads the four of a round it needs through
+// its offsets into the block (b3_quad_schedule, made once per kernel).
+
+struct B3Quad {
+  uint32_t off[28];  // word of the block for round r: off[4r], off[4r+1] columns, +2, +3 diagonals
+};
+
+// Words s of the schedule's rows for lanes 0..3, a nibble each.
+__device__ __forceinline__ uint32_t b3_nibble(uint32_t s0, uint32_t s1, uint32_t s2, uint32_t s3,
+                                              uint32_t q) {
+  return ((s0 | s1 << 4 | s2 << 8 | s3 << 12) >> (4 * q)) & 15u;
+}
+
+__device__ __forceinline__ B3Quad b3_quad_schedule(uint32_t q) {
+  B3Quad t;
+#define POTS_B3_SCHED(r, s0, s1, s2, s3, s4, s5, s6, s7, s8, s9, s10, s11, s12, s13, s14, s15) \
+  t.off[4 * r] = b3_nibble(s0, s2, s4, s6, q);                                               \
+  t.off[4 * r + 1] = b3_nibble(s1, s3, s5, s7, q);                                           \
+  t.off[4 * r + 2] = b3_nibble(s8, s10, s12, s14, q);                                        \
+  t.off[4 * r + 3] = b3_nibble(s9, s11, s13, s15, q)
+  POTS_B3_SCHED(0, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
+  POTS_B3_SCHED(1, 2, 6, 3, 10, 7, 0, 4, 13, 1, 11, 12, 5, 9, 14, 15, 8);
+  POTS_B3_SCHED(2, 3, 4, 10, 12, 13, 2, 7, 14, 6, 5, 9, 0, 11, 15, 8, 1);
+  POTS_B3_SCHED(3, 10, 7, 12, 9, 14, 3, 13, 15, 4, 0, 11, 2, 5, 8, 1, 6);
+  POTS_B3_SCHED(4, 12, 13, 9, 11, 15, 10, 14, 8, 7, 2, 5, 3, 0, 1, 6, 4);
+  POTS_B3_SCHED(5, 9, 14, 11, 5, 8, 12, 15, 1, 13, 3, 0, 10, 2, 6, 4, 7);
+  POTS_B3_SCHED(6, 11, 15, 5, 0, 1, 9, 8, 6, 14, 10, 2, 12, 3, 4, 7, 13);
+#undef POTS_B3_SCHED
+  return t;
+}
+
+// Lane q of each quad receives lane (q + N) mod 4's value.
+template <int N>
+__device__ __forceinline__ uint32_t quad_next(uint32_t v) {
+  constexpr int perm = N == 1 ? 0x39 : N == 2 ? 0x4E : 0x93;
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, perm, 0xF, 0xF, false);
+}
+
+// One compression of the block `m` (16 words in LDS) under the chaining value (lane q holds
+// words q and 4 + q in lo, hi), which it replaces. `tail` is lane q's word 12 + q of the
+// state: the counter's low and high words, the block length, the flags.
+__device__ __forceinline__ void b3_quad_compress(const B3Quad& t, const uint32_t* m, uint32_t q,
+                                                 uint32_t tail, uint32_t& lo, uint32_t& hi) {
+  uint32_t a = lo, b = hi, d = tail;
+  uint32_t c = q == 0 ? B3_IV0 : q == 1 ? B3_IV1 : q == 2 ? B3_IV2 : B3_IV3;
+#pragma unroll
+  for (int r = 0; r < 7; r++) {
+    const uint32_t m0 = m[t.off[4 * r]], m1 = m[t.off[4 * r + 1]];
+    const uint32_t m2 = m[t.off[4 * r + 2]], m3 = m[t.off[4 * r + 3]];
+    POTS_B3_G(a, b, c, d, m0, m1);
+    b = quad_next<1>(b);
+    c = quad_next<2>(c);
+    d = quad_next<3>(d);
+    POTS_B3_G(a, b, c, d, m2, m3);
+    b = quad_next<3>(b);
+    c = quad_next<2>(c);
+    d = quad_next<1>(d);
+  }
+  lo = a ^ c;
+  hi = b ^ d;
+}
+
+// Lane q's words q and 4 + q of the unkeyed IV.
+__device__ __forceinline__ void b3_quad_iv(uint32_t q, uint32_t& lo, uint32_t& hi) {
+  lo = q == 0 ? B3_IV0 : q == 1 ? B3_IV1 : q == 2 ? B3_IV2 : B3_IV3;
+  hi = q == 0 ? B3_IV4 : q == 1 ? B3_IV5 : q == 2 ? B3_IV6 : B3_IV7;
+}
+
 }  // namespace pots

@@ -4,9 +4,9 @@
 // Reference: verification/commitment/native.c:171-259 (pots_hash_leaves, hash_leaf,
 // leaf_worker) and verification/commitment/leaves.py:312-437 (the batching around it).
 //
-// Decomposition. Every leaf's message is cut into BLAKE3's 1 KiB chunks; one lane compresses
-// one chunk (up to 16 blocks) and writes its chaining value, or the digest itself when the
-// leaf is a single chunk. The chunk CVs of a leaf form BLAKE3's tree, which has the RFC 6962
+// Decomposition. Every leaf's message is cut into BLAKE3's 1 KiB chunks; one lane (or, in a
+// plan of few chunks, four) compresses one chunk (up to 16 blocks) and writes its chaining
+// value, or the digest itself when the leaf is a single chunk. The chunk CVs of a leaf form BLAKE3's tree, which has the RFC 6962
 // shape (a run of n > 1 chunks splits at the largest power of two below n), so it is reduced
 // level by level: level l+1 node j is the parent of level-l nodes 2j and 2j+1, or node 2j
 // itself when it has no sibling. The node that covers the whole leaf gets the ROOT flag.
@@ -89,17 +89,18 @@ struct LevelEntry {     // one leaf with >= 2 nodes at the input level of one fo
 static_assert(sizeof(LevelEntry) == 32, "LevelEntry layout");
 
 constexpr int kThreads = 256;
-// Consecutive chunks one lane hashes in a row: each chunk after the first takes its first
-// bytes from the unit its predecessor's last pair loaded, so the 128-byte line before a 1 KiB
-// boundary is read once, not again by the next chunk.
-#ifndef POTS_CHUNK_RUN
-#define POTS_CHUNK_RUN 4
-#endif
-constexpr uint32_t kRun = POTS_CHUNK_RUN;
+// Consecutive chunks one lane hashes in a row, at most: each chunk after the first takes its
+// first bytes from the unit its predecessor's last pair loaded, so the 128-byte line before a
+// 1 KiB boundary is read once, not again by the next chunk.
+constexpr uint32_t kRun = 4;
+// Chunks per wave of the four-lane chunk kernel, and the words of one chunk's place in its LDS
+// (1 KiB and 16 bytes: neighbouring quads' words sit 4 banks apart).
+constexpr uint32_t kQuadChunks = 16, kQuadStride = 260;
 // Tree levels one launch of level_kernel reduces.
 constexpr uint32_t kFold = 3;
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4w __attribute__((ext_vector_type(4), aligned(4)));  // word aligned
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
 // The NaN/Inf test of a chunk's payload words, one accumulator per lane: `mask` keeps each
@@ -427,13 +428,15 @@ __device__ __forceinline__ void hash_chunk(const LeafDesc& d, const uint32_t* __
 }
 
 // A chunk order: entry e covers slots first[e] .. first[e + 1] of leaf leaf[e], and the
-// entries of block b's slots (kThreads of them) lie in blk_ent[b] .. blk_ent[b + 1].
+// entries of block b's slots (kThreads of them; kQuadChunks for the four-lane kernel) lie in
+// blk_ent[b] .. blk_ent[b + 1].
 struct Order {
   const uint64_t* __restrict__ first;
   const uint32_t* __restrict__ leaf;
   const uint32_t* __restrict__ blk_ent;
   uint64_t n_slots;   // slots of the order
-  uint32_t n_blocks;  // ceil(n_slots / kThreads)
+  uint32_t n_blocks;  // ceil(n_slots / slots per block)
+  uint32_t run;       // chunks per slot (the plain order)
 };
 
 __device__ __forceinline__ uint32_t order_entry(const Order& od, uint64_t g, uint32_t blk) {
@@ -472,7 +475,7 @@ __device__ __forceinline__ void hash_run(const LeafDesc& d, const uint32_t* __re
 }
 
 // Every chunk of the unfused leaves: slot g of the plain order is run g − first[e] of leaf
-// leaf[e], its chunks kRun·(g − first[e]) onwards (slots past a leaf's runs are idle). Block b
+// leaf[e], its chunks run·(g − first[e]) onwards (slots past a leaf's runs are idle). Block b
 // hashes slot blocks b, b + gridDim.x, ... so a grid smaller than the order holds a bounded
 // share of the GPU and leaves the rest to kernels on other streams.
 __global__ __launch_bounds__(kThreads) void chunk_kernel(
@@ -485,9 +488,9 @@ __global__ __launch_bounds__(kThreads) void chunk_kernel(
     const uint32_t e = order_entry(od, g, blk);
     const uint32_t i = od.leaf[e];
     const LeafDesc d = leaves[i];
-    const uint64_t c0 = (g - od.first[e]) * kRun;
+    const uint64_t c0 = (g - od.first[e]) * od.run;
     if (c0 >= d.n_chunks) continue;
-    const uint64_t c1 = min<uint64_t>(c0 + kRun, d.n_chunks);
+    const uint64_t c1 = min<uint64_t>(c0 + od.run, d.n_chunks);
     Fin fin(d.kind);
     switch ((uint32_t)((d.payload - d.head_len) >> 2) & 3u) {
       case 0: hash_run<0>(d, head, i, c0, c1, fin, cv_out, digests); break;
@@ -495,6 +498,89 @@ __global__ __launch_bounds__(kThreads) void chunk_kernel(
       case 2: hash_run<2>(d, head, i, c0, c1, fin, cv_out, digests); break;
       default: hash_run<3>(d, head, i, c0, c1, fin, cv_out, digests); break;
     }
+    if (fin.bad()) atomicMin(first_bad, i);
+  }
+}
+
+// The chunks of the unfused leaves on four lanes each (b3_quad_compress), for plans of few
+// chunks, where a chunk's sixteen serial compressions are the call's latency and most of the
+// GPU would idle. A wave hashes kQuadChunks chunks. The quad's lanes load the chunk's sixteen
+// blocks 16 bytes a lane, all in flight at once, into the wave's LDS: groups wholly inside the
+// payload (past the header) as they lie, at word alignment, the loads of the others clamped
+// into the payload and their words then rewritten one by one (header words, zeros past the
+// end). No other wave touches that LDS, so the wave's own program order is the only ordering
+// it needs.
+__global__ __launch_bounds__(64) void chunk_kernel_quad(
+    const LeafDesc* __restrict__ leaves, Order od, const uint32_t* __restrict__ head,
+    uint32_t* __restrict__ cv_out, uint32_t* __restrict__ digests,
+    uint32_t* __restrict__ first_bad) {
+  __shared__ __align__(16) uint32_t s_msg[kQuadChunks * kQuadStride];
+  const uint32_t q = threadIdx.x & 3, slot = threadIdx.x >> 2;
+  uint32_t* const msg = s_msg + slot * kQuadStride;
+  const B3Quad sched = b3_quad_schedule(q);
+  for (uint32_t blk = blockIdx.x; blk < od.n_blocks; blk += gridDim.x) {
+    const uint64_t g = (uint64_t)blk * kQuadChunks + slot;
+    if (g >= od.n_slots) continue;
+    const uint32_t e = order_entry(od, g, blk);
+    const uint32_t i = od.leaf[e];
+    const LeafDesc d = leaves[i];
+    const uint64_t c = g - od.first[e];  // < n_chunks: a slot per chunk
+    const uint64_t H = d.head_len, L = H + d.len, cstart = c * 1024u;
+    const uint64_t from = max<uint64_t>(H, d.fin_from);  // payload words begin here
+    const uint64_t cbytes = min<uint64_t>(1024u, L - cstart);
+    const uint32_t nb = max(1u, (uint32_t)((cbytes + 63) / 64));
+    Fin fin(d.kind);
+    if (d.len >= 16) {
+      const uint64_t last = (d.len - 16) & ~uint64_t(3);
+      u32x4 w[16];
+#pragma unroll
+      for (uint32_t b = 0; b < 16; b++) {
+        const uint64_t o = cstart + 64u * b + 16u * q;
+        w[b] = gload<u32x4w>(reinterpret_cast<const char*>(d.payload) +
+                             (o < H ? 0 : min<uint64_t>(o - H, last)));
+      }
+#pragma unroll
+      for (uint32_t b = 0; b < 16; b++) {
+        const uint64_t o = cstart + 64u * b + 16u * q;
+        if (o >= from && o + 16 <= L)
+#pragma unroll
+          for (int t = 0; t < 4; t++) fin.add(w[b][t]);
+        *reinterpret_cast<u32x4*>(msg + 16 * b + 4 * q) = w[b];
+      }
+    }
+    if (cstart < from || cstart + 1024 > L || d.len < 16) {
+      for (uint32_t b = 0; b < nb; b++) {
+        const uint64_t o = cstart + 64u * b + 16u * q;
+        if (o >= from && o + 16 <= L && d.len >= 16) continue;
+#pragma unroll
+        for (uint32_t t = 0; t < 4; t++) {
+          const uint64_t at = o + 4u * t;
+          uint32_t mw = 0;
+          if (at < H) {
+            mw = gload<uint32_t>(head + d.head_word + (uint32_t)(at >> 2));
+          } else if (at < L) {
+            mw = gload<uint32_t>(reinterpret_cast<const char*>(d.payload) + (at - H));
+            if (L - at < 4) mw &= (1u << (8 * (uint32_t)(L - at))) - 1u;
+            if (at >= d.fin_from) fin.add(mw);
+          }
+          msg[16 * b + 4 * q + t] = mw;
+        }
+      }
+    }
+    const bool root = d.n_chunks == 1;
+    uint32_t lo, hi;
+    b3_quad_iv(q, lo, hi);
+#pragma unroll 1
+    for (uint32_t b = 0; b < nb; b++) {
+      const uint32_t blen = min<uint32_t>(64u, (uint32_t)cbytes - 64u * b);
+      uint32_t flags = b == 0 ? B3_CHUNK_START : 0u;
+      if (b + 1 == nb) flags |= B3_CHUNK_END | (root ? B3_ROOT : 0u);
+      const uint32_t tail = q == 0 ? (uint32_t)c : q == 1 ? 0u : q == 2 ? blen : flags;
+      b3_quad_compress(sched, msg + 16 * b, q, tail, lo, hi);
+    }
+    uint32_t* out = root ? digests + 8ull * i : cv_out + 8ull * (d.cv_first + c);
+    gstore<uint32_t>(out + q, lo);
+    gstore<uint32_t>(out + 4 + q, hi);
     if (fin.bad()) atomicMin(first_bad, i);
   }
 }
@@ -642,6 +728,7 @@ struct LeafPlan {
   uint64_t fused_msg = 0, fused_chunks = 0, fused_records = 0;  // per run of the fused kernel
   FuseDesc* d_fuse = nullptr;
   Order plain{}, fused{};  // the two kernels' chunk orders (device tables)
+  bool quad = false;       // the plain order is chunk_kernel_quad's
   bool owned = false;
   char* base = nullptr;  // one device allocation: metadata, then workspace
   size_t total = 0;
@@ -664,20 +751,21 @@ struct OrderHost {
   std::vector<uint32_t> blk_ent;
   uint64_t n_slots = 0;
   uint32_t n_blocks = 0;
+  uint32_t run = 1;  // chunks per slot (the plain order)
   void add(uint32_t i, uint64_t slots) {
     first.push_back(n_slots);
     leaf.push_back(i);
     n_slots += slots;
   }
-  bool finish() {
+  bool finish(uint32_t per_block) {
     first.push_back(n_slots);
-    const uint64_t nb = (n_slots + kThreads - 1) / kThreads;
+    const uint64_t nb = (n_slots + per_block - 1) / per_block;
     if (nb >= 0x7FFFFFFFull || leaf.size() >= 0xFFFFFFFFull) return false;
     n_blocks = (uint32_t)nb;
     blk_ent.assign(n_blocks + 1, 0);
     size_t e = 0;
     for (uint32_t b = 0; b < n_blocks; b++) {
-      const uint64_t g = (uint64_t)b * kThreads;
+      const uint64_t g = (uint64_t)b * per_block;
       while (first[e + 1] <= g) e++;
       blk_ent[b] = (uint32_t)e;
     }
@@ -687,12 +775,12 @@ struct OrderHost {
 };
 
 // A fused leaf's chunk order: T classes (chunk c in class c mod T, T = lcm(row bytes, 1024) /
-// 1024, so a class's chunks start at one offset in the row). A lane's run is RC = min(T, kRun)
-// consecutive classes of one period, or, when T < kRun, PG = kRun / T whole periods; the runs
+// 1024, so a class's chunks start at one offset in the row). A lane's run is RC = min(T, lrun)
+// consecutive classes of one period, or, when T < lrun, PG = lrun / T whole periods; the runs
 // of one class range get Q lanes, the number of runs rounded up to 64. Fusing is declined when
 // the padding would exceed 1/16 of the chunks even with runs of one chunk.
-static bool fuse_shape(uint64_t msg_bytes, uint32_t row_bytes, uint32_t* T, uint32_t* Q,
-                       uint32_t* run, uint32_t* nf, uint64_t* slots) {
+static bool fuse_shape(uint64_t msg_bytes, uint32_t row_bytes, uint32_t lrun, uint32_t* T,
+                       uint32_t* Q, uint32_t* run, uint32_t* nf, uint64_t* slots) {
   const uint64_t n_chunks = (msg_bytes + 1023) / 1024;
   const uint64_t f = msg_bytes % 1024 != 0 && msg_bytes % 1024 < 128 ? n_chunks - 1 : n_chunks;
   uint64_t a = row_bytes, b = 1024;
@@ -703,9 +791,9 @@ static bool fuse_shape(uint64_t msg_bytes, uint32_t row_bytes, uint32_t* T, uint
   }
   const uint64_t t = (uint64_t)row_bytes / a;  // lcm / 1024
   const uint64_t periods = (f + t - 1) / t;
-  // Runs of kRun chunks, or, where rounding their count up to 64 pads too much (a leaf of
-  // few periods with T < kRun), runs of one chunk.
-  const uint64_t shapes[2][2] = {{std::min<uint64_t>(t, kRun), t >= kRun ? 1 : kRun / t},
+  // Runs of lrun chunks, or, where rounding their count up to 64 pads too much (a leaf of
+  // few periods with T < lrun), runs of one chunk.
+  const uint64_t shapes[2][2] = {{std::min<uint64_t>(t, lrun), t >= lrun ? 1 : lrun / t},
                                  {1, 1}};
   for (const auto& sh : shapes) {
     const uint64_t rc = sh[0], pg = sh[1];
@@ -721,6 +809,19 @@ static bool fuse_shape(uint64_t msg_bytes, uint32_t row_bytes, uint32_t* T, uint
   }
   return false;
 }
+
+// How a plan's chunks are cut into work, by their count (one leaf of each size, MI355X, the
+// chunk kernel alone; four chunks a lane / one a lane / four lanes a chunk, us):
+//   6 KiB 102 / 40 / 19;  16 MiB 101 / 37 / 19;  32 MiB 110 / 35 / 26;  48 MiB 111 / 41 / 46;
+//   64 MiB 109 / 42 / 54;  256 MiB 123 / 104;  384 MiB 200 / 155;  512 MiB 209 / 202;
+//   1 GiB 382 / 385 / 551;  4 GiB 1444 / 1410 / 2069
+// A chunk is sixteen compressions, each needing the last one's output, so below a wave for
+// every SIMD (64 Ki lanes) the time is one lane's serial chain: short runs, and lanes in
+// quads while those still find idle SIMDs. Once every SIMD has eight waves the runs cost
+// nothing and save the second read of the lines between chunks.
+constexpr uint64_t kQuadMost = 32768;      // chunks hashed by four lanes each, at most
+constexpr uint64_t kRunLeast = 512 << 10;  // chunks from which a lane takes kRun of them
+static uint32_t run_for(uint64_t chunks) { return chunks >= kRunLeast ? kRun : 1; }
 
 static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
                       const uint32_t* hdr_len, const uint32_t* hdr_idx,
@@ -745,6 +846,11 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
   std::vector<FuseDesc> fdesc;                 // per fused leaf
   std::vector<uint32_t> fprod, fhead;          // its product and head bytes
   std::unordered_set<uint32_t> fused_prods;
+  std::vector<uint32_t> plain_leaves;
+  uint64_t plain_chunks = 0, all_chunks = 0;
+  for (size_t i = 0; i < n; i++)
+    all_chunks += (payload_len[i] >> 10) + 1;
+  const uint32_t lrun = run_for(all_chunks);
   uint64_t nc = 0;
   for (size_t i = 0; i < n; i++) {
     const uint32_t u = hdr_idx[i];
@@ -794,7 +900,7 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
     uint64_t slots = 0;
     if (fv && !stage && (kind[i] == POTS_KIND_BF16 || kind[i] == POTS_KIND_F32) &&
         (ptr - hl) % 16 == 4 && fv_fuse_candidate(fv, ptr, len, kind[i], &fp) &&
-        !fused_prods.count(fp.prod) && fuse_shape(L, fp.w * fp.esz, &T, &Q, &run, &nf, &slots)) {
+        !fused_prods.count(fp.prod) && fuse_shape(L, fp.w * fp.esz, lrun, &T, &Q, &run, &nf, &slots)) {
       fused_prods.insert(fp.prod);
       P->fuse_k = fp.k;  // one Freivalds plan: every fused product has the plan's k
       FuseDesc f;
@@ -824,7 +930,8 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
         }
       }
     } else {
-      plain.add((uint32_t)i, (nck + kRun - 1) / kRun);
+      plain_leaves.push_back((uint32_t)i);
+      plain_chunks += nck;
     }
     nc += nck;
     P->bytes += L;
@@ -836,7 +943,10 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
     return POTS_E_ARG;
   }
 
-  if (!plain.finish() || !fused.finish()) {
+  P->quad = plain_chunks <= kQuadMost;
+  plain.run = P->quad ? 1 : lrun;
+  for (uint32_t i : plain_leaves) plain.add(i, (desc[i].n_chunks + plain.run - 1) / plain.run);
+  if (!plain.finish(P->quad ? kQuadChunks : kThreads) || !fused.finish(kThreads)) {
     delete P;
     return POTS_E_ARG;
   }
@@ -957,6 +1067,7 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
     dords[k]->blk_ent = reinterpret_cast<const uint32_t*>(P->base + o_ord[k][2]);
     dords[k]->n_slots = ords[k]->n_slots;
     dords[k]->n_blocks = ords[k]->n_blocks;
+    dords[k]->run = ords[k]->run;
   }
   P->d_head = reinterpret_cast<uint32_t*>(P->base + o_head);
   P->d_levels = reinterpret_cast<LevelEntry*>(P->base + o_lev);
@@ -1056,7 +1167,15 @@ static int plan_stage(LeafPlan* P, int stage, uint32_t* d_digests, uint32_t* d_f
       }
       return POTS_E_OK;
     case POTS_LEAF_STAGE_PLAIN_CHUNKS:
-      if (P->plain.n_blocks) {
+      if (P->plain.n_blocks && P->quad) {
+        // a limit counts blocks of 256 lanes, four of this kernel's
+        const uint64_t most = P->max_grid ? 4ull * P->max_grid : P->plain.n_blocks;
+        hipLaunchKernelGGL(chunk_kernel_quad,
+                           dim3((uint32_t)std::min<uint64_t>(most, P->plain.n_blocks)), dim3(64),
+                           0, stream, P->d_leaves, P->plain, P->d_head, P->d_cv[0], d_digests,
+                           d_first_bad);
+        POTS_HIP(hipGetLastError());
+      } else if (P->plain.n_blocks) {
         hipLaunchKernelGGL(chunk_kernel,
                            dim3(P->max_grid ? std::min(P->max_grid, P->plain.n_blocks)
                                             : P->plain.n_blocks),

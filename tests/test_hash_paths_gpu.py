@@ -1,0 +1,80 @@
+"""The leaf hasher's ways of cutting work, each against the CPU oracle bit for bit: chunks on
+four lanes, one lane per chunk, and runs of chunks per lane, chosen by a plan's chunk count."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+KINDS = (torch.float32, torch.bfloat16, torch.float16, torch.int32)
+
+
+def _values(n, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    if dtype == torch.int32:
+        return torch.randint(-2**31, 2**31 - 1, (n,), generator=g, dtype=torch.int32)
+    return torch.randn(n, generator=g).to(dtype)
+
+
+def _leaves():
+    """Lengths around the edges of words, 16-byte groups, blocks, pairs of blocks and chunks
+    (the header takes the first 8, 12 or 16 bytes of a message), from payloads at every word
+    shift, as 1-D to 3-D tensors."""
+    out = []
+    for i, nbytes in enumerate((4, 8, 12, 16, 20, 44, 48, 52, 56, 60, 64, 108, 112, 116, 120, 128,
+                                1000, 1004, 1008, 1012, 1016, 1020, 1024, 1028, 2036, 2040, 2044,
+                                4084, 4088, 5000, 16 * 1024 - 12, 16 * 1024 - 8, 70000)):
+        dtype = KINDS[i % 4]
+        n = nbytes // dtype.itemsize
+        pad = (i % 5) * (4 // min(4, dtype.itemsize))  # 4-byte steps: word shifts of the payload
+        flat = _values(n + pad, dtype, 100 + i).to(DEV)[pad:]
+        out.append(flat.view([(n,), (1, n), (1, n, 1)][i % 3]))
+    odd = _values(3001, torch.bfloat16, 7).to(DEV)
+    return out + [odd[1:2], odd[1:], odd[3:2000]]  # 2-byte aligned: staged
+
+
+@pytest.mark.parametrize("filler_mib", [0, 33, 513])  # quads; a chunk per lane; runs of chunks
+def test_chunk_paths_match_oracle(lib, filler_mib):
+    from verification.commitment import native
+    ts = _leaves()
+    if filler_mib:
+        ts.append(torch.randn(filler_mib * 262144 - 5, device=DEV))
+    want, bad = O.hash_leaves([(O.tensor_leaf_header(3, t), t.cpu(), O.FINITE_KIND[t.dtype])
+                               for t in ts], simd=O.simd_degree() > 1)
+    assert bad == len(ts)
+    plan = lib.leaf_plan([O.tensor_leaf_header(3, t) for t in ts], ts,
+                         [native.FINITE_KIND[t.dtype] for t in ts])
+    d, first_bad = plan.run()
+    assert int(first_bad) == len(ts)
+    assert [bytes(x) for x in d.cpu().numpy()] == want
+    # a NaN in a leaf's last value, then in the first value of an earlier one
+    floats = [i for i, t in enumerate(ts[:33]) if t.dtype != torch.int32]
+    for i, at in ((floats[-1], -1), (floats[3], 0)):
+        ts[i].view(-1)[at] = float("nan")
+        assert int(plan.run()[1]) == i
+    plan.set_grid(3)  # a block limit: the same digests
+    for i in floats:
+        ts[i].view(-1)[0 if i == floats[3] else -1] = 1.0
+    a = plan.run()[0].cpu()
+    plan.set_grid(0)
+    assert torch.equal(a, plan.run()[0].cpu())
+    plan.close()
+
+
+def test_messages_with_no_payload(lib):
+    """Host messages are headers alone: every length around a block and a chunk."""
+    msgs = [bytes((7 * i + j) & 255 for j in range(n)) for i, n in enumerate(
+        (0, 1, 2, 3, 4, 15, 16, 17, 62, 63, 64, 65, 127, 128, 1022, 1023, 1024, 1025, 3071))]
+    n = len(msgs)
+    lens = np.array([len(m) for m in msgs], np.uint32)
+    offs = np.concatenate([[0], np.cumsum(lens[:-1])]).astype(np.uint64)
+    zero = np.zeros(n, np.uint64)
+    d, bad = lib.hash_leaves(b"".join(msgs), offs, lens, np.arange(n, dtype=np.uint32), zero, zero,
+                             np.zeros(n, np.uint8))
+    assert bad == n
+    assert [bytes(x) for x in d] == [O.hash_leaf(m) for m in msgs]
