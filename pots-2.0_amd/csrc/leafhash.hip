@@ -6,10 +6,11 @@
 //
 // Decomposition. Every leaf's message is cut into BLAKE3's 1 KiB chunks; one lane (or, in a
 // plan of few chunks, four) compresses one chunk (up to 16 blocks) and writes its chaining
-// value, or the digest itself when the leaf is a single chunk. The chunk CVs of a leaf form BLAKE3's tree, which has the RFC 6962
-// shape (a run of n > 1 chunks splits at the largest power of two below n), so it is reduced
-// level by level: level l+1 node j is the parent of level-l nodes 2j and 2j+1, or node 2j
-// itself when it has no sibling. The node that covers the whole leaf gets the ROOT flag.
+// value, or the digest itself when the leaf is a single chunk. The chunk CVs of a leaf form
+// BLAKE3's tree, which has the RFC 6962 shape (a run of n > 1 chunks splits at the largest
+// power of two below n), so it is reduced level by level, ten levels a launch: level l+1 node j
+// is the parent of level-l nodes 2j and 2j+1, or node 2j itself when it has no sibling. The
+// node that covers the whole leaf gets the ROOT flag.
 //
 // Message layout in HBM. The 0x00 prefix and the tensor header are 4(1 + ndim) bytes, a whole
 // number of words, so message word w of a leaf is payload word w - H/4 and no byte shifting is
@@ -82,7 +83,7 @@ static_assert(sizeof(FuseDesc) == 48, "FuseDesc layout");
 struct LevelEntry {     // one leaf with >= 2 nodes at the input level of one fold
   uint64_t in_off;      // its first node in the level's input buffer
   uint64_t out_off;     // its first node in the fold's output buffer
-  uint64_t out_first;   // its first output, counted over the level's entries
+  uint64_t out_first;   // its first output (and block), counted over the fold's entries
   uint32_t n_in;        // its nodes at this level
   uint32_t leaf;
 };
@@ -96,8 +97,8 @@ constexpr uint32_t kRun = 4;
 // Chunks per wave of the four-lane chunk kernel, and the words of one chunk's place in its LDS
 // (1 KiB and 16 bytes: neighbouring quads' words sit 4 banks apart).
 constexpr uint32_t kQuadChunks = 16, kQuadStride = 260;
-// Tree levels one launch of level_kernel reduces.
-constexpr uint32_t kFold = 3;
+// Tree levels one launch of level_kernel reduces, and the nodes a block takes to reduce them.
+constexpr uint32_t kFold = 10, kTile = 1u << kFold;
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4w __attribute__((ext_vector_type(4), aligned(4)));  // word aligned
@@ -640,63 +641,127 @@ __global__ __launch_bounds__(kThreads) void chunk_kernel_fused(
   }
 }
 
-// Levels kFold at a time: thread t makes output node o of its leaf at level l + kFold from the
-// (at most 2^kFold) nodes o·2^kFold .. of level l, level by level in registers with
-// BLAKE3's rule (pairs are hashed, a last odd node is promoted). A leaf whose tree closes
-// inside the fold writes its digest (the compression that makes the single top node carries
-// ROOT). Block b's outputs lie in entries blk_ent[b] .. blk_ent[b + 1].
+// Levels kFold at a time: block b makes one output node of its leaf (entry blk_ent[b]) at level
+// l + kFold from the (at most kTile) nodes o·kTile .. of level l, with BLAKE3's rule at each
+// level (pairs are hashed, a last odd node is promoted; kFold levels of it compose to a tile's
+// own reduction, since tiles begin at multiples of kTile). A leaf whose tree closes inside the
+// fold writes its digest: the compression that makes the single top node carries ROOT.
+//
+// A tile's first levels are wide, a lane per parent, the first straight from HBM; from 64
+// parents on a level is one compression of latency on four lanes each (b3_quad_compress), the
+// nodes in LDS throughout. (Three levels per launch, one lane each, took 44, 69, 80, 99 and
+// 166 us for leaves of 1, 64, 256, 1024 and 4096 MiB; this takes 21, 27, 30, 54 and 132.)
+//
+// Node j lies at node_at(j): a pair is one 64-byte message, and pairs sit 20 words apart, so
+// that the quads of a wave read different banks.
+__device__ __forceinline__ uint32_t node_at(uint32_t j) { return (j >> 1) * 20 + (j & 1) * 8; }
+
+__device__ __forceinline__ void lds_put8(uint32_t* p, const uint32_t v[8]) {
+  *reinterpret_cast<u32x4*>(p) = u32x4{v[0], v[1], v[2], v[3]};
+  *reinterpret_cast<u32x4*>(p + 4) = u32x4{v[4], v[5], v[6], v[7]};
+}
+
+__device__ __forceinline__ void get8(const u32x4& a, const u32x4& b, uint32_t v[8]) {
+#pragma unroll
+  for (int t = 0; t < 4; t++) {
+    v[t] = a[t];
+    v[4 + t] = b[t];
+  }
+}
+
 __global__ __launch_bounds__(kThreads) void level_kernel(
-    const LevelEntry* __restrict__ ents, const uint32_t* __restrict__ blk_ent, uint64_t n_out,
+    const LevelEntry* __restrict__ ents, const uint32_t* __restrict__ blk_ent,
     const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
     uint32_t* __restrict__ digests) {
-  const uint64_t t = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
-  if (t >= n_out) return;
-  uint32_t lo = blk_ent[blockIdx.x], hi = blk_ent[blockIdx.x + 1];
-  while (lo < hi) {
-    const uint32_t mid = (lo + hi + 1) >> 1;
-    if (ents[mid].out_first <= t) lo = mid;
-    else hi = mid - 1;
-  }
-  const LevelEntry e = ents[lo];
-  const uint64_t o = t - e.out_first;
-  constexpr uint32_t W = 1u << kFold;
-  const uint64_t first = o * W;
-  const uint32_t cnt = (uint32_t)min<uint64_t>(W, e.n_in - first);
-  uint32_t cv[W][8];
-  const uint4* src = reinterpret_cast<const uint4*>(in + 8ull * (e.in_off + first));
+  __shared__ __align__(16) uint32_t s_wide[kTile / 4 * 20];  // up to kTile / 2 nodes
+  __shared__ __align__(16) uint32_t s_quad[32 * 20];         // up to 64 nodes
+  const uint32_t tid = threadIdx.x;
+  const LevelEntry e = ents[blk_ent[blockIdx.x]];
+  const uint64_t o = blockIdx.x - e.out_first, first = o * kTile;
+  const uint32_t cnt = (uint32_t)min<uint64_t>(kTile, e.n_in - first);
+  const u32x4* src = reinterpret_cast<const u32x4*>(in + 8ull * (e.in_off + first));
+  // m: the tile's nodes at the current level; n: the leaf's
+  uint32_t m = cnt, n = e.n_in;
+  if (cnt <= 128) {
+    if (tid < 2 * cnt)
+      *reinterpret_cast<u32x4*>(s_wide + node_at(tid >> 1) + 4 * (tid & 1)) =
+          gload<u32x4>(src + tid);
+    __syncthreads();
+  } else {
+    static_assert(kTile == 4 * kThreads, "two parents per thread at the first level");
+    u32x4 x[2][4];
 #pragma unroll
-  for (uint32_t a = 0; a < W; a++) {
-    uint4 x = make_uint4(0, 0, 0, 0), y = make_uint4(0, 0, 0, 0);
-    if (a < cnt) {
-      x = src[2 * a];
-      y = src[2 * a + 1];
+    for (uint32_t h = 0; h < 2; h++) {
+      const uint32_t t = tid + kThreads * h;
+      // (a child past the tile rereads the tile's last node; its value is not used)
+#pragma unroll
+      for (uint32_t u = 0; u < 4; u++)
+        x[h][u] = gload<u32x4>(src + 2 * min(2 * t + (u >> 1), cnt - 1) + (u & 1));
     }
-    cv[a][0] = x.x; cv[a][1] = x.y; cv[a][2] = x.z; cv[a][3] = x.w;
-    cv[a][4] = y.x; cv[a][5] = y.y; cv[a][6] = y.z; cv[a][7] = y.w;
-  }
-  // m: this thread's nodes at the current level; n: the leaf's nodes at the current level.
-  uint32_t m = cnt;
-  uint64_t n = e.n_in;
 #pragma unroll
-  for (uint32_t lvl = 0; lvl < kFold; lvl++) {
-    const uint64_t n_next = (n + 1) / 2;
-    const uint32_t flags = n_next == 1 ? B3_ROOT : 0u;
-#pragma unroll
-    for (uint32_t a = 0; a < (W >> (lvl + 1)); a++) {
-      if (2 * a + 1 < m) {
-        b3_parent_cv(cv[2 * a], cv[2 * a + 1], flags, cv[a]);
-      } else if (2 * a < m) {
-#pragma unroll
-        for (int q = 0; q < 8; q++) cv[a][q] = cv[2 * a][q];
+    for (uint32_t h = 0; h < 2; h++) {
+      const uint32_t t = tid + kThreads * h;
+      uint32_t l[8], r[8], v[8];
+      get8(x[h][0], x[h][1], l);
+      get8(x[h][2], x[h][3], r);
+      if (2 * t + 1 < cnt) {
+        b3_parent_cv(l, r, 0u, v);
+        lds_put8(s_wide + node_at(t), v);
+      } else if (2 * t < cnt) {
+        lds_put8(s_wide + node_at(t), l);
       }
     }
     m = (m + 1) / 2;
-    n = n_next;
+    n = (n + 1) / 2;
+    __syncthreads();
+    while (m > 128) {
+      uint32_t l[8], r[8], v[8];
+      const bool pair = 2 * tid + 1 < m, one = 2 * tid < m;
+      if (one) {
+        const u32x4* p = reinterpret_cast<const u32x4*>(s_wide + 20 * tid);
+        get8(p[0], p[1], l);
+        get8(p[2], p[3], r);
+      }
+      __syncthreads();  // every child is read before a parent overwrites one
+      if (pair) {
+        b3_parent_cv(l, r, 0u, v);
+        lds_put8(s_wide + node_at(tid), v);
+      } else if (one) {
+        lds_put8(s_wide + node_at(tid), l);
+      }
+      m = (m + 1) / 2;
+      n = (n + 1) / 2;
+      __syncthreads();
+    }
   }
-  uint4* dst = reinterpret_cast<uint4*>(n == 1 ? digests + 8ull * e.leaf
-                                               : out + 8ull * (e.out_off + o));
-  dst[0] = make_uint4(cv[0][0], cv[0][1], cv[0][2], cv[0][3]);
-  dst[1] = make_uint4(cv[0][4], cv[0][5], cv[0][6], cv[0][7]);
+  const uint32_t q = tid & 3, t = tid >> 2;
+  const B3Quad sched = b3_quad_schedule(q);
+  uint32_t *cur = s_wide, *nxt = s_quad;
+  while (m > 1) {
+    n = (n + 1) / 2;
+    const uint32_t flags = B3_PARENT | (n == 1 ? B3_ROOT : 0u);
+    const uint32_t tail = q < 2 ? 0u : q == 2 ? 64u : flags;
+    uint32_t* dst = nxt + node_at(t);
+    if (2 * t + 1 < m) {
+      uint32_t lo, hi;
+      b3_quad_iv(q, lo, hi);
+      b3_quad_compress(sched, cur + 20 * t, q, tail, lo, hi);
+      dst[q] = lo;
+      dst[4 + q] = hi;
+    } else if (2 * t < m) {
+      dst[q] = cur[20 * t + q];
+      dst[4 + q] = cur[20 * t + 4 + q];
+    }
+    m = (m + 1) / 2;
+    __syncthreads();
+    uint32_t* const swap = cur;
+    cur = nxt;
+    nxt = swap;
+  }
+  if (tid < 8)
+    gstore<uint32_t>((e.n_in <= kTile ? digests + 8ull * e.leaf : out + 8ull * (e.out_off + o)) +
+                         tid,
+                     cur[tid]);
 }
 
 __global__ void fill_u32(uint32_t* p, uint32_t v) { *p = v; }
@@ -952,8 +1017,8 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
   }
 
   // Reduction folds of kFold levels each. Level 0 nodes of leaf i sit at desc[i].cv_first in
-  // cv0; a fold takes a leaf's n nodes to ceil(n / 2^kFold) (BLAKE3's halving with a
-  // promoted odd node, kFold times, composes to that ceiling).
+  // cv0; a fold takes a leaf's n nodes to ceil(n / kTile) (BLAKE3's halving with a promoted
+  // odd node, kFold times, composes to that ceiling), a block each.
   std::vector<LevelEntry> ents;
   std::vector<uint32_t> blk_ent;
   std::vector<uint64_t> n_nodes(n), off(n);
@@ -968,7 +1033,7 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
     uint64_t out_next = 0;
     for (size_t i = 0; i < n; i++) {
       if (n_nodes[i] < 2) continue;
-      const uint64_t nout = (n_nodes[i] + (1u << kFold) - 1) >> kFold;
+      const uint64_t nout = (n_nodes[i] + kTile - 1) >> kFold;
       LevelEntry e;
       e.in_off = off[i];
       e.out_off = out_next;
@@ -983,16 +1048,15 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
       out_next += nout;
     }
     if (li.n_ents == 0) break;
-    // Per block of kThreads outputs: the fold-relative index of the entry holding its first
-    // output, and a closing bound.
-    const uint64_t nb = (li.n_out + kThreads - 1) / kThreads;
-    uint32_t k = 0;
-    for (uint64_t b = 0; b < nb; b++) {
-      const uint64_t first_out = b * kThreads;
-      while (k + 1 < li.n_ents && ents[li.ent_first + k + 1].out_first <= first_out) k++;
-      blk_ent.push_back(k);
+    if (li.n_out >= 0x7FFFFFFFull) {
+      delete P;
+      return POTS_E_ARG;
     }
-    blk_ent.push_back(li.n_ents - 1);
+    // Per block (one output each): the fold-relative index of its entry.
+    for (uint32_t k = 0; k < li.n_ents; k++) {
+      const uint64_t end = k + 1 < li.n_ents ? ents[li.ent_first + k + 1].out_first : li.n_out;
+      blk_ent.resize(li.blk_first + end, k);
+    }
     if (li.out_buf == 1) cv1_need = std::max(cv1_need, out_next);
     P->levels.push_back(li);
     in_buf = 1 - in_buf;
@@ -1186,9 +1250,8 @@ static int plan_stage(LeafPlan* P, int stage, uint32_t* d_digests, uint32_t* d_f
       return POTS_E_OK;
     case 2:
       for (const LevelInfo& li : P->levels) {
-        const uint64_t blocks = (li.n_out + kThreads - 1) / kThreads;
-        hipLaunchKernelGGL(level_kernel, dim3((uint32_t)blocks), dim3(kThreads), 0, stream,
-                           P->d_levels + li.ent_first, P->d_blk_ent + li.blk_first, li.n_out,
+        hipLaunchKernelGGL(level_kernel, dim3((uint32_t)li.n_out), dim3(kThreads), 0, stream,
+                           P->d_levels + li.ent_first, P->d_blk_ent + li.blk_first,
                            P->d_cv[li.in_buf], P->d_cv[li.out_buf], d_digests);
         POTS_HIP(hipGetLastError());
       }

@@ -78,3 +78,21 @@ def test_messages_with_no_payload(lib):
                              np.zeros(n, np.uint8))
     assert bad == n
     assert [bytes(x) for x in d] == [O.hash_leaf(m) for m in msgs]
+
+
+@pytest.mark.parametrize("chunks", [
+    [2, 127, 128, 129, 130, 255, 257, 1022, 1023, 1024, 1025, 1026, 1151, 1152, 1153, 2047, 2048,
+     2049, 3000],            # a tile's quads alone, its wide levels, one tile and several
+    [1024 * 1024 + 1],       # three folds, the last tile a single node promoted through two
+    [1024 * 1024, 1024 * 1025 - 1]])
+def test_leaf_trees_at_tile_edges(lib, chunks):
+    from verification.commitment import native
+    ts = [torch.randint(0, 2**31 - 1, ((1024 * n - 100) // 4,), device=DEV, dtype=torch.int32)
+          for n in chunks]
+    heads = [O.tensor_leaf_header(2, t) for t in ts]
+    want, _ = O.hash_leaves([(h, t.cpu(), 0) for h, t in zip(heads, ts)],
+                            simd=O.simd_degree() > 1)
+    plan = lib.leaf_plan(heads, ts, [native.KIND_NONE] * len(ts))
+    assert plan.chunks == sum(chunks)
+    assert [bytes(x) for x in plan.run()[0].cpu().numpy()] == want
+    plan.close()
