@@ -96,3 +96,11 @@ def test_leaf_trees_at_tile_edges(lib, chunks):
     assert plan.chunks == sum(chunks)
     assert [bytes(x) for x in plan.run()[0].cpu().numpy()] == want
     plan.close()
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 127, 128, 129, 255, 256, 257, 258, 511, 512, 513, 65535,
+                               65536, 65537, 65793, 100003])
+def test_outer_tree_at_tile_edges(lib, n):
+    d = torch.randint(0, 256, (n, 32), device=DEV, dtype=torch.uint8)
+    want = O.merkle_tree([bytes(x) for x in d.cpu().numpy()])
+    assert lib.merkle_tree_device(d).cpu().numpy().tobytes() == want
