@@ -1114,101 +1114,129 @@ struct RedJob {
   uint64_t pdot, pabs, psq;  // the B job's partials
   uint64_t vout;             // packed B·R for the A pass
   uint64_t u, w;             // b1 = |B|·1 and b2 = B²·1, fp32 [q]
-  uint64_t group_first;      // prefix of (8-row groups x k) over the jobs before it
+  uint32_t blk_first;        // prefix of kRedRows-row blocks over the jobs before it
   uint32_t rows, rows_pad;   // q and its padding
   uint32_t n_chunks, a_dt;   // the A pass's dtype decides the packing
-  uint32_t u_slots, pad;     // 1: also pack b1's three bf16 terms into slots 12..14 (a
+  uint32_t u_slots;          // 1: also pack b1's three bf16 terms into slots 12..14 (a
                              // twin product, whose |A|·b1 runs on the matrix cores)
 };
-static_assert(sizeof(RedJob) == 80, "RedJob layout");
+static_assert(sizeof(RedJob) == 72, "RedJob layout");
 
+constexpr uint32_t kRedRows = 32;  // rows of B a block reduces (a packed K-step of bf16)
+
+// A block adds kRedRows rows' partials over the column chunks: a thread per value, so a chunk's
+// values of the block's rows are one contiguous read, four chunks' reads in flight, then packs
+// them from LDS eight rows at a time. (A thread per eight-row group and challenge read its rows
+// one by one: 107 us for a 1536 x 151936 B of 38 chunks, k = 4, against 10, and 12 us for a
+// 4096 x 4096 one of four, k = 8, against 5.) Sums in fp64, in chunk order.
 __global__ __launch_bounds__(256) void reduce_b(const RedJob* __restrict__ jobs, uint32_t n_jobs,
-                                                uint64_t n_threads, uint32_t k) {
-  const uint64_t g = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-  if (g >= n_threads) return;
+                                                uint32_t k) {
+  extern __shared__ float s_red[];  // [kRedRows][k], then |B|·1's kRedRows
   uint32_t lo = 0, hi = n_jobs - 1;
   while (lo < hi) {
     const uint32_t mid = (lo + hi + 1) >> 1;
-    if (jobs[mid].group_first <= g) lo = mid;
+    if (jobs[mid].blk_first <= blockIdx.x) lo = mid;
     else hi = mid - 1;
   }
   const RedJob J = jobs[lo];
-  const uint64_t local = g - J.group_first;
-  const uint32_t grp = (uint32_t)(local / k), j = (uint32_t)(local % k);
-  const float* pdot = reinterpret_cast<const float*>(J.pdot);
-  float v[8];
+  const uint32_t r0 = (blockIdx.x - J.blk_first) * kRedRows, nv = kRedRows * k;
+  const uint32_t live = min(kRedRows, J.rows - r0);  // rows past the matrix: zero
+  float* const s_abs = s_red + nv;
+  const float* pdot = reinterpret_cast<const float*>(J.pdot) + (uint64_t)r0 * k;
+  const uint64_t cstride = (uint64_t)J.rows_pad * k;
+  for (uint32_t t = threadIdx.x; t < nv; t += 256) {
+    double sum = 0.0;
+    if (t < live * k)
+      for (uint32_t c0 = 0; c0 < J.n_chunks; c0 += 4) {
+        float x[4];
 #pragma unroll
-  for (int e = 0; e < 8; e++) {
-    const uint32_t row = 8 * grp + e;
-    double s = 0.0;
-    if (row < J.rows)
-      for (uint32_t c = 0; c < J.n_chunks; c++)
-        s += (double)gload<float>(pdot + ((uint64_t)c * J.rows_pad + row) * k + j);
-    v[e] = (float)s;
+        for (uint32_t c = 0; c < 4; c++)
+          x[c] = gload<float>(pdot + min(c0 + c, J.n_chunks - 1) * cstride + t);
+#pragma unroll
+        for (uint32_t c = 0; c < 4; c++)
+          if (c0 + c < J.n_chunks) sum += (double)x[c];
+      }
+    s_red[t] = (float)sum;
   }
-  if (J.a_dt == DT_BF16) {
+  if (threadIdx.x >= 256 - kRedRows) {  // the last threads, idle above at small k
+    const uint32_t e = threadIdx.x - (256 - kRedRows);
+    double a = 0.0, q = 0.0;
+    if (e < live) {
+      const float* pabs = reinterpret_cast<const float*>(J.pabs) + r0 + e;
+      const double* psq = reinterpret_cast<const double*>(J.psq) + r0 + e;
+      for (uint32_t c0 = 0; c0 < J.n_chunks; c0 += 4) {
+        float x[4];
+        double y[4];
+#pragma unroll
+        for (uint32_t c = 0; c < 4; c++) {
+          const uint64_t at = (uint64_t)min(c0 + c, J.n_chunks - 1) * J.rows_pad;
+          x[c] = gload<float>(pabs + at);
+          y[c] = gload<double>(psq + at);
+        }
+#pragma unroll
+        for (uint32_t c = 0; c < 4; c++)
+          if (c0 + c < J.n_chunks) {
+            a += (double)x[c];
+            q += y[c];
+          }
+      }
+      gstore<float>(reinterpret_cast<float*>(J.u) + r0 + e, (float)a);
+      gstore<float>(reinterpret_cast<float*>(J.w) + r0 + e, (float)q);
+    }
+    s_abs[e] = (float)a;
+  }
+  __syncthreads();
+  // eight rows of a column as three bf16 terms, in three consecutive slots
+  auto put3 = [](uint16_t* dst, const float (&v)[8]) {
     uint16_t pl[3][8];
 #pragma unroll
     for (int e = 0; e < 8; e++) split_bf16x3(v[e], pl[0][e], pl[1][e], pl[2][e]);
-    uint16_t* dst = reinterpret_cast<uint16_t*>(J.vout) +
-                    (((uint64_t)grp * groups_b3(k) + j / 5) * 16 + 3 * (j % 5)) * 8;
 #pragma unroll
     for (int p = 0; p < 3; p++)
       gstore<u32x4>(dst + 8 * p, u32x4{pl[p][0] | (uint32_t)pl[p][1] << 16,
                                        pl[p][2] | (uint32_t)pl[p][3] << 16,
                                        pl[p][4] | (uint32_t)pl[p][5] << 16,
                                        pl[p][6] | (uint32_t)pl[p][7] << 16});
-  } else {
-    float* base = reinterpret_cast<float*>(J.vout);
-    const uint32_t njg = groups_f4(k);
+  };
+  for (uint32_t t = threadIdx.x; t < kRedRows / 8 * k; t += 256) {
+    const uint32_t g = t / k, j = t - g * k;
+    const uint64_t grp = r0 / 8 + g;
+    float v[8];
 #pragma unroll
-    for (int h = 0; h < 2; h++)
-      gstore<u32x4>(base + (((uint64_t)(2 * grp + h) * njg + j / 16) * 16 + j % 16) * 4,
-                    u32x4{__float_as_uint(v[4 * h]), __float_as_uint(v[4 * h + 1]),
-                          __float_as_uint(v[4 * h + 2]), __float_as_uint(v[4 * h + 3])});
+    for (uint32_t e = 0; e < 8; e++) v[e] = s_red[(8 * g + e) * k + j];
+    if (J.a_dt == DT_BF16) {
+      put3(reinterpret_cast<uint16_t*>(J.vout) +
+               ((grp * groups_b3(k) + j / 5) * 16 + 3 * (j % 5)) * 8,
+           v);
+    } else {
+      float* base = reinterpret_cast<float*>(J.vout);
+      const uint32_t njg = groups_f4(k);
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+        gstore<u32x4>(base + (((2 * grp + h) * njg + j / 16) * 16 + j % 16) * 4,
+                      u32x4{__float_as_uint(v[4 * h]), __float_as_uint(v[4 * h + 1]),
+                            __float_as_uint(v[4 * h + 2]), __float_as_uint(v[4 * h + 3])});
+    }
   }
-  if (j == 0) {
-    const float* pabs = reinterpret_cast<const float*>(J.pabs);
-    const double* psq = reinterpret_cast<const double*>(J.psq);
-    float* u = reinterpret_cast<float*>(J.u);
-    float* w = reinterpret_cast<float*>(J.w);
-    float ua[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};  // rows past the matrix: zero
+  if (J.u_slots && threadIdx.x < kRedRows / 8) {
+    const uint32_t g = threadIdx.x;
+    float v[8];
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
-      const uint32_t row = 8 * grp + e;
-      if (row >= J.rows) continue;
-      double a = 0.0, q = 0.0;
-      for (uint32_t c = 0; c < J.n_chunks; c++) {
-        a += (double)gload<float>(pabs + (uint64_t)c * J.rows_pad + row);
-        q += gload<double>(psq + (uint64_t)c * J.rows_pad + row);
-      }
-      gstore<float>(u + row, (float)a);
-      gstore<float>(w + row, (float)q);
-      ua[e] = (float)a;
-    }
-    if (J.u_slots) {
-      uint16_t pl[3][8];
-#pragma unroll
-      for (int e = 0; e < 8; e++) split_bf16x3(ua[e], pl[0][e], pl[1][e], pl[2][e]);
-      uint16_t* dst = reinterpret_cast<uint16_t*>(J.vout) + ((uint64_t)grp * 16 + 12) * 8;
-#pragma unroll
-      for (int p = 0; p < 3; p++)
-        gstore<u32x4>(dst + 8 * p, u32x4{pl[p][0] | (uint32_t)pl[p][1] << 16,
-                                         pl[p][2] | (uint32_t)pl[p][3] << 16,
-                                         pl[p][4] | (uint32_t)pl[p][5] << 16,
-                                         pl[p][6] | (uint32_t)pl[p][7] << 16});
-    }
+    for (uint32_t e = 0; e < 8; e++) v[e] = s_abs[8 * g + e];
+    put3(reinterpret_cast<uint16_t*>(J.vout) + ((uint64_t)(r0 / 8 + g) * 16 + 12) * 8, v);
   }
 }
 
 // ---- finish: one product's row ------------------------------------------------------------
 //
 // Three kernels. bias_terms: per biased product, ‖b‖₁, ‖b‖² and bᵀR_j. finish_slices: per
-// slice of at most kSliceRows rows of a product, the fp64 sums over its rows of ν_i², |P|1_i²,
+// slice of 256 to kSliceRows rows of a product (as many as leave the launch 512 blocks; fewer
+// where a product has many chunks), the fp64 sums over its rows of ν_i², |P|1_i²,
 // ‖P_i‖², (A²(B²1))_i and d_ij², written as one record. finish_final: per product, the slices'
 // records added in slice order, then the square roots. Every sum has a fixed order, so the
-// row does not depend on timing; slicing keeps the largest products (150k rows) from running
-// on one block.
+// row does not depend on timing. (Slices of 2048 rows whatever the plan: 30 us for the four of an
+// 8192-row product against 10 for 32; but of 256 rows for a layer's 750 thousand rows: 56 us
+// against 46, a block's own sums being most of it.)
 
 constexpr uint32_t kSliceRows = 2048;
 
@@ -1235,52 +1263,7 @@ struct BiasOut {
   double bsq;
 };
 
-__device__ __forceinline__ double block_sum(double v, double* sh) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  const int wv = threadIdx.x >> 6, ln = threadIdx.x & 63;
-  __syncthreads();
-  if (ln == 0) sh[wv] = v;
-  __syncthreads();
-  double t = 0.0;
-  for (int i = 0; i < (int)(blockDim.x >> 6); i++) t += sh[i];
-  __syncthreads();
-  return t;
-}
-
-// One block per biased product (index list `which`).
-__global__ __launch_bounds__(256) void bias_terms(const FinJob* __restrict__ jobs,
-                                                  const uint32_t* __restrict__ which, uint32_t k,
-                                                  BiasOut* __restrict__ bout,
-                                                  float* __restrict__ br) {
-  __shared__ double sh[4];
-  const uint32_t pi = which[blockIdx.x];
-  const FinJob J = jobs[pi];
-  const float* bias = reinterpret_cast<const float*>(J.bias);
-  const float* R = reinterpret_cast<const float*>(J.r);
-  double a = 0.0, q = 0.0;
-  for (uint32_t c = threadIdx.x; c < J.w; c += blockDim.x) {
-    const double b = gload<float>(bias + c);
-    a += fabs(b);
-    q += b * b;
-  }
-  a = block_sum(a, sh);
-  q = block_sum(q, sh);
-  if (threadIdx.x == 0) {
-    BiasOut o;
-    o.babs = __float_as_uint((float)a);
-    o.bsq = q;
-    bout[pi] = o;
-  }
-  for (uint32_t j = 0; j < k; j++) {
-    double t = 0.0;
-    for (uint32_t c = threadIdx.x; c < J.w; c += blockDim.x)
-      t += (double)gload<float>(bias + c) * (double)gload<float>(R + (uint64_t)c * k + j);
-    t = block_sum(t, sh);
-    if (threadIdx.x == 0) br[(uint64_t)pi * k + j] = (float)t;
-  }
-}
-
-// block_sum of N values at once: each value's additions are block_sum's, in the same order.
+// The block's sums of N values per thread (sh: 4·N doubles), in a fixed order.
 template <int N>
 __device__ __forceinline__ void block_sums(double (&v)[N], double* sh) {
 #pragma unroll
@@ -1300,6 +1283,45 @@ __device__ __forceinline__ void block_sums(double (&v)[N], double* sh) {
     v[n] = t;
   }
   __syncthreads();
+}
+
+// One block per biased product (index list `which`): ‖b‖₁, ‖b‖² and bᵀR_j in one sweep over b
+// with the first eight challenges, each further eight in a sweep of their own.
+__global__ __launch_bounds__(256) void bias_terms(const FinJob* __restrict__ jobs,
+                                                  const uint32_t* __restrict__ which, uint32_t k,
+                                                  BiasOut* __restrict__ bout,
+                                                  float* __restrict__ br) {
+  __shared__ double sh[10 * 4];
+  const uint32_t pi = which[blockIdx.x];
+  const FinJob J = jobs[pi];
+  const float* bias = reinterpret_cast<const float*>(J.bias);
+  const float* R = reinterpret_cast<const float*>(J.r);
+  for (uint32_t j0 = 0; j0 < k; j0 += 8) {
+    const uint32_t nj = min(8u, k - j0);
+    double acc[10];  // bᵀR_j0 .. bᵀR_j0+7, Σ|b|, Σb²
+#pragma unroll
+    for (int t = 0; t < 10; t++) acc[t] = 0.0;
+    for (uint32_t c = threadIdx.x; c < J.w; c += blockDim.x) {
+      const double b = gload<float>(bias + c);
+#pragma unroll
+      for (uint32_t jj = 0; jj < 8; jj++)
+        if (jj < nj) acc[jj] += b * (double)gload<float>(R + (uint64_t)c * k + j0 + jj);
+      acc[8] += fabs(b);
+      acc[9] += b * b;
+    }
+    block_sums<10>(acc, sh);
+    if (threadIdx.x == 0) {
+      if (j0 == 0) {
+        BiasOut o;
+        o.babs = __float_as_uint((float)acc[8]);
+        o.bsq = acc[9];
+        bout[pi] = o;
+      }
+#pragma unroll
+      for (uint32_t jj = 0; jj < 8; jj++)
+        if (jj < nj) br[(uint64_t)pi * k + j0 + jj] = (float)acc[jj];
+    }
+  }
 }
 
 // Adds a row's partial dot products X·V_j, j = j0 .. j0 + nj − 1, over its column chunks in
@@ -1434,7 +1456,8 @@ __global__ __launch_bounds__(256) void finish_slices(const FinJob* __restrict__ 
         }
       }
     }
-    block_sums<12>(acc, sh);
+    if (nj <= 4) block_sums<8>(*reinterpret_cast<double(*)[8]>(acc), sh);
+    else block_sums<12>(acc, sh);
     if (tid == 0) {
       if (first)
         for (int t = 0; t < 4; t++) out[t] = acc[t];
@@ -1443,27 +1466,43 @@ __global__ __launch_bounds__(256) void finish_slices(const FinJob* __restrict__ 
   }
 }
 
-// One thread per product: the slices' records in order, then the row.
-__global__ __launch_bounds__(256) void finish_final(const FinJob* __restrict__ jobs,
-                                                    uint32_t n, uint32_t k, uint32_t guard,
-                                                    const BiasOut* __restrict__ bout,
-                                                    const double* __restrict__ recs,
-                                                    double* __restrict__ rows) {
-  const uint32_t pi = blockIdx.x * blockDim.x + threadIdx.x;
-  if (pi >= n) return;
+// One wave per product: lane l adds slices l, l + 64, ... of each column, eight columns' loads in
+// flight, then the lanes in a fixed order. (One thread per product, column after column: 216 us
+// beside the hashing where one product has 128 slices, against 9.)
+__global__ __launch_bounds__(64) void finish_final(const FinJob* __restrict__ jobs, uint32_t k,
+                                                   uint32_t guard,
+                                                   const BiasOut* __restrict__ bout,
+                                                   const double* __restrict__ recs,
+                                                   double* __restrict__ rows) {
+  const uint32_t pi = blockIdx.x, lane = threadIdx.x;
   const FinJob J = jobs[pi];
   double* out = rows + (uint64_t)pi * (5 + k);
-  const double nan = __builtin_nan("");
-  for (uint32_t col = 0; col < 4 + k; col++) {
-    double t = 0.0;
-    for (uint32_t sl = 0; sl < J.n_slices; sl++)
-      t += recs[(uint64_t)(J.slice_first + sl) * (4 + k) + col];
-    if (col < 2) out[col] = guard ? sqrt(t) : nan;
-    else if (col == 2) out[2] = sqrt(t);
-    else if (col == 3) out[3] = t;
-    else out[1 + col] = sqrt(t);
+  for (uint32_t c0 = 0; c0 < 4 + k; c0 += 8) {
+    double acc[8];
+#pragma unroll
+    for (int t = 0; t < 8; t++) acc[t] = 0.0;
+    for (uint32_t sl = lane; sl < J.n_slices; sl += 64) {
+      const double* rec = recs + (uint64_t)(J.slice_first + sl) * (4 + k) + c0;
+#pragma unroll
+      for (uint32_t t = 0; t < 8; t++)
+        if (c0 + t < 4 + k) acc[t] += rec[t];
+    }
+    if (J.n_slices > 1) {  // (a single slice's sums are in lane 0 already)
+#pragma unroll
+      for (int t = 0; t < 8; t++)
+        for (int o = 32; o > 0; o >>= 1) acc[t] += __shfl_xor(acc[t], o);
+    }
+    if (lane == 0) {
+#pragma unroll
+      for (uint32_t t = 0; t < 8; t++) {
+        const uint32_t col = c0 + t;
+        if (col < 2) out[col] = guard ? sqrt(acc[t]) : __builtin_nan("");
+        else if (col == 3) out[3] = acc[t];
+        else if (col < 4 + k) out[col == 2 ? 2 : 1 + col] = sqrt(acc[t]);
+      }
+    }
   }
-  out[4] = J.bias != 0 ? bout[pi].bsq : 0.0;
+  if (lane == 0) out[4] = J.bias != 0 ? bout[pi].bsq : 0.0;
 }
 
 // ---- P-pass sums of fused products, from the chunk kernel's run records -------------------
@@ -1476,21 +1515,33 @@ struct FixJob {
   uint64_t row_first;        // prefix of rows over the jobs before it
   uint32_t n, w;
   uint32_t head, esz;
-  uint32_t J, k;             // record slots per row; challenges (1, 2 or 4)
+  uint32_t J, pad;           // record slots per row
 };
 static_assert(sizeof(FixJob) == 80, "FixJob layout");
 
-// One thread per row: the row's records in chunk order (fp64), then the elements of the
-// leaf's first bytes up to the first 128-byte boundary of the message (row 0) and of its last
-// bytes after the last one (the last row), which no chunk's interior pairs took. Rounded to
-// the P job's partial formats as one column chunk.
+// The rows' records (fp64), then the elements of the leaf's first bytes up to the first
+// 128-byte boundary of the message (row 0) and of its last bytes after the last one (the last
+// row), which no chunk's interior pairs took. Rounded to the P job's partial formats as one
+// column chunk.
+//
+// A block takes 64 rows; each of its four waves adds every fourth record of them (a lane a row,
+// so a wave's loads are contiguous), four records' loads in flight, and the first wave adds the
+// waves' sums in wave order. (A thread per row was one chain of loads as long as the row's
+// records, 298 for a 151936-column product: 1017 us beside the hashing in a two-layer step,
+// where this takes 720, 62 alone.)
 // `blk[b]`: the job of block b's first row (blk[gridDim.x] the last job), so a thread searches
 // only the few jobs its block's rows span instead of all of them (a dozen dependent loads).
+constexpr uint32_t kFixRows = 64;
+
+template <int K>
 __global__ __launch_bounds__(256) void fused_rows(const FixJob* __restrict__ jobs,
                                                   const uint32_t* __restrict__ blk,
-                                                  uint64_t n_threads) {
-  const uint64_t g = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-  if (g >= n_threads) return;
+                                                  uint64_t n_rows) {
+  __shared__ double s_sum[3][K + 2][kFixRows];
+  __shared__ uint32_t s_exact[3][kFixRows];
+  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  // (lanes past the last row take it too and write nothing)
+  const uint64_t g0 = (uint64_t)blockIdx.x * kFixRows + lane, g = min(g0, n_rows - 1);
   uint32_t lo = blk[blockIdx.x], hi = blk[blockIdx.x + 1];
   while (lo < hi) {
     const uint32_t mid = (lo + hi + 1) >> 1;
@@ -1502,31 +1553,46 @@ __global__ __launch_bounds__(256) void fused_rows(const FixJob* __restrict__ job
   const uint64_t rb = (uint64_t)J.w * J.esz, H = J.head, L = H + (uint64_t)J.n * rb;
   const uint64_t hc = (H + 127) & ~uint64_t(127), lf = L & ~uint64_t(127);
   const uint64_t fs = max<uint64_t>(H + i * rb, hc), fe = min<uint64_t>(H + (i + 1) * rb, lf);
-  double d[4] = {0.0, 0.0, 0.0, 0.0}, s1 = 0.0, s2 = 0.0;
+  const uint32_t count = fs < fe ? (uint32_t)(((fe - 1) >> 10) - (fs >> 10) + 1) : 0u;
+  double d[K + 2];  // Σ p·R_j, Σ|p|, Σp²
+#pragma unroll
+  for (int j = 0; j < K + 2; j++) d[j] = 0.0;
   bool exact = false;
-  if (fs < fe) {
-    const char* rec = reinterpret_cast<const char*>(J.seg) + (uint64_t)kRunBytes * i;
-    const uint64_t stride = (uint64_t)kRunBytes * J.n;
-    auto add = [&](const v4f32& a, const u32x4& b) {
-      for (uint32_t j = 0; j < J.k; j++) d[j] += (double)a[j];
-      s1 += (double)__uint_as_float(b.x);
-      exact |= b.y != 0u;
-      s2 += __longlong_as_double((long long)((uint64_t)b.w << 32 | b.z));
-    };
-    // Four records' loads are issued before their sums, which are taken in record order.
-    uint64_t left = ((fe - 1) >> 10) - (fs >> 10) + 1;
-    for (; left >= 4; left -= 4, rec += 4 * stride) {
-      v4f32 a[4];
-      u32x4 b[4];
+  const char* rec = reinterpret_cast<const char*>(J.seg) + (uint64_t)kRunBytes * i;
+  const uint64_t stride = (uint64_t)kRunBytes * J.n;
+  auto add = [&](const v4f32& a, const u32x4& b) {
 #pragma unroll
-      for (int u = 0; u < 4; u++) {
-        a[u] = gload<v4f32>(rec + u * stride);
-        b[u] = gload<u32x4>(rec + u * stride + 16);
-      }
+    for (int j = 0; j < K; j++) d[j] += (double)a[j];
+    d[K] += (double)__uint_as_float(b.x);
+    exact |= b.y != 0u;
+    d[K + 1] += __longlong_as_double((long long)((uint64_t)b.w << 32 | b.z));
+  };
+  uint32_t c = wave;
+  for (; c + 12 < count; c += 16) {
+    v4f32 a[4];
+    u32x4 b[4];
 #pragma unroll
-      for (int u = 0; u < 4; u++) add(a[u], b[u]);
+    for (uint32_t u = 0; u < 4; u++) {
+      a[u] = gload<v4f32>(rec + (c + 4 * u) * stride);
+      b[u] = gload<u32x4>(rec + (c + 4 * u) * stride + 16);
     }
-    for (; left > 0; left--, rec += stride) add(gload<v4f32>(rec), gload<u32x4>(rec + 16));
+#pragma unroll
+    for (int u = 0; u < 4; u++) add(a[u], b[u]);
+  }
+  for (; c < count; c += 4)
+    add(gload<v4f32>(rec + c * stride), gload<u32x4>(rec + c * stride + 16));
+  if (wave) {
+#pragma unroll
+    for (int j = 0; j < K + 2; j++) s_sum[wave - 1][j][lane] = d[j];
+    s_exact[wave - 1][lane] = exact ? 1u : 0u;
+  }
+  __syncthreads();
+  if (wave || g0 >= n_rows) return;
+#pragma unroll
+  for (int w = 0; w < 3; w++) {
+#pragma unroll
+    for (int j = 0; j < K + 2; j++) d[j] += s_sum[w][j][lane];
+    exact |= s_exact[w][lane] != 0u;
   }
   const float* R = reinterpret_cast<const float*>(J.r);
   auto elem = [&](uint64_t e) {
@@ -1539,10 +1605,11 @@ __global__ __launch_bounds__(256) void fused_rows(const FixJob* __restrict__ job
     for (uint64_t e = b0 / J.esz; e < b1 / J.esz; e++) {
       const float x = elem(e);
       const uint64_t col = e - (uint64_t)i * J.w;
-      for (uint32_t j = 0; j < J.k; j++)
-        d[j] += (double)x * (double)gload<float>(R + col * J.k + j);
-      s1 += fabs((double)x);
-      s2 += (double)x * (double)x;
+#pragma unroll
+      for (int j = 0; j < K; j++)
+        d[j] += (double)x * (double)gload<float>(R + col * K + j);
+      d[K] += fabs((double)x);
+      d[K + 1] += (double)x * (double)x;
     }
   };
   if (i == 0 && hc > H) rest(0, hc - H);
@@ -1550,18 +1617,19 @@ __global__ __launch_bounds__(256) void fused_rows(const FixJob* __restrict__ job
   if (exact) {  // a run met exponents out of fp32 squares' range: the row's sums in fp64
     // (|x| too: the chunk kernel takes a bf16 pair's |x| with v_dot2, whose subnormal inputs
     // are those of a pair marked here)
-    s1 = 0.0;
-    s2 = 0.0;
+    d[K] = 0.0;
+    d[K + 1] = 0.0;
     for (uint64_t e = (uint64_t)i * J.w; e < (uint64_t)(i + 1) * J.w; e++) {
       const double x = elem(e);
-      s1 += fabs(x);
-      s2 += x * x;
+      d[K] += fabs(x);
+      d[K + 1] += x * x;
     }
   }
   float* pdot = reinterpret_cast<float*>(J.pdot);
-  for (uint32_t j = 0; j < J.k; j++) gstore<float>(pdot + (uint64_t)i * J.k + j, (float)d[j]);
-  gstore<float>(reinterpret_cast<float*>(J.pabs) + i, (float)s1);
-  gstore<double>(reinterpret_cast<double*>(J.psq) + i, s2);
+#pragma unroll
+  for (int j = 0; j < K; j++) gstore<float>(pdot + (uint64_t)i * K + j, (float)d[j]);
+  gstore<float>(reinterpret_cast<float*>(J.pabs) + i, (float)d[K]);
+  gstore<double>(reinterpret_cast<double*>(J.psq) + i, d[K + 1]);
 }
 
 // ---- the plan ---------------------------------------------------------------------------
@@ -1592,7 +1660,7 @@ struct FvPlan {
   uint32_t* d_blk = nullptr;
   RedJob* d_red = nullptr;
   uint32_t n_red = 0;
-  uint64_t n_red_threads = 0;
+  uint32_t n_red_blocks = 0;
   FinJob* d_fin = nullptr;
   SliceJob* d_slices = nullptr;
   uint32_t n_slices = 0;
@@ -1950,11 +2018,15 @@ extern "C" int pots_fv_plan_create(size_t n, const pots_fv_product* prods, uint3
     a_chunks[twins[t].first] = tw[t].n_ct;
     a_chunks[twins[t].second] = tw[t].n_rt;
   }
+  uint64_t all_rows = 0;
+  for (size_t i = 0; i < n; i++) all_rows += prods[i].n;
+  uint32_t slice_most = 256;  // (a row per thread)
+  while (slice_most < kSliceRows && all_rows > 512ull * slice_most) slice_most *= 2;
   std::vector<SliceJob> slices;
   std::vector<uint32_t> slice_first(n), slice_rows(n), biased;
   for (size_t i = 0; i < n; i++) {
     const uint32_t chunks = std::max(a_chunks[i], jobs[2 * n + i].n_chunks);
-    uint32_t sr = kSliceRows;
+    uint32_t sr = slice_most;
     while (sr > 64 && (uint64_t)sr * chunks > 8ull * kSliceRows) sr /= 2;
     slice_rows[i] = sr;
     slice_first[i] = (uint32_t)slices.size();
@@ -2036,7 +2108,7 @@ extern "C" int pots_fv_plan_create(size_t n, const pots_fv_product* prods, uint3
   // (PassJob::pack); the reduction takes the others.
   std::vector<RedJob> red;
   red.reserve(n);
-  uint64_t gthreads = 0;
+  uint32_t red_blocks = 0;
   for (size_t i = 0; i < n; i++) {
     PassJob& J = ordered[pos[i]];
     if (J.n_chunks == 1 && prods[i].a_dtype == DT_BF16 && prods[i].b_dtype == DT_BF16) {
@@ -2054,16 +2126,16 @@ extern "C" int pots_fv_plan_create(size_t n, const pots_fv_product* prods, uint3
     R.vout = base + o_br + off_br[i];
     R.u = base + o_br + off_b1[i];
     R.w = base + o_br + off_b2[i];
-    R.group_first = gthreads;
+    R.blk_first = red_blocks;
     R.rows = prods[i].q;
     R.rows_pad = J.rows_pad;
     R.n_chunks = J.n_chunks;
     R.a_dt = prods[i].a_dtype;
     R.u_slots = twin_of[i] >= 0;  // a twin's |A|·b1 runs on the matrix cores
-    gthreads += (uint64_t)(pad32(prods[i].q) / 8) * k;
+    red_blocks += (uint32_t)(pad32(prods[i].q) / kRedRows);
   }
   P->n_red = (uint32_t)red.size();
-  P->n_red_threads = gthreads;
+  P->n_red_blocks = red_blocks;
   std::vector<FinJob> fin(n);
   for (size_t i = 0; i < n; i++) {
     const PassJob& A = ordered[pos[n + i]];
@@ -2195,7 +2267,7 @@ int fv_fuse_commit(void* fv, const std::vector<uint32_t>& prods,
   const size_t o_fix = place(prods.size() * sizeof(FixJob));
   uint64_t all_rows = 0;
   for (uint32_t i : prods) all_rows += P->h_prods[i].n;
-  const uint64_t fix_blocks = (all_rows + 255) / 256;
+  const uint64_t fix_blocks = (all_rows + kFixRows - 1) / kFixRows;
   const size_t o_fix_blk = place((fix_blocks + 1) * 4);
   std::vector<size_t> o_seg(prods.size());
   for (size_t f = 0; f < prods.size(); f++) {
@@ -2231,13 +2303,12 @@ int fv_fuse_commit(void* fv, const std::vector<uint32_t>& prods,
     x.head = head_len[f];
     x.esz = p.p_dtype == DT_BF16 ? 2 : 4;
     x.J = (uint32_t)(((uint64_t)p.w * x.esz + 1023) / 1024 + 1);
-    x.k = P->k;
     rows += p.n;
     (*seg_out)[f] = x.seg;
   }
   std::vector<uint32_t> fix_blk(fix_blocks + 1);
   for (size_t f = 0, b = 0; b < fix_blocks; b++) {
-    while (f + 1 < fix.size() && fix[f + 1].row_first <= b * 256) f++;
+    while (f + 1 < fix.size() && fix[f + 1].row_first <= b * kFixRows) f++;
     fix_blk[b] = (uint32_t)f;
   }
   fix_blk[fix_blocks] = fix.empty() ? 0u : (uint32_t)(fix.size() - 1);
@@ -2370,14 +2441,13 @@ static int run_stage(FvPlan* P, int stage, const uint8_t* d_key, double* d_rows,
       for (const PassLaunch& L : P->pass_b)
         if ((rc = run_pass(P, L, 1, s)) != POTS_E_OK) return rc;
       return POTS_E_OK;
-    case 2: {
-      const uint64_t blocks = (P->n_red_threads + 255) / 256;
-      if (blocks == 0) return POTS_E_OK;
-      hipLaunchKernelGGL(reduce_b, dim3((uint32_t)blocks), dim3(256), 0, s, P->d_red, P->n_red,
-                         P->n_red_threads, P->k);
+    case 2:
+      if (P->n_red_blocks == 0) return POTS_E_OK;
+      hipLaunchKernelGGL(reduce_b, dim3(P->n_red_blocks), dim3(256),
+                         (kRedRows * P->k + kRedRows) * sizeof(float), s, P->d_red, P->n_red,
+                         P->k);
       POTS_HIP(hipGetLastError());
       return POTS_E_OK;
-    }
     case 3:  // the A pass: the row pass over the A's that are no twin's, then the twins'
       if ((rc = run_stage(P, POTS_FV_STAGE_A_ROWS, d_key, d_rows, s)) != POTS_E_OK) return rc;
       return run_stage(P, POTS_FV_STAGE_TWINS, d_key, d_rows, s);
@@ -2406,8 +2476,9 @@ static int run_stage(FvPlan* P, int stage, const uint8_t* d_key, double* d_rows,
     case POTS_FV_STAGE_P_FUSED:
       if (P->fused) {
         if (P->n_fix == 0) return POTS_E_HIP;  // a fusion that failed half way
-        hipLaunchKernelGGL(fused_rows, dim3((uint32_t)((P->n_fix_rows + 255) / 256)), dim3(256),
-                           0, s, P->d_fix, P->d_fix_blk, P->n_fix_rows);
+        const auto kernel = P->k == 1 ? fused_rows<1> : P->k == 2 ? fused_rows<2> : fused_rows<4>;
+        hipLaunchKernelGGL(kernel, dim3((uint32_t)((P->n_fix_rows + kFixRows - 1) / kFixRows)),
+                           dim3(256), 0, s, P->d_fix, P->d_fix_blk, P->n_fix_rows);
         POTS_HIP(hipGetLastError());
       }
       return POTS_E_OK;
@@ -2420,9 +2491,8 @@ static int run_stage(FvPlan* P, int stage, const uint8_t* d_key, double* d_rows,
       hipLaunchKernelGGL(finish_slices, dim3(P->n_slices), dim3(256), 0, s, P->d_fin,
                          P->d_slices, P->k, P->d_bout, P->d_br, P->d_recs);
       POTS_HIP(hipGetLastError());
-      hipLaunchKernelGGL(finish_final, dim3((uint32_t)((P->n + 255) / 256)), dim3(256), 0, s,
-                         P->d_fin, (uint32_t)P->n, P->k, P->guard, P->d_bout, P->d_recs,
-                         d_rows);
+      hipLaunchKernelGGL(finish_final, dim3((uint32_t)P->n), dim3(64), 0, s, P->d_fin, P->k,
+                         P->guard, P->d_bout, P->d_recs, d_rows);
       POTS_HIP(hipGetLastError());
       return POTS_E_OK;
     default:
