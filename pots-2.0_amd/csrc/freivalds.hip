@@ -98,7 +98,7 @@ struct PassJob {
   uint32_t n_chunks, n_rg;  // column chunks; 64-row groups
   uint32_t n_jg, n_jt;      // 16-slot column groups; blocks per (row group, chunk)
   uint64_t block_first;     // prefix of blocks over the launch's jobs before it
-  uint32_t aligned;         // 16-byte aligned rows and base
+  uint32_t narrow;          // 16 rows lie within 32-bit offsets (16-byte loads)
   uint32_t pack;            // a B-pass job of one column chunk for a bf16 A pass: bit 0, the
                             // pass writes the reduction's outputs itself (vout, uo, wo) in
                             // place of partials; bit 1, also b1's terms in slots 12..14
@@ -176,13 +176,34 @@ struct Lane {
   uint32_t voff;      // this lane's V bytes past vjt (its K-group, its slot)
   uint32_t g, c1;
   uint32_t nvalid;    // groups of this block that exist (the last block of a row may hold fewer)
-  bool kaligned;      // an aligned job whose chunk ends on a K-step: its last partial stage
-                      // takes load_partial
+  bool narrow;        // the job's 16 rows lie within 32-bit offsets: its partial stages take
+                      // load_partial, its others load_full
   brsrc xr, vr;       // buffer resources at xbase and vjt (the full and partial stages' and
                       // the V staging's loads)
 };
 
-// A whole stage of an aligned job, every column inside the chunk: plain 16-byte loads.
+// This lane's columns of the K-step at cu, one element at a time; columns past c1 read as zero.
+template <uint32_t XT>
+__device__ __forceinline__ u32x4 load_elements(const Lane& L, uint32_t cu) {
+  using G = Geo<XT>;
+  const uint32_t cl = cu + G::PER * L.g;
+  if (XT == DT_BF16) {
+    const uint16_t* p = reinterpret_cast<const uint16_t*>(L.xrow);
+    uint32_t e[8];
+#pragma unroll
+    for (uint32_t t = 0; t < 8; t++) e[t] = cl + t < L.c1 ? gload<uint16_t>(p + cl + t) : 0u;
+    return u32x4{e[0] | e[1] << 16, e[2] | e[3] << 16, e[4] | e[5] << 16, e[6] | e[7] << 16};
+  }
+  const uint32_t* p = reinterpret_cast<const uint32_t*>(L.xrow);
+  uint32_t e[4];
+#pragma unroll
+  for (uint32_t t = 0; t < 4; t++) e[t] = cl + t < L.c1 ? gload<uint32_t>(p + cl + t) : 0u;
+  return u32x4{e[0], e[1], e[2], e[3]};
+}
+
+// A whole stage of a narrow job, every column inside the chunk: plain 16-byte loads, at
+// whatever alignment the rows have (gfx950 loads take any; a row that is not 16-byte aligned
+// costs its wave the lines two lanes share).
 template <uint32_t XT, uint32_t NJG, bool VS>
 __device__ __forceinline__ void load_full(StageRegs<NJG, VS>& r, const Lane& L, uint32_t cs) {
   using G = Geo<XT>;
@@ -202,10 +223,11 @@ __device__ __forceinline__ void load_full(StageRegs<NJG, VS>& r, const Lane& L, 
   }
 }
 
-// The last, partial stage of an aligned job's chunk whose columns end on a K-step (a narrow
-// X, such as an attention head's 64 columns, is one such stage per row): K-steps inside the
-// chunk take one 16-byte load per lane, the rest read as zero, and so does the lane's own V
-// of K-steps past c1 (V rows past the matrix are zero in memory).
+// The last, partial stage of a narrow job's chunk (a narrow X, such as an attention head's 64
+// columns, is one such stage per row): K-steps inside the chunk take one 16-byte load per lane,
+// the K-step across the chunk's end, if there is one, element loads under a column guard, and
+// the rest read as zero, as does the lane's own V of K-steps past c1 (V rows past the matrix
+// are zero in memory).
 template <uint32_t XT, uint32_t NJG, bool VS>
 __device__ __forceinline__ void load_partial(StageRegs<NJG, VS>& r, const Lane& L,
                                              uint32_t cs) {
@@ -213,7 +235,10 @@ __device__ __forceinline__ void load_partial(StageRegs<NJG, VS>& r, const Lane& 
 #pragma unroll
   for (uint32_t u = 0; u < KU; u++) {
     const uint32_t cu = cs + u * G::KSTEP;
-    r.x[u] = cu < L.c1 ? bload128(L.xr, L.xoff, cu * G::ESZ) : u32x4{0, 0, 0, 0};
+    if (cu + G::KSTEP <= L.c1 || cu >= L.c1)
+      r.x[u] = cu < L.c1 ? bload128(L.xr, L.xoff, cu * G::ESZ) : u32x4{0, 0, 0, 0};
+    else
+      r.x[u] = load_elements<XT>(L, cu);
     if constexpr (!VS) {
       const uint32_t vb = (cu / G::PER) * (uint32_t)L.vstep;  // uniform
 #pragma unroll
@@ -229,9 +254,9 @@ __device__ __forceinline__ void load_partial(StageRegs<NJG, VS>& r, const Lane& 
   __builtin_amdgcn_s_waitcnt(0x0F70);
 }
 
-// A stage that may run past the chunk's end across a K-step, or of an unaligned job: element
-// loads with a column guard; columns past c1 read as zero, and so does the lane's own V of
-// K-steps past c1 (V rows past the matrix are zero in memory).
+// Any stage of a job whose 16 rows span more than the 32-bit offsets: element loads from
+// 64-bit addresses under a column guard; columns past c1 read as zero, and so does the lane's
+// own V of K-steps past c1.
 template <uint32_t XT, uint32_t NJG, bool VS>
 __device__ __forceinline__ void load_guarded(StageRegs<NJG, VS>& r, const Lane& L,
                                              uint32_t cs) {
@@ -239,20 +264,7 @@ __device__ __forceinline__ void load_guarded(StageRegs<NJG, VS>& r, const Lane& 
 #pragma unroll
   for (uint32_t u = 0; u < KU; u++) {
     const uint32_t cu = cs + u * G::KSTEP;
-    const uint32_t cl = cu + G::PER * L.g;
-    if (XT == DT_BF16) {
-      const uint16_t* p = reinterpret_cast<const uint16_t*>(L.xrow);
-      uint32_t e[8];
-#pragma unroll
-      for (uint32_t t = 0; t < 8; t++) e[t] = cl + t < L.c1 ? gload<uint16_t>(p + cl + t) : 0u;
-      r.x[u] = u32x4{e[0] | e[1] << 16, e[2] | e[3] << 16, e[4] | e[5] << 16, e[6] | e[7] << 16};
-    } else {
-      const uint32_t* p = reinterpret_cast<const uint32_t*>(L.xrow);
-      uint32_t e[4];
-#pragma unroll
-      for (uint32_t t = 0; t < 4; t++) e[t] = cl + t < L.c1 ? gload<uint32_t>(p + cl + t) : 0u;
-      r.x[u] = u32x4{e[0], e[1], e[2], e[3]};
-    }
+    r.x[u] = load_elements<XT>(L, cu);
     if constexpr (!VS) {
       const char* vp = L.vlane + (uint64_t)(cu / G::PER) * L.vstep;
 #pragma unroll
@@ -541,19 +553,18 @@ __device__ __forceinline__ void row_tile(const PassJob* __restrict__ jobs,
   L.voff = (uint32_t)((uint64_t)g * L.vstep) + i * 16;
   L.vlane = L.vjt + L.voff;
   // the same addresses as uniform bases and 32-bit lane offsets (plan creation keeps 16 rows
-  // of an aligned job's X below 2^31 bytes; 4 K-groups of V are far below)
+  // of a narrow job's X below 2^31 bytes; 4 K-groups of V are far below)
   L.xbase = reinterpret_cast<const char*>(J.x) + (uint64_t)r0 * J.ld * G::ESZ;
   L.xoff = (uint32_t)((uint64_t)(rowc - r0) * J.ld * G::ESZ) + G::PER * g * G::ESZ;
   L.g = g;
   L.c1 = c1;
   L.nvalid = min(NJG, J.n_jg - jt * NJG);
-  L.kaligned = J.aligned != 0 && (c1 - c0) % G::KSTEP == 0;
+  L.narrow = J.narrow != 0;
   L.xr = make_rsrc(L.xbase);
   L.vr = make_rsrc(L.vjt);
-  // The chunk's stages: the first nfull of an aligned job are whole (plain 16-byte loads);
-  // an aligned chunk's last partial stage takes load_partial when the chunk ends on a K-step,
-  // else the guarded loads, which every stage of an unaligned job takes.
-  const uint32_t nfull = J.aligned ? (c1 - c0) / SSTEP : 0;
+  // The chunk's stages: the first nfull of a narrow job are whole (plain 16-byte loads), its
+  // last, if partial, takes load_partial; every stage of any other job takes load_guarded.
+  const uint32_t nfull = J.narrow ? (c1 - c0) / SSTEP : 0;
   const uint32_t nst = (c1 - c0 + SSTEP - 1) / SSTEP;
   u32x4* const sv0 = s_v;
   u32x4* const sv1 = s_v + VStage<NJG>::kUnits;
@@ -565,7 +576,7 @@ __device__ __forceinline__ void row_tile(const PassJob* __restrict__ jobs,
   if constexpr (VS) vstage_load<XT, NJG>(vs, L, c0);
   if (active) {
     if (nfull > 0) load_full<XT, NJG, VS>(ra, L, c0);
-    else if (L.kaligned) load_partial<XT, NJG, VS>(ra, L, c0);
+    else if (L.narrow) load_partial<XT, NJG, VS>(ra, L, c0);
     else load_guarded<XT, NJG, VS>(ra, L, c0);
   }
   if (WEIGHTED && sums) stage_weights<G::CHUNK>(J.u, J.w, c0, c1, J.chunk_cols, s_u, s_w);
@@ -594,7 +605,7 @@ __device__ __forceinline__ void row_tile(const PassJob* __restrict__ jobs,
       if constexpr (VS) vstage_load<XT, NJG>(vs, L, cs + SSTEP);
       if (active) {
         if (s + 1 < nfull) load_full<XT, NJG, VS>(nxt, L, cs + SSTEP);
-        else if (L.kaligned) load_partial<XT, NJG, VS>(nxt, L, cs + SSTEP);
+        else if (L.narrow) load_partial<XT, NJG, VS>(nxt, L, cs + SSTEP);
         else load_guarded<XT, NJG, VS>(nxt, L, cs + SSTEP);
       } else {
         __builtin_amdgcn_s_waitcnt(0x0F70);
@@ -1848,10 +1859,9 @@ extern "C" int pots_fv_plan_create(size_t n, const pots_fv_product* prods, uint3
     J.n_jg = groups_for(s.dt, k);
     J.n_jt = (J.n_jg + njg_for(s.dt, k) - 1) / njg_for(s.dt, k);
     const uint32_t esz = s.dt == DT_BF16 ? 2 : 4;
-    // The full stages address a wave's 16 rows by 32-bit offsets from its first row: a row
+    // The 16-byte loads address a wave's 16 rows by 32-bit offsets from its first row: a row
     // stride beyond that (rows of over 128 MiB) takes the guarded loads' 64-bit addresses.
-    J.aligned = (s.x % 16 == 0) && ((s.ld * esz) % 16 == 0) &&
-                (uint64_t)s.ld * esz * 16 < (1ull << 31);
+    J.narrow = (uint64_t)s.ld * esz * 16 < (1ull << 31);
     return J;
   };
   // Partial buffers, per job: dot [chunks][rows_pad][k] f32, abs [chunks][rows_pad] f32,
