@@ -1709,6 +1709,16 @@ struct FvPlan {
 // the matrix are zero.
 static uint64_t pad32(uint64_t rows) { return (rows + 31) / 32 * 32; }
 
+// How far a pass's chunks are cut for the sake of tiles: the tiles it should have, and the
+// columns a chunk keeps at least. A bf16 B keeps more: of one chunk, it packs the A pass's
+// operand itself, and cutting it costs the reduction's launch. Passes of 100 to 8192 rows,
+// us, with whole chunks / these: the B, A and P passes of six 100 x 390 x 257 fp32 products
+// 12, 14, 12 / 11, 9, 10; of eight 1000 x 2050 x 1537 bf16 ones under sixteen challenges 49, 30,
+// 33 / 45, 24, 24; the B pass of an 8192 x 4096 x 4096 fp32 one 25 / 17. (2048 tiles wanted:
+// its A pass 28 -> 35, each chunk's partials costing more than its block hides.)
+constexpr uint64_t kTilesWanted = 1024;
+constexpr uint32_t kLeastF32 = 128, kLeastBf16 = 512, kLeastBf16B = 1024;
+
 static uint32_t chunk_cols_for(uint32_t cols, uint32_t sstep, uint32_t cmax) {
   // At most cmax columns per chunk, in whole pipeline stages, balanced over the chunks (cmax
   // is a multiple of the stage width, so rounding up stays within it).
@@ -1843,7 +1853,47 @@ extern "C" int pots_fv_plan_create(size_t n, const pots_fv_product* prods, uint3
     uint32_t rows, cols, dt;
     uint64_t x, ld;
   };
-  auto make_job = [&](const Shape& s) {
+  // Columns per chunk at most, by pass and dtype: Geo's CHUNK, halved while the pass would have
+  // fewer than kTilesWanted tiles. A tile is a chain of stages, each a load's latency, and it
+  // takes several blocks on a CU to hide one another's.
+  auto chunk_most = [&](uint32_t dt, uint32_t most, uint32_t least, auto&& shape_of) {
+    for (; most > least; most /= 2) {
+      uint64_t tiles = 0;
+      for (size_t i = 0; i < n && tiles < kTilesWanted; i++) {
+        const Shape s = shape_of(i);
+        if (s.dt == dt)
+          tiles += (uint64_t)((s.rows + kRowsPerBlock - 1) / kRowsPerBlock) *
+                   ((s.cols + most - 1) / most);
+      }
+      if (tiles >= kTilesWanted || tiles == 0) break;
+    }
+    return most;
+  };
+  auto b_shape = [&](size_t i) {
+    const pots_fv_product& p = prods[i];
+    return Shape{p.q, p.w, p.b_dtype, reinterpret_cast<uint64_t>(p.b), p.ldb};
+  };
+  auto a_shape = [&](size_t i) {
+    const pots_fv_product& p = prods[i];
+    return Shape{p.n, p.q, p.a_dtype, reinterpret_cast<uint64_t>(p.a), p.lda};
+  };
+  auto p_shape = [&](size_t i) {
+    const pots_fv_product& p = prods[i];
+    return Shape{p.n, p.w, p.p_dtype, reinterpret_cast<uint64_t>(p.p), p.ldp};
+  };
+  auto a_rows_shape = [&](size_t i) {  // of the A row pass: a twin's A is not in it
+    Shape s = a_shape(i);
+    if (twin_of[i] >= 0) s.dt = 2;
+    return s;
+  };
+  constexpr uint32_t kF32 = Geo<DT_F32>::CHUNK, kBf16 = Geo<DT_BF16>::CHUNK;
+  const uint32_t b_most[2] = {chunk_most(DT_F32, kF32, kLeastF32, b_shape),
+                              chunk_most(DT_BF16, kBf16, kLeastBf16B, b_shape)};
+  const uint32_t a_most[2] = {chunk_most(DT_F32, kF32, kLeastF32, a_rows_shape),
+                              chunk_most(DT_BF16, kBf16, kLeastBf16, a_rows_shape)};
+  const uint32_t p_most[2] = {chunk_most(DT_F32, kF32, kLeastF32, p_shape),
+                              chunk_most(DT_BF16, kBf16, kLeastBf16, p_shape)};
+  auto make_job = [&](const Shape& s, const uint32_t (&most)[2]) {
     PassJob J;
     memset(&J, 0, sizeof J);
     J.x = s.x;
@@ -1852,8 +1902,8 @@ extern "C" int pots_fv_plan_create(size_t n, const pots_fv_product* prods, uint3
     J.cols = s.cols;
     J.rows_pad = (s.rows + kRowsPerBlock - 1) / kRowsPerBlock * kRowsPerBlock;
     J.chunk_cols = s.dt == DT_BF16
-                       ? chunk_cols_for(s.cols, Geo<DT_BF16>::KSTEP * KU, Geo<DT_BF16>::CHUNK)
-                       : chunk_cols_for(s.cols, Geo<DT_F32>::KSTEP * KU, Geo<DT_F32>::CHUNK);
+                       ? chunk_cols_for(s.cols, Geo<DT_BF16>::KSTEP * KU, most[DT_BF16])
+                       : chunk_cols_for(s.cols, Geo<DT_F32>::KSTEP * KU, most[DT_F32]);
     J.n_chunks = (s.cols + J.chunk_cols - 1) / J.chunk_cols;
     J.n_rg = J.rows_pad / kRowsPerBlock;
     J.n_jg = groups_for(s.dt, k);
@@ -1882,7 +1932,7 @@ extern "C" int pots_fv_plan_create(size_t n, const pots_fv_product* prods, uint3
   std::vector<size_t> off_br, off_b1, off_b2;
   for (size_t i = 0; i < n; i++) {
     const pots_fv_product& p = prods[i];
-    PassJob J = make_job({p.q, p.w, p.b_dtype, reinterpret_cast<uint64_t>(p.b), p.ldb});
+    PassJob J = make_job(b_shape(i), b_most);
     jobs.push_back(J);
     reserve_part(J);
     const uint64_t qpad = pad32(p.q);
@@ -1898,8 +1948,7 @@ extern "C" int pots_fv_plan_create(size_t n, const pots_fv_product* prods, uint3
                 (uint64_t)p.n * p.w * (p.p_dtype == DT_BF16 ? 2 : 4);
   }
   for (size_t i = 0; i < n; i++) {
-    const pots_fv_product& p = prods[i];
-    PassJob J = make_job({p.n, p.q, p.a_dtype, reinterpret_cast<uint64_t>(p.a), p.lda});
+    PassJob J = make_job(a_shape(i), a_most);
     jobs.push_back(J);
     if (twin_of[i] >= 0) {  // its A pass is the twin job's: no row-pass partials
       J.n_chunks = 0;
@@ -1908,8 +1957,7 @@ extern "C" int pots_fv_plan_create(size_t n, const pots_fv_product* prods, uint3
     reserve_part(J);
   }
   for (size_t i = 0; i < n; i++) {
-    const pots_fv_product& p = prods[i];
-    PassJob J = make_job({p.n, p.w, p.p_dtype, reinterpret_cast<uint64_t>(p.p), p.ldp});
+    PassJob J = make_job(p_shape(i), p_most);
     jobs.push_back(J);
     reserve_part(J);
   }
