@@ -764,17 +764,69 @@ __global__ __launch_bounds__(kThreads) void level_kernel(
                      cur[tid]);
 }
 
-__global__ void fill_u32(uint32_t* p, uint32_t v) { *p = v; }
+// Messages that are not word aligned where they lie (a record, a view at an odd element) are
+// staged: 0x00 || header || payload in one aligned buffer. One launch writes them all, 16 bytes
+// a thread, and resets the first-bad word; a payload in host memory (to == head) is copied in
+// after it. (Two device copies per leaf and the reset, each a launch of its own, were 17 launches
+// and about 80 us for eight records.)
+struct StageJob {
+  uint64_t dst;      // the staged message, 16-byte aligned, with room to a multiple of 16 bytes
+  uint64_t head;     // device address of the head bytes in the metadata region
+  uint64_t payload;  // device address of the payload, at any alignment
+  uint64_t head_bytes;
+  uint64_t to;        // message bytes to write
+  uint64_t blk_first;  // prefix of blocks over the jobs before it
+};
+static_assert(sizeof(StageJob) == 48, "StageJob layout");
+constexpr uint32_t kStageBytes = 16 * kThreads;  // of a message, per block
+
+__global__ __launch_bounds__(kThreads) void stage_kernel(const StageJob* __restrict__ jobs,
+                                                         uint32_t n_jobs, uint32_t* first_bad,
+                                                         uint32_t n_leaves) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *first_bad = n_leaves;
+  if (n_jobs == 0) return;
+  uint32_t lo = 0, hi = n_jobs - 1;
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi + 1) >> 1;
+    if (jobs[mid].blk_first <= blockIdx.x) lo = mid;
+    else hi = mid - 1;
+  }
+  const StageJob J = jobs[lo];
+  const uint64_t m0 = (blockIdx.x - J.blk_first) * kStageBytes + 16ull * threadIdx.x;
+  if (m0 >= J.to) return;
+  const char* head = reinterpret_cast<const char*>(J.head);
+  const char* payload = reinterpret_cast<const char*>(J.payload);
+  u32x4 v = {0, 0, 0, 0};
+  if (m0 >= J.head_bytes && m0 + 16 <= J.to) {
+    // the aligned words the sixteen bytes lie in, none of them past the payload's last
+    const uint64_t src = J.payload + (m0 - J.head_bytes);
+    const char* at = reinterpret_cast<const char*>(src & ~uint64_t(3));
+    const uint32_t sh = 8 * (uint32_t)(src & 3);
+    const u32x4 w = gload<u32x4w>(at);
+    if (sh == 0) {
+      v = w;
+    } else {
+      const uint32_t last = gload<uint32_t>(at + 16);
+#pragma unroll
+      for (int t = 0; t < 4; t++) v[t] = (w[t] >> sh) | ((t < 3 ? w[t + 1] : last) << (32 - sh));
+    }
+  } else {
+#pragma unroll
+    for (uint32_t t = 0; t < 16; t++) {
+      const uint64_t m = m0 + t;
+      uint32_t byte = 0;
+      if (m < J.head_bytes) byte = gload<uint8_t>(head + m);
+      else if (m < J.to) byte = gload<uint8_t>(payload + (m - J.head_bytes));
+      v[t / 4] |= byte << (8 * (t % 4));
+    }
+  }
+  gstore<u32x4>(reinterpret_cast<char*>(J.dst) + m0, v);
+}
 
 // ---- host side ----------------------------------------------------------------------------
 
-struct StageCopy {  // a staged leaf: its head bytes, then its payload, into one aligned buffer
-  uint64_t dst;         // device address of the staged message
-  uint64_t head_src;    // device address of the head bytes in the metadata region
-  uint64_t head_bytes;
-  uint64_t payload_src; // payload address (host or device)
-  uint64_t payload_bytes;
-  bool host;            // payload in host memory
+struct HostCopy {  // a staged leaf's payload in host memory, copied into its staged message
+  uint64_t dst, src, bytes;
 };
 
 struct LevelInfo {
@@ -805,7 +857,9 @@ struct LeafPlan {
   uint32_t* d_cv[2] = {nullptr, nullptr};
   uint32_t max_grid = 0;  // chunk kernel's grid limit; 0 = one block per slot
   std::vector<LevelInfo> levels;
-  std::vector<StageCopy> stages;
+  StageJob* d_stages = nullptr;
+  uint32_t n_stages = 0, stage_blocks = 0;
+  std::vector<HostCopy> host_copies;  // after the staging kernel
 };
 
 // Build the plan's host image and sizes. `device_only` refuses host payloads.
@@ -906,8 +960,9 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
   std::vector<uint8_t> headbytes;  // word-aligned heads of direct leaves, then staged heads
   OrderHost plain, fused;
   std::vector<int64_t> stage_head_at(n, -1);
-  uint64_t stage_bytes = 0;
+  uint64_t stage_bytes = 0, stage_blocks = 0;
   std::vector<uint64_t> stage_off(n, 0);
+  std::vector<StageJob> stages;  // offsets until the plan's memory is placed
   std::vector<FuseDesc> fdesc;                 // per fused leaf
   std::vector<uint32_t> fprod, fhead;          // its product and head bytes
   std::unordered_set<uint32_t> fused_prods;
@@ -949,7 +1004,10 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
       d.len = hl + len;
       d.head_word = 0;
       d.head_len = 0;
-      P->stages.push_back(StageCopy{stage_off[i], at, hl, ptr, len, host});
+      const uint64_t to = host ? hl : hl + len;
+      stages.push_back(StageJob{stage_off[i], at, ptr, hl, to, stage_blocks});
+      stage_blocks += (to + kStageBytes - 1) / kStageBytes;
+      if (host) P->host_copies.push_back(HostCopy{stage_off[i] + hl, ptr, len});
     }
     const uint64_t L = hl + len;
     if (L >> 42) {  // 2^32 chunks: the chunk kernel's 32-bit counter
@@ -1003,7 +1061,7 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
   }
   P->n_chunks = nc;
   P->n_fused = (uint32_t)fdesc.size();
-  if (headbytes.size() / 4 >= 0xFFFFFFFFull) {
+  if (headbytes.size() / 4 >= 0xFFFFFFFFull || stage_blocks >= 0x7FFFFFFFull) {
     delete P;
     return POTS_E_ARG;
   }
@@ -1081,6 +1139,7 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
   const size_t o_head = place(std::max<size_t>(headbytes.size(), 4));
   const size_t o_lev = place(std::max<size_t>(ents.size(), 1) * sizeof(LevelEntry));
   const size_t o_blk_ent = place(std::max<size_t>(blk_ent.size(), 1) * sizeof(uint32_t));
+  const size_t o_stages = place(std::max<size_t>(stages.size(), 1) * sizeof(StageJob));
   const size_t meta_bytes = at;
   const size_t o_cv0 = place(nc * 32);
   const size_t o_cv1 = place(std::max<uint64_t>(cv1_need, 1) * 32);
@@ -1114,14 +1173,16 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
     P->base = static_cast<char*>(p);
   }
   const uint64_t B = reinterpret_cast<uint64_t>(P->base);
-  for (size_t i = 0, s = 0; i < n; i++) {
-    if (stage_head_at[i] >= 0) {
-      desc[i].payload = B + o_stage + stage_off[i];
-      StageCopy& sc = P->stages[s++];
-      sc.dst = B + o_stage + sc.dst;
-      sc.head_src = B + o_head + sc.head_src;
-    }
+  for (size_t i = 0; i < n; i++)
+    if (stage_head_at[i] >= 0) desc[i].payload = B + o_stage + stage_off[i];
+  for (StageJob& j : stages) {
+    j.dst += B + o_stage;
+    j.head += B + o_head;
   }
+  for (HostCopy& c : P->host_copies) c.dst += B + o_stage;
+  P->d_stages = reinterpret_cast<StageJob*>(P->base + o_stages);
+  P->n_stages = (uint32_t)stages.size();
+  P->stage_blocks = (uint32_t)stage_blocks;
   P->d_leaves = reinterpret_cast<LeafDesc*>(P->base + o_leaves);
   P->d_fuse = reinterpret_cast<FuseDesc*>(P->base + o_fuse);
   Order* dords[2] = {&P->plain, &P->fused};
@@ -1164,6 +1225,8 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
     memcpy(img.data() + o_ord[k][2], ords[k]->blk_ent.data(),
            ords[k]->blk_ent.size() * sizeof(uint32_t));
   }
+  if (!stages.empty())
+    memcpy(img.data() + o_stages, stages.data(), stages.size() * sizeof(StageJob));
   if (!headbytes.empty()) memcpy(img.data() + o_head, headbytes.data(), headbytes.size());
   if (!ents.empty()) memcpy(img.data() + o_lev, ents.data(), ents.size() * sizeof(LevelEntry));
   if (!blk_ent.empty())
@@ -1186,17 +1249,11 @@ static int plan_stage(LeafPlan* P, int stage, uint32_t* d_digests, uint32_t* d_f
   int rc;
   switch (stage) {
     case 0:
-      for (const StageCopy& s : P->stages) {
-        POTS_HIP(hipMemcpyAsync(reinterpret_cast<void*>(s.dst),
-                                reinterpret_cast<const void*>(s.head_src), s.head_bytes,
-                                hipMemcpyDeviceToDevice, stream));
-        if (s.payload_bytes)
-          POTS_HIP(hipMemcpyAsync(reinterpret_cast<void*>(s.dst + s.head_bytes),
-                                  reinterpret_cast<const void*>(s.payload_src), s.payload_bytes,
-                                  s.host ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice,
-                                  stream));
-      }
-      hipLaunchKernelGGL(fill_u32, dim3(1), dim3(1), 0, stream, d_first_bad, (uint32_t)P->n);
+      hipLaunchKernelGGL(stage_kernel, dim3(std::max(1u, P->stage_blocks)), dim3(kThreads), 0,
+                         stream, P->d_stages, P->n_stages, d_first_bad, (uint32_t)P->n);
+      for (const HostCopy& c : P->host_copies)
+        POTS_HIP(hipMemcpyAsync(reinterpret_cast<void*>(c.dst), reinterpret_cast<const void*>(c.src),
+                                c.bytes, hipMemcpyHostToDevice, stream));
       POTS_HIP(hipGetLastError());
       return POTS_E_OK;
     case 1:  // both chunk kernels: the fused leaves' (3), then the others' (4)
