@@ -206,6 +206,11 @@ typedef struct {
 int pots_fv_plan_create(size_t n, const pots_fv_product *products, uint32_t k, uint32_t guard,
                         void **plan);
 
+/* Enqueue on `stream`: the 32 bytes at `key` (host memory, read before the call returns) to
+ * d_key (device memory, 4-byte aligned), for the calls below that take a device-resident root.
+ * No copy, no sync, no allocation. No counterpart in the reference. */
+int pots_set_key_async(uint8_t *d_key, const uint8_t key[32], void *stream);
+
 /* Enqueue on `stream`: the challenge matrices keyed on the 32-byte d_key (device memory,
  * the claimed root), the three streaming passes and the reduction, writing one fp64 row per
  * product to d_rows [n][5 + k] in freivalds.ROW order (freivalds.py:255): nu, ‖|P|1‖, ‖P‖_F,

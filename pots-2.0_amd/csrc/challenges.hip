@@ -77,7 +77,7 @@ __global__ __launch_bounds__(256) void xof_kernel(const uint32_t* __restrict__ k
       uint16_t pl[3][8];
 #pragma unroll
       for (int e = 0; e < 8; e++) split_bf16x3(r[8 * h + e], pl[0][e], pl[1][e], pl[2][e]);
-      uint16_t* grp = out_b3 + it.pk_off + (((uint64_t)(2 * t + h) * njg + jg) * 16 + slot) * 8;
+      uint16_t* grp = out_b3 + it.b3_off + (((uint64_t)(2 * t + h) * njg + jg) * 16 + slot) * 8;
 #pragma unroll
       for (int p = 0; p < 3; p++)
         *reinterpret_cast<uint4*>(grp + 8 * p) =
@@ -91,7 +91,7 @@ __global__ __launch_bounds__(256) void xof_kernel(const uint32_t* __restrict__ k
 #pragma unroll
     for (int h = 0; h < 4; h++) {
       float4* dst = reinterpret_cast<float4*>(
-          out_f4 + it.pk_off + (((uint64_t)(4 * t + h) * njg + jg) * 16 + slot) * 4);
+          out_f4 + it.f4_off + (((uint64_t)(4 * t + h) * njg + jg) * 16 + slot) * 4);
       *dst = make_float4(r[4 * h], r[4 * h + 1], r[4 * h + 2], r[4 * h + 3]);
     }
   }
@@ -110,9 +110,28 @@ int challenges_enqueue(const uint32_t* d_key, const ChallengeItem* d_items, uint
   return POTS_E_OK;
 }
 
+// A root given by the host, as the launch's arguments: no copy, nothing to wait for.
+struct Key {
+  uint32_t w[8];
+};
+
+__global__ void set_key(uint32_t* __restrict__ dst, Key key) {
+  if (threadIdx.x < 8) dst[threadIdx.x] = key.w[threadIdx.x];
+}
+
 }  // namespace pots
 
 using namespace pots;
+
+extern "C" int pots_set_key_async(uint8_t* d_key, const uint8_t key[32], void* stream) {
+  if (!d_key || !key || reinterpret_cast<uintptr_t>(d_key) % 4 != 0) return POTS_E_ARG;
+  Key k;
+  memcpy(k.w, key, 32);
+  hipLaunchKernelGGL(set_key, dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream),
+                     reinterpret_cast<uint32_t*>(d_key), k);
+  POTS_HIP(hipGetLastError());
+  return POTS_E_OK;
+}
 
 extern "C" int pots_challenges(const uint8_t key[32], uint32_t k, size_t n, const uint32_t* ms,
                                const uint32_t* widths, const uint64_t* offsets, float* out,
@@ -125,7 +144,7 @@ extern "C" int pots_challenges(const uint8_t key[32], uint32_t k, size_t n, cons
   uint64_t units = 0, end = 0;
   for (size_t i = 0; i < n; i++) {
     if (ms[i] == 0 || widths[i] == 0) return POTS_E_ARG;
-    items[i] = ChallengeItem{ms[i], widths[i], offsets[i], 0, units};
+    items[i] = ChallengeItem{ms[i], widths[i], offsets[i], 0, 0, units};
     units += (widths[i] + 15) / 16;
     end = std::max<uint64_t>(end, offsets[i] + (uint64_t)widths[i] * k);
   }

@@ -9,16 +9,16 @@
 namespace pots {
 
 // One challenge matrix: product label m, its width (rows of R), where its row-major [width, k]
-// fp32 copy goes (float offset) and where its packed copy goes (element offset), and the
-// prefix of 16-row XOF units over the items before it.
+// fp32 copy and its packed copies go (element offsets), and the prefix of 16-row XOF units over
+// the items before it.
 struct ChallengeItem {
   uint32_t m;
   uint32_t width;
   uint64_t out_off;
-  uint64_t pk_off;
+  uint64_t b3_off, f4_off;
   uint64_t unit_first;
 };
-static_assert(sizeof(ChallengeItem) == 32, "ChallengeItem layout");
+static_assert(sizeof(ChallengeItem) == 40, "ChallengeItem layout");
 
 // The packed operands of the row pass hold each K-group of PER rows (8 for bf16 X, 4 for
 // fp32 X) as groups of 16 slots of PER values: slot 3·jl + t of group jg is term t of

@@ -1140,9 +1140,9 @@ constexpr uint32_t kRedRows = 32;  // rows of B a block reduces (a packed K-step
 // them from LDS eight rows at a time. (A thread per eight-row group and challenge read its rows
 // one by one: 107 us for a 1536 x 151936 B of 38 chunks, k = 4, against 10, and 12 us for a
 // 4096 x 4096 one of four, k = 8, against 5.) Sums in fp64, in chunk order.
-__global__ __launch_bounds__(256) void reduce_b(const RedJob* __restrict__ jobs, uint32_t n_jobs,
-                                                uint32_t k) {
-  extern __shared__ float s_red[];  // [kRedRows][k], then |B|·1's kRedRows
+__device__ __forceinline__ void reduce_rows(const RedJob* __restrict__ jobs, uint32_t n_jobs,
+                                            uint32_t k, float* s_red) {
+  // s_red: [kRedRows][k], then |B|·1's kRedRows
   uint32_t lo = 0, hi = n_jobs - 1;
   while (lo < hi) {
     const uint32_t mid = (lo + hi + 1) >> 1;
@@ -1240,7 +1240,7 @@ __global__ __launch_bounds__(256) void reduce_b(const RedJob* __restrict__ jobs,
 
 // ---- finish: one product's row ------------------------------------------------------------
 //
-// Three kernels. bias_terms: per biased product, ‖b‖₁, ‖b‖² and bᵀR_j. finish_slices: per
+// Per biased product, beside B's reduction (reduce_bias), ‖b‖₁, ‖b‖² and bᵀR_j. finish_slices: per
 // slice of 256 to kSliceRows rows of a product (as many as leave the launch 512 blocks; fewer
 // where a product has many chunks), the fp64 sums over its rows of ν_i², |P|1_i²,
 // ‖P_i‖², (A²(B²1))_i and d_ij², written as one record. finish_final: per product, the slices'
@@ -1298,12 +1298,11 @@ __device__ __forceinline__ void block_sums(double (&v)[N], double* sh) {
 
 // One block per biased product (index list `which`): ‖b‖₁, ‖b‖² and bᵀR_j in one sweep over b
 // with the first eight challenges, each further eight in a sweep of their own.
-__global__ __launch_bounds__(256) void bias_terms(const FinJob* __restrict__ jobs,
-                                                  const uint32_t* __restrict__ which, uint32_t k,
-                                                  BiasOut* __restrict__ bout,
-                                                  float* __restrict__ br) {
-  __shared__ double sh[10 * 4];
-  const uint32_t pi = which[blockIdx.x];
+__device__ __forceinline__ void bias_terms(const FinJob* __restrict__ jobs,
+                                           const uint32_t* __restrict__ which, uint32_t at,
+                                           uint32_t k, BiasOut* __restrict__ bout,
+                                           float* __restrict__ br, double* sh) {
+  const uint32_t pi = which[at];
   const FinJob J = jobs[pi];
   const float* bias = reinterpret_cast<const float*>(J.bias);
   const float* R = reinterpret_cast<const float*>(J.r);
@@ -1333,6 +1332,19 @@ __global__ __launch_bounds__(256) void bias_terms(const FinJob* __restrict__ job
         if (jj < nj) br[(uint64_t)pi * k + j0 + jj] = (float)acc[jj];
     }
   }
+}
+
+// B's reduction, then the biased products' terms, which need R alone: one launch.
+__global__ __launch_bounds__(256) void reduce_bias(const RedJob* __restrict__ red,
+                                                   uint32_t n_red, uint32_t red_blocks,
+                                                   const FinJob* __restrict__ jobs,
+                                                   const uint32_t* __restrict__ which, uint32_t k,
+                                                   BiasOut* __restrict__ bout,
+                                                   float* __restrict__ br) {
+  extern __shared__ float s_red[];
+  __shared__ double sh[10 * 4];
+  if (blockIdx.x < red_blocks) reduce_rows(red, n_red, k, s_red);
+  else bias_terms(jobs, which, blockIdx.x - red_blocks, k, bout, br, sh);
 }
 
 // Adds a row's partial dot products X·V_j, j = j0 .. j0 + nj − 1, over its column chunks in
@@ -1402,19 +1414,30 @@ __device__ __forceinline__ void chunk_sums(const float* __restrict__ abs_,
   }
 }
 
+// The sum of record column `col` as its column of the row.
+__device__ __forceinline__ void put_column(double* row, uint32_t col, double sum,
+                                           uint32_t guard) {
+  if (col < 2) row[col] = guard ? sqrt(sum) : __builtin_nan("");
+  else if (col == 3) row[3] = sum;
+  else row[col == 2 ? 2 : 1 + col] = sqrt(sum);
+}
+
 // One block per slice. Record layout: [Σν², Σ|P|1², Σ‖P_i‖², Σ(A²(B²1))_i, Σd_1², ..., Σd_k²].
 // One sweep over the slice's rows takes the four sums and the residuals of challenges 1..8;
 // each further 8 challenges take a sweep of their own.
 __global__ __launch_bounds__(256) void finish_slices(const FinJob* __restrict__ jobs,
                                                      const SliceJob* __restrict__ slices,
                                                      uint32_t k, const BiasOut* __restrict__ bout,
-                                                     const float* __restrict__ br,
-                                                     double* __restrict__ recs) {
+                                                     const float* __restrict__ br, uint32_t guard,
+                                                     double* __restrict__ recs,
+                                                     double* __restrict__ rows) {
   __shared__ double sh[12 * 4];
   const SliceJob S = slices[blockIdx.x];
   const FinJob J = jobs[S.prod];
   const uint32_t tid = threadIdx.x;
   double* out = recs + (uint64_t)blockIdx.x * (4 + k);
+  // a product of one slice: its record is its row's sums
+  double* row = J.n_slices == 1 ? rows + (uint64_t)S.prod * (5 + k) : nullptr;
   const bool biased = J.bias != 0;
   const float babs = biased ? __uint_as_float((uint32_t)bout[S.prod].babs) : 0.f;
   const float* adot = reinterpret_cast<const float*>(J.a_dot);
@@ -1469,10 +1492,20 @@ __global__ __launch_bounds__(256) void finish_slices(const FinJob* __restrict__ 
     }
     if (nj <= 4) block_sums<8>(*reinterpret_cast<double(*)[8]>(acc), sh);
     else block_sums<12>(acc, sh);
-    if (tid == 0) {
+    if (tid == 0 && row) {
+      if (first) {
+        for (uint32_t t = 0; t < 4; t++) put_column(row, t, acc[t], guard);
+        row[4] = biased ? bout[S.prod].bsq : 0.0;
+      }
+#pragma unroll
+      for (uint32_t jj = 0; jj < 8; jj++)
+        if (jj < nj) put_column(row, 4 + j0 + jj, acc[4 + jj], guard);
+    } else if (tid == 0) {
       if (first)
         for (int t = 0; t < 4; t++) out[t] = acc[t];
-      for (uint32_t jj = 0; jj < nj; jj++) out[4 + j0 + jj] = acc[4 + jj];
+#pragma unroll
+      for (uint32_t jj = 0; jj < 8; jj++)
+        if (jj < nj) out[4 + j0 + jj] = acc[4 + jj];
     }
   }
 }
@@ -1487,6 +1520,7 @@ __global__ __launch_bounds__(64) void finish_final(const FinJob* __restrict__ jo
                                                    double* __restrict__ rows) {
   const uint32_t pi = blockIdx.x, lane = threadIdx.x;
   const FinJob J = jobs[pi];
+  if (J.n_slices == 1) return;  // finish_slices wrote its row
   double* out = rows + (uint64_t)pi * (5 + k);
   for (uint32_t c0 = 0; c0 < 4 + k; c0 += 8) {
     double acc[8];
@@ -1498,19 +1532,13 @@ __global__ __launch_bounds__(64) void finish_final(const FinJob* __restrict__ jo
       for (uint32_t t = 0; t < 8; t++)
         if (c0 + t < 4 + k) acc[t] += rec[t];
     }
-    if (J.n_slices > 1) {  // (a single slice's sums are in lane 0 already)
 #pragma unroll
-      for (int t = 0; t < 8; t++)
-        for (int o = 32; o > 0; o >>= 1) acc[t] += __shfl_xor(acc[t], o);
-    }
+    for (int t = 0; t < 8; t++)
+      for (int o = 32; o > 0; o >>= 1) acc[t] += __shfl_xor(acc[t], o);
     if (lane == 0) {
 #pragma unroll
-      for (uint32_t t = 0; t < 8; t++) {
-        const uint32_t col = c0 + t;
-        if (col < 2) out[col] = guard ? sqrt(acc[t]) : __builtin_nan("");
-        else if (col == 3) out[3] = acc[t];
-        else if (col < 4 + k) out[col == 2 ? 2 : 1 + col] = sqrt(acc[t]);
-      }
+      for (uint32_t t = 0; t < 8; t++)
+        if (c0 + t < 4 + k) put_column(out, c0 + t, acc[t], guard);
     }
   }
   if (lane == 0) out[4] = J.bias != 0 ? bout[pi].bsq : 0.0;
@@ -1660,8 +1688,7 @@ struct FvPlan {
   size_t total = 0;
   uint32_t* d_key = nullptr;
   uint32_t* d_queue = nullptr;  // a row pass's kQueues tile queue counters per stage (grid-limited)
-  ChallengeItem* d_items_b3 = nullptr;  // items whose R is read by bf16 passes
-  ChallengeItem* d_items_f4 = nullptr;
+  ChallengeItem* d_items = nullptr;
   uint32_t n_items = 0;
   uint64_t n_units = 0;
   float* d_r = nullptr;
@@ -1781,27 +1808,15 @@ extern "C" int pots_fv_plan_create(size_t n, const pots_fv_product* prods, uint3
     // R packed in the layouts the B and P passes read.
     P->need_b3 |= p.b_dtype == DT_BF16 || p.p_dtype == DT_BF16;
     P->need_f4 |= p.b_dtype == DT_F32 || p.p_dtype == DT_F32;
-    items[i].pk_off = 0;
+    items[i].b3_off = b3_elems;
+    items[i].f4_off = f4_floats;
     b3_elems += wpad * b3_per_row;
     f4_floats += wpad * f4_per_row;
   }
   P->n_items = (uint32_t)n;
   P->n_units = units;
   P->r_floats = r_floats;
-  // Packed offsets: the same item order in both layouts.
-  std::vector<ChallengeItem> items_b3 = items, items_f4 = items;
-  {
-    uint64_t ob = 0, of = 0;
-    for (size_t i = 0; i < n; i++) {
-      const uint64_t wpad = pad32(prods[i].w);
-      items_b3[i].pk_off = ob;
-      items_f4[i].pk_off = of;
-      ob += wpad * b3_per_row;
-      of += wpad * f4_per_row;
-    }
-  }
-  const size_t o_items_b3 = place(n * sizeof(ChallengeItem));
-  const size_t o_items_f4 = place(n * sizeof(ChallengeItem));
+  const size_t o_items = place(n * sizeof(ChallengeItem));
   const size_t o_r = place(r_floats * 4);
   const size_t o_rb3 = place(P->need_b3 ? b3_elems * 2 : 16);
   const size_t o_rf4 = place(P->need_f4 ? f4_floats * 4 : 16);
@@ -2117,8 +2132,7 @@ extern "C" int pots_fv_plan_create(size_t n, const pots_fv_product* prods, uint3
   const uint64_t base = reinterpret_cast<uint64_t>(P->base);
   P->d_key = reinterpret_cast<uint32_t*>(P->base + o_key);
   P->d_queue = reinterpret_cast<uint32_t*>(P->base + o_queue);
-  P->d_items_b3 = reinterpret_cast<ChallengeItem*>(P->base + o_items_b3);
-  P->d_items_f4 = reinterpret_cast<ChallengeItem*>(P->base + o_items_f4);
+  P->d_items = reinterpret_cast<ChallengeItem*>(P->base + o_items);
   P->d_r = reinterpret_cast<float*>(P->base + o_r);
   P->d_r_b3 = reinterpret_cast<uint16_t*>(P->base + o_rb3);
   P->d_r_f4 = reinterpret_cast<float*>(P->base + o_rf4);
@@ -2148,15 +2162,15 @@ extern "C" int pots_fv_plan_create(size_t n, const pots_fv_product* prods, uint3
     const size_t pi = src % n;
     const pots_fv_product& p = prods[pi];
     if (src < n) {  // B pass: V = R in B's layout
-      J.v = p.b_dtype == DT_BF16 ? base + o_rb3 + 2 * items_b3[pi].pk_off
-                                 : base + o_rf4 + 4 * items_f4[pi].pk_off;
+      J.v = p.b_dtype == DT_BF16 ? base + o_rb3 + 2 * items[pi].b3_off
+                                 : base + o_rf4 + 4 * items[pi].f4_off;
     } else if (src < 2 * n) {  // A pass: V = packed B·R, weights b1 and b2
       J.v = base + o_br + off_br[pi];
       J.u = base + o_br + off_b1[pi];
       J.w = base + o_br + off_b2[pi];
     } else {  // P pass: V = R in P's layout
-      J.v = p.p_dtype == DT_BF16 ? base + o_rb3 + 2 * items_b3[pi].pk_off
-                                 : base + o_rf4 + 4 * items_f4[pi].pk_off;
+      J.v = p.p_dtype == DT_BF16 ? base + o_rb3 + 2 * items[pi].b3_off
+                                 : base + o_rf4 + 4 * items[pi].f4_off;
     }
   }
   // The original job index -> ordered position, for the reduction and finish tables.
@@ -2244,8 +2258,7 @@ extern "C" int pots_fv_plan_create(size_t n, const pots_fv_product* prods, uint3
     return POTS_E_OK;
   };
   int rc = POTS_E_OK;
-  if ((rc = up(o_items_b3, items_b3.data(), n * sizeof(ChallengeItem))) ||
-      (rc = up(o_items_f4, items_f4.data(), n * sizeof(ChallengeItem))) ||
+  if ((rc = up(o_items, items.data(), n * sizeof(ChallengeItem))) ||
       (rc = up(o_jobs, ordered.data(), ordered.size() * sizeof(PassJob))) ||
       (rc = up(o_blk, blk_table.data(), blk_table.size() * 4)) ||
       (rc = up(o_red, red.data(), red.size() * sizeof(RedJob))) ||
@@ -2484,26 +2497,25 @@ static int run_stage(FvPlan* P, int stage, const uint8_t* d_key, double* d_rows,
   int rc;
   switch (stage) {
     case 0:
-      POTS_HIP(hipMemcpyAsync(P->d_key, d_key, 32, hipMemcpyDeviceToDevice, s));
-      // R in row-major form (for the bias term and the API) and in the packed layouts.
-      if ((rc = challenges_enqueue(P->d_key, P->d_items_b3, P->n_items, P->n_units, P->k,
-                                   P->d_r, P->need_b3 ? P->d_r_b3 : nullptr, nullptr, s)) !=
-          POTS_E_OK)
-        return rc;
-      if (P->need_f4 &&
-          (rc = challenges_enqueue(P->d_key, P->d_items_f4, P->n_items, P->n_units, P->k,
-                                   nullptr, nullptr, P->d_r_f4, s)) != POTS_E_OK)
-        return rc;
-      return POTS_E_OK;
+      // R in row-major form (for the bias term and the API) and in the packed layouts. (A key
+      // that is not word aligned is copied to one that is.)
+      if (reinterpret_cast<uintptr_t>(d_key) % 4 != 0) {
+        POTS_HIP(hipMemcpyAsync(P->d_key, d_key, 32, hipMemcpyDeviceToDevice, s));
+        d_key = reinterpret_cast<const uint8_t*>(P->d_key);
+      }
+      return challenges_enqueue(reinterpret_cast<const uint32_t*>(d_key), P->d_items, P->n_items,
+                                P->n_units, P->k, P->d_r, P->need_b3 ? P->d_r_b3 : nullptr,
+                                P->need_f4 ? P->d_r_f4 : nullptr, s);
     case 1:
       for (const PassLaunch& L : P->pass_b)
         if ((rc = run_pass(P, L, 1, s)) != POTS_E_OK) return rc;
       return POTS_E_OK;
     case 2:
-      if (P->n_red_blocks == 0) return POTS_E_OK;
-      hipLaunchKernelGGL(reduce_b, dim3(P->n_red_blocks), dim3(256),
-                         (kRedRows * P->k + kRedRows) * sizeof(float), s, P->d_red, P->n_red,
-                         P->k);
+      if (P->n_red_blocks + P->n_biased == 0) return POTS_E_OK;
+      hipLaunchKernelGGL(reduce_bias, dim3(P->n_red_blocks + P->n_biased), dim3(256),
+                         P->n_red_blocks ? (kRedRows * P->k + kRedRows) * sizeof(float) : 0, s,
+                         P->d_red, P->n_red, P->n_red_blocks, P->d_fin, P->d_biased, P->k,
+                         P->d_bout, P->d_br);
       POTS_HIP(hipGetLastError());
       return POTS_E_OK;
     case 3:  // the A pass: the row pass over the A's that are no twin's, then the twins'
@@ -2541,16 +2553,12 @@ static int run_stage(FvPlan* P, int stage, const uint8_t* d_key, double* d_rows,
       }
       return POTS_E_OK;
     case 5:
-      if (P->n_biased) {
-        hipLaunchKernelGGL(bias_terms, dim3(P->n_biased), dim3(256), 0, s, P->d_fin,
-                           P->d_biased, P->k, P->d_bout, P->d_br);
-        POTS_HIP(hipGetLastError());
-      }
       hipLaunchKernelGGL(finish_slices, dim3(P->n_slices), dim3(256), 0, s, P->d_fin,
-                         P->d_slices, P->k, P->d_bout, P->d_br, P->d_recs);
+                         P->d_slices, P->k, P->d_bout, P->d_br, P->guard, P->d_recs, d_rows);
       POTS_HIP(hipGetLastError());
-      hipLaunchKernelGGL(finish_final, dim3((uint32_t)P->n), dim3(64), 0, s, P->d_fin, P->k,
-                         P->guard, P->d_bout, P->d_recs, d_rows);
+      if (P->n_slices > P->n)  // else every product is one slice, its row written
+        hipLaunchKernelGGL(finish_final, dim3((uint32_t)P->n), dim3(64), 0, s, P->d_fin, P->k,
+                           P->guard, P->d_bout, P->d_recs, d_rows);
       POTS_HIP(hipGetLastError());
       return POTS_E_OK;
     default:

@@ -30,13 +30,12 @@ static_assert(sizeof(VerdictSpec) == 24, "VerdictSpec layout");
 
 __device__ __forceinline__ bool finite(double x) { return isfinite(x); }
 
-__global__ __launch_bounds__(256) void verdict_kernel(
-    const double* __restrict__ rows, uint32_t k, const VerdictSpec* __restrict__ specs, uint32_t n,
-    double eps_in, double eps_acc, double tau, double sigma_r, double sqrt2, uint32_t guard,
-    uint32_t judge, int32_t* __restrict__ codes, double* __restrict__ finished,
-    uint32_t* __restrict__ first_fail) {
-  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
+// Product i's verdict, written to codes (and finished); its code.
+__device__ __forceinline__ int32_t verdict(
+    uint32_t i, const double* __restrict__ rows, uint32_t k,
+    const VerdictSpec* __restrict__ specs, double eps_in, double eps_acc, double tau,
+    double sigma_r, double sqrt2, uint32_t guard, uint32_t judge, int32_t* __restrict__ codes,
+    double* __restrict__ finished) {
   const double* r = rows + (uint64_t)i * (5 + k);
   const VerdictSpec s = specs[i];
   const double nu = r[0], p_abs1 = r[1], p_norm = r[2];
@@ -86,7 +85,41 @@ __global__ __launch_bounds__(256) void verdict_kernel(
     f[1] = unit;
     f[2] = u;
   }
-  if (code != 0) atomicMin(first_fail, i);
+  return code;
+}
+
+// One block for all products: the smallest rejected index comes from its own reduction, and one
+// launch does it. A thread takes products t, t + 256, ..., a few microseconds each.
+constexpr uint32_t kOneBlock = 1024;  // products, at most
+
+__global__ __launch_bounds__(256) void verdict_one(
+    const double* __restrict__ rows, uint32_t k, const VerdictSpec* __restrict__ specs, uint32_t n,
+    double eps_in, double eps_acc, double tau, double sigma_r, double sqrt2, uint32_t guard,
+    uint32_t judge, int32_t* __restrict__ codes, double* __restrict__ finished,
+    uint32_t* __restrict__ first_fail) {
+  __shared__ uint32_t s_first[4];
+  uint32_t first = n;
+  for (uint32_t i = threadIdx.x; i < n; i += 256)
+    if (verdict(i, rows, k, specs, eps_in, eps_acc, tau, sigma_r, sqrt2, guard, judge, codes,
+                finished) != 0)
+      first = min(first, i);
+  for (int o = 32; o > 0; o >>= 1) first = min(first, (uint32_t)__shfl_xor((int)first, o));
+  if ((threadIdx.x & 63) == 0) s_first[threadIdx.x >> 6] = first;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    *first_fail = min(min(s_first[0], s_first[1]), min(s_first[2], s_first[3]));
+}
+
+// A thread per product; *first_fail holds n at launch.
+__global__ __launch_bounds__(256) void verdict_kernel(
+    const double* __restrict__ rows, uint32_t k, const VerdictSpec* __restrict__ specs, uint32_t n,
+    double eps_in, double eps_acc, double tau, double sigma_r, double sqrt2, uint32_t guard,
+    uint32_t judge, int32_t* __restrict__ codes, double* __restrict__ finished,
+    uint32_t* __restrict__ first_fail) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n && verdict(i, rows, k, specs, eps_in, eps_acc, tau, sigma_r, sqrt2, guard, judge,
+                       codes, finished) != 0)
+    atomicMin(first_fail, i);
 }
 
 __global__ void fill_u32v(uint32_t* p, uint32_t v) { *p = v; }
@@ -104,6 +137,13 @@ extern "C" int pots_verdicts_async(size_t n, const double* d_rows, uint32_t k,
   if (!d_rows || !d_specs || !d_codes || !d_first_fail || k < 1 || n >= 0xFFFFFFFFull)
     return POTS_E_ARG;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (n <= kOneBlock) {
+    hipLaunchKernelGGL(verdict_one, dim3(1), dim3(256), 0, s, d_rows, k,
+                       static_cast<const VerdictSpec*>(d_specs), (uint32_t)n, eps_in, eps_acc, tau,
+                       sigma_r, sqrt2, guard, judge, d_codes, d_finished, d_first_fail);
+    POTS_HIP(hipGetLastError());
+    return POTS_E_OK;
+  }
   hipLaunchKernelGGL(fill_u32v, dim3(1), dim3(1), 0, s, d_first_fail, (uint32_t)n);
   POTS_HIP(hipGetLastError());
   hipLaunchKernelGGL(verdict_kernel, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, d_rows,

@@ -132,6 +132,7 @@ class Native:
             "pots_step_run": ([_vp, _vp, _vp, _vp, _vp, _vp, _vp], _int),
             "pots_merkle_tree_async": ([_sz, _vp, _vp, _vp], _int),
             "pots_challenges": ([_vp, _u32, _sz, _vp, _vp, _vp, _vp, _u32], _int),
+            "pots_set_key_async": ([_vp, ctypes.c_char_p, _vp], _int),
             "pots_fv_plan_create": ([_sz, _vp, _u32, _u32, ctypes.POINTER(_vp)], _int),
             "pots_fv_plan_run": ([_vp, _vp, _vp, _vp], _int),
             "pots_fv_plan_run_stage": ([_vp, _int, _vp, _vp, _vp], _int),
@@ -262,6 +263,18 @@ class Native:
                                               _addr(offs), out.data_ptr(), 1),
                     "pots_challenges")
         return out
+
+    def set_key(self, key: torch.Tensor, h: bytes,
+                stream: torch.cuda.Stream | None = None) -> None:
+        """The root ``h`` (32 host bytes) into ``key`` (uint8 ``[32]`` on the GPU), in stream
+        order: the bytes travel as a launch's arguments, so nothing is copied or waited for."""
+        if len(h) != 32:
+            raise ValueError("h must be 32 bytes")
+        if key.dtype != torch.uint8 or key.numel() != 32 or not (key.is_cuda and
+                                                                  key.is_contiguous()):
+            raise ValueError("key must be a contiguous GPU uint8 tensor of 32 bytes")
+        self._check(self._lib.pots_set_key_async(key.data_ptr(), bytes(h), _stream(stream)),
+                    "pots_set_key_async")
 
     def fv_plan(self, products: Sequence[FvProduct], k: int, guard: bool = True) -> FvPlan:
         """A Freivalds plan over GPU-resident products (``pots_fv_plan_*``)."""
@@ -665,7 +678,7 @@ class FvPlan:
             if len(h) != 32:
                 raise ValueError("h must be 32 bytes")
             key = self._key
-            key.copy_(torch.frombuffer(bytearray(h), dtype=torch.uint8), non_blocking=False)
+            self._lib.set_key(key, h, stream)
         if out is None:
             out = torch.empty(self.n, 5 + self.k, dtype=torch.float64, device=self.device)
         self._lib._check(self._lib._lib.pots_fv_plan_run(self._h, key.data_ptr(), out.data_ptr(),

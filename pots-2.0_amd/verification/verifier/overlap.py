@@ -362,7 +362,7 @@ def decide(c: Any, store: TranscriptStore, ctx: StepContext, bands: Bands,
         buf = e.buffers
         key = buf["key"]
         _stage_records(e, records)
-        key.copy_(torch.frombuffer(bytearray(claimed), dtype=torch.uint8))
+        native.get().set_key(key, claimed)
         start = torch.cuda.Event()
         start.record(main)
         _enqueue_hashing(e, key, start)
@@ -449,7 +449,7 @@ def decide(c: Any, store: TranscriptStore, ctx: StepContext, bands: Bands,
         buf = e.buffers
         key = buf["key"]
         _stage_records(e, records)
-        key.copy_(torch.frombuffer(bytearray(claimed), dtype=torch.uint8))
+        native.get().set_key(key, claimed)
         if e.leaf.fused:  # the A stage's grid, timed on this step's own schedule
             _, e.grid_times = calibrate_a_grid(e.fv, lambda: _timed_run(e, key, update), dev)
         start = torch.cuda.Event()

@@ -217,7 +217,7 @@ class DeviceStepVerifier:
         if isinstance(claimed, torch.Tensor):
             self.key.copy_(claimed)
         else:
-            self.key.copy_(torch.frombuffer(bytearray(claimed), dtype=torch.uint8))
+            self.lib.set_key(self.key, claimed)
         timing = events is not None
         start = torch.cuda.Event(enable_timing=timing)
         start.record(main)

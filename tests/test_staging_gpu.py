@@ -1,6 +1,6 @@
 """Staged leaves (messages not word aligned where they lie): every header length and payload
 alignment, from device and host memory, beside leaves hashed in place. Bit for bit against the
-CPU oracle."""
+CPU oracle. And a root set from host memory."""
 
 from __future__ import annotations
 
@@ -35,3 +35,16 @@ def test_headers_and_alignments(lib, host):
     d, bad = lib.hash_leaves(b"".join(heads), hdr_off, hdr_len, np.arange(n, dtype=np.uint32), ptr,
                              ln, np.zeros(n, np.uint8))
     assert bad == n and [bytes(x) for x in d] == want
+
+
+def test_root_from_host_memory(lib):
+    key = torch.empty(3, 32, dtype=torch.uint8, device=DEV)
+    roots = [bytes((7 * i + j) & 255 for j in range(32)) for i in range(3)]
+    for i, r in enumerate(roots):
+        lib.set_key(key[i], r)
+    assert [bytes(x) for x in key.cpu().numpy()] == roots
+    for bad in (roots[0][:31], roots[0] + b"x"):
+        with pytest.raises(ValueError):
+            lib.set_key(key[0], bad)
+    with pytest.raises(ValueError):
+        lib.set_key(key, roots[0])
