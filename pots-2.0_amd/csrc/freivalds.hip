@@ -795,6 +795,24 @@ __global__ __launch_bounds__(256) void row_pass(const PassJob* __restrict__ jobs
   });
 }
 
+// The B pass's tiles, then the P pass's, of one dtype in one launch: both read R and neither the
+// other's results, so the P pass's tiles fill the CUs that the B pass's last ones leave, and a
+// small plan pays one launch and one chain of latencies for the two.
+template <uint32_t XT, uint32_t NJG>
+__global__ __launch_bounds__(256) void row_pass_bp(const PassJob* __restrict__ b_jobs,
+                                                   const uint32_t* __restrict__ b_blk,
+                                                   uint32_t n_b,
+                                                   const PassJob* __restrict__ p_jobs,
+                                                   const uint32_t* __restrict__ p_blk,
+                                                   uint32_t k) {
+  __shared__ __align__(16) u32x4 s_v[2 * VStage<NJG>::kUnits];
+  if (blockIdx.x < n_b)
+    row_tile<XT, false, false, NJG, true>(b_jobs, b_blk, k, blockIdx.x, nullptr, nullptr, s_v);
+  else
+    row_tile<XT, false, true, NJG, true>(p_jobs, p_blk, k, blockIdx.x - n_b, nullptr, nullptr,
+                                         s_v);
+}
+
 __global__ void queue_reset(uint32_t* q) {
   if (threadIdx.x < kQueues) q[threadIdx.x] = 0u;
 }
@@ -2489,6 +2507,39 @@ static int run_pass(const FvPlan* P, const PassLaunch& L, int stage, hipStream_t
   return POTS_E_OK;
 }
 
+template <uint32_t XT>
+static void launch_bp(const FvPlan* P, const PassLaunch& B, const PassLaunch& Q, hipStream_t s) {
+  const auto kernel = B.njg == 1   ? row_pass_bp<XT, 1>
+                      : B.njg == 2 ? row_pass_bp<XT, 2>
+                      : B.njg == 3 ? row_pass_bp<XT, 3>
+                                   : row_pass_bp<XT, 4>;
+  hipLaunchKernelGGL(kernel, dim3(B.n_blocks + Q.n_blocks), dim3(256), 0, s,
+                     P->d_jobs + B.job_off, P->d_blk + B.blk_off, B.n_blocks,
+                     P->d_jobs + Q.job_off, P->d_blk + Q.blk_off, P->k);
+}
+
+// The B and P passes, those of one dtype in one launch where neither has a grid limit.
+static int run_b_and_p(const FvPlan* P, hipStream_t s) {
+  int rc;
+  for (uint32_t xt = 0; xt < 2; xt++) {
+    const PassLaunch *B = nullptr, *Q = nullptr;
+    for (const PassLaunch& L : P->pass_b)
+      if (L.xt == xt) B = &L;
+    for (const PassLaunch& L : P->pass_ap)
+      if (!L.weighted && L.xt == xt) Q = &L;
+    if (B && Q && B->n_blocks && Q->n_blocks && !P->max_grid[1] && !P->max_grid[4] &&
+        (uint64_t)B->n_blocks + Q->n_blocks < 0x7FFFFFFFull) {
+      if (xt == DT_F32) launch_bp<DT_F32>(P, *B, *Q, s);
+      else launch_bp<DT_BF16>(P, *B, *Q, s);
+      POTS_HIP(hipGetLastError());
+      continue;
+    }
+    if (B && (rc = run_pass(P, *B, 1, s)) != POTS_E_OK) return rc;
+    if (Q && (rc = run_pass(P, *Q, 4, s)) != POTS_E_OK) return rc;
+  }
+  return POTS_E_OK;
+}
+
 // One stage of a plan's run: 0 challenges, 1 B pass, 2 reduce of B's vectors, 3 A pass,
 // 4 P pass, 5 rows. The stages run in this order on one stream; each reads what the earlier
 // ones wrote.
@@ -2570,11 +2621,12 @@ extern "C" int pots_fv_plan_run(void* plan, const uint8_t* d_key, double* d_rows
   if (!plan || !d_key || !d_rows) return POTS_E_ARG;
   FvPlan* P = static_cast<FvPlan*>(plan);
   if (P->fused) return POTS_E_ARG;  // stage 4 needs the leaf plan's chunk stage first
-  for (int stage = 0; stage < POTS_FV_STAGES; stage++) {
-    const int rc = run_stage(P, stage, d_key, d_rows, static_cast<hipStream_t>(stream));
-    if (rc != POTS_E_OK) return rc;
-  }
-  return POTS_E_OK;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  int rc;
+  if ((rc = run_stage(P, 0, d_key, d_rows, s)) || (rc = run_b_and_p(P, s)) ||
+      (rc = run_stage(P, 2, d_key, d_rows, s)) || (rc = run_stage(P, 3, d_key, d_rows, s)))
+    return rc;
+  return run_stage(P, 5, d_key, d_rows, s);
 }
 
 extern "C" int pots_fv_plan_run_stage(void* plan, int stage, const uint8_t* d_key,
