@@ -942,11 +942,16 @@ constexpr uint64_t kQuadMost = 32768;      // chunks hashed by four lanes each, 
 constexpr uint64_t kRunLeast = 512 << 10;  // chunks from which a lane takes kRun of them
 static uint32_t run_for(uint64_t chunks) { return chunks >= kRunLeast ? kRun : 1; }
 
+// Pinned memory of the synchronous entry point, per direction: a plan's metadata on the way up,
+// digests on the way down. Larger ones (some 5000 leaves, 32 thousand) take pageable copies.
+constexpr size_t kPinnedBytes = size_t(1) << 20;
+
 static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
                       const uint32_t* hdr_len, const uint32_t* hdr_idx,
                       const uint64_t* payload_ptr, const uint64_t* payload_len,
                       const uint8_t* kind, bool device_only, bool owned, void* fv,
-                      LeafPlan** out, char* ext_base = nullptr, size_t ext_cap = 0) {
+                      LeafPlan** out, char* ext_base = nullptr, size_t ext_cap = 0,
+                      void* pinned = nullptr) {
   if (n == 0 || n >= 0xFFFFFFFFull) return POTS_E_ARG;
   for (size_t i = 0; i < n; i++)
     if (kind[i] > POTS_KIND_F16) return POTS_E_ARG;
@@ -1212,7 +1217,8 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
     for (size_t f = 0; f < fdesc.size(); f++) fdesc[f].seg = segs[f];
   }
 
-  // Upload the metadata in one copy.
+  // Upload the metadata in one copy; from pinned memory of kPinnedBytes, if given, in the null
+  // stream's order, the caller waiting for that stream before it lets the memory go.
   std::vector<char> img(meta_bytes, 0);
   memcpy(img.data() + o_leaves, desc.data(), n * sizeof(LeafDesc));
   if (!fdesc.empty()) memcpy(img.data() + o_fuse, fdesc.data(), fdesc.size() * sizeof(FuseDesc));
@@ -1231,7 +1237,13 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
   if (!ents.empty()) memcpy(img.data() + o_lev, ents.data(), ents.size() * sizeof(LevelEntry));
   if (!blk_ent.empty())
     memcpy(img.data() + o_blk_ent, blk_ent.data(), blk_ent.size() * sizeof(uint32_t));
-  hipError_t e = hipMemcpy(P->base, img.data(), meta_bytes, hipMemcpyHostToDevice);
+  hipError_t e;
+  if (pinned && meta_bytes <= kPinnedBytes) {
+    memcpy(pinned, img.data(), meta_bytes);
+    e = hipMemcpyAsync(P->base, pinned, meta_bytes, hipMemcpyHostToDevice, 0);
+  } else {
+    e = hipMemcpy(P->base, img.data(), meta_bytes, hipMemcpyHostToDevice);
+  }
   if (e != hipSuccess) {
     note_hip_error(e, "hipMemcpy(leaf plan metadata)", __FILE__, __LINE__);
     if (owned) (void)hipFree(P->base);
@@ -1343,23 +1355,43 @@ extern "C" size_t pots_hash_leaves(size_t n, const uint8_t* hdr_buf, const uint6
                                    const uint8_t* kind, uint8_t* out, uint32_t n_threads) {
   (void)n_threads;
   if (n == 0) return 0;
+  // One call at a time: they share the arenas and the pinned memory. A small call's metadata and
+  // digests go through pinned memory, one copy each way in the null stream's order and one wait
+  // at the end (three pageable copies, each waited for, were 30 us of a norm's leaf hash).
+  static std::mutex mu;
+  std::lock_guard<std::mutex> lock(mu);
+  void* pinned = nullptr;
+  if (pinned_get(0, 2 * kPinnedBytes, &pinned) != POTS_E_OK) pinned = nullptr;
   LeafPlan* P = nullptr;
-  if (plan_build(n, hdr_buf, hdr_off, hdr_len, hdr_idx, payload_ptr, payload_len, kind,
-                 /*device_only=*/false, /*owned=*/false, nullptr, &P) != POTS_E_OK)
-    return SIZE_MAX;
   void* res = nullptr;
   size_t bad = SIZE_MAX;
-  if (arena_get(1, 32 * n + 16, &res) == POTS_E_OK) {
+  const size_t res_bytes = 32 * n + 4;
+  if (plan_build(n, hdr_buf, hdr_off, hdr_len, hdr_idx, payload_ptr, payload_len, kind,
+                 /*device_only=*/false, /*owned=*/false, nullptr, &P, nullptr, 0, pinned) ==
+          POTS_E_OK &&
+      arena_get(1, 32 * n + 16, &res) == POTS_E_OK) {
     uint32_t* d_dig = static_cast<uint32_t*>(res);
     uint32_t* d_bad = reinterpret_cast<uint32_t*>(static_cast<char*>(res) + 32 * n);
+    char* back = static_cast<char*>(pinned) + (pinned ? kPinnedBytes : 0);
     uint32_t h_bad = 0;
     if (plan_run(P, d_dig, d_bad, 0) == POTS_E_OK) {
-      hipError_t e = hipMemcpy(out, d_dig, 32 * n, hipMemcpyDeviceToHost);
-      if (e == hipSuccess) e = hipMemcpy(&h_bad, d_bad, 4, hipMemcpyDeviceToHost);
+      hipError_t e;
+      if (pinned && res_bytes <= kPinnedBytes) {
+        e = hipMemcpyAsync(back, res, res_bytes, hipMemcpyDeviceToHost, 0);
+        if (e == hipSuccess) e = hipStreamSynchronize(0);
+        if (e == hipSuccess) {
+          memcpy(out, back, 32 * n);
+          memcpy(&h_bad, back + 32 * n, 4);
+        }
+      } else {
+        e = hipMemcpy(out, d_dig, 32 * n, hipMemcpyDeviceToHost);
+        if (e == hipSuccess) e = hipMemcpy(&h_bad, d_bad, 4, hipMemcpyDeviceToHost);
+      }
       if (e == hipSuccess) bad = h_bad;
       else note_hip_error(e, "hipMemcpy(digests)", __FILE__, __LINE__);
     }
   }
+  if (bad == SIZE_MAX) (void)hipStreamSynchronize(0);  // a copy from the pinned memory may be left
   plan_free(P);
   return bad;
 }
