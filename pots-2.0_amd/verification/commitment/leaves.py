@@ -200,7 +200,17 @@ def _slot_table(c: DeclaredComputation) -> list[_Slot]:
     except TypeError:  # not weakly referenceable: build it every time
         table = None
     if table is None or len(table) != c.n_leaves - c.n_s:
-        table = [_Slot(*_tensor_slot(c, i)[:3]) for i in range(c.n_s, c.n_leaves)]
+        made: dict[tuple[int, tuple[int, ...]], _Slot] = {}  # slots alike are one object
+
+        def slot(tag: int, shape: tuple[int, ...], dtype: torch.dtype) -> _Slot:
+            got = made.get((tag, shape))
+            if got is None:
+                got = made[(tag, shape)] = _Slot(tag, shape, dtype)
+            return got
+
+        shapes, w_dtype, p_dtype = c.weight_shapes, c.weight_dtype, c.product_dtype
+        weights = [slot(TAG_WEIGHT, tuple(shapes[n]), w_dtype) for n in c.weight_names]
+        table = weights + [slot(TAG_PRODUCT, s.p_shape, p_dtype) for s in c.products] + weights
         try:
             _SLOT_TABLES[c] = table
         except TypeError:
@@ -387,47 +397,74 @@ class StepHasher:
             raise ValueError(f"transcript has {len(leaves)} leaves, the computation declares "
                              f"{c.n_leaves}")
         dev = device or next(t.device for t in leaves[c.n_s:] if isinstance(t, torch.Tensor))
-        headers, payloads, kinds = [], [], []
+        n_s = c.n_s
+        headers: list[bytes] = []
+        payloads: list[Any] = []
+        kinds: list[int] = []
         host_records: list[tuple[int, torch.Tensor]] = []
         record_headers: dict[tuple[int, torch.dtype, tuple[int, ...]], bytes] = {}
-        for i, obj in enumerate(leaves):
-            if i < c.n_s:
-                as_tensor = c.record_leaf(obj)
-                if as_tensor is not None:  # a tensor leaf: hashed where it lies
-                    tag, t = as_tensor
-                    key = (tag, t.dtype, tuple(t.shape))
-                    if key not in record_headers:
-                        record_headers[key] = tensor_leaf_header(tag, t)
-                    headers.append(record_headers[key])
-                    kinds.append(native.FINITE_KIND[t.dtype])
-                    payloads.append(t if t.is_cuda else None)
-                    if not t.is_cuda:
-                        host_records.append((i, t))
-                    continue
-                rec = np.frombuffer(c.encode_record(obj), dtype=np.uint8).copy()
-                headers.append(b"")
-                payloads.append(torch.from_numpy(rec).to(dev))
-                kinds.append(0)
+        for i in range(n_s):
+            as_tensor = c.record_leaf(leaves[i])
+            if as_tensor is not None:  # a tensor leaf: hashed where it lies
+                tag, t = as_tensor
+                key = (tag, t.dtype, tuple(t.shape))
+                if key not in record_headers:
+                    record_headers[key] = tensor_leaf_header(tag, t)
+                headers.append(record_headers[key])
+                kinds.append(native.FINITE_KIND[t.dtype])
+                payloads.append(t if t.is_cuda else None)
+                if not t.is_cuda:
+                    host_records.append((i, t))
                 continue
-            tag, t = _checked_tensor(c, i, obj)
-            if not t.is_cuda:
-                raise ValueError(f"leaf {i} is not on the GPU")
-            headers.append(tensor_leaf_header(tag, t))
-            payloads.append(t)
-            kinds.append(native.FINITE_KIND[t.dtype])
-        if host_records:  # one copy to the device for every host record tensor
+            rec = np.frombuffer(c.encode_record(leaves[i]), dtype=np.uint8).copy()
+            headers.append(b"")
+            payloads.append(None)
+            kinds.append(0)
+            host_records.append((i, torch.from_numpy(rec)))
+        if host_records:  # one copy to the device for every record in host memory
             flat = torch.cat([t.contiguous().view(-1).view(torch.uint8)
                               for _, t in host_records]).to(dev)
-            self._records = flat
             o = 0
             for i, t in host_records:
                 n = t.numel() * t.element_size()
-                payloads[i] = flat[o:o + n].view(t.dtype).view(t.shape)
+                payloads[i] = flat[o:o + n]
                 o += n
+        for i, t in enumerate(payloads):
+            if not (t.is_cuda and t.is_contiguous()):
+                raise ValueError(f"payload {i} must be a contiguous GPU tensor")
+        uniq: dict[bytes, int] = {}
+        idx = [uniq.setdefault(h, len(uniq)) for h in headers]
+        ptr = [t.data_ptr() for t in payloads]
+        nbytes = [t.nbytes for t in payloads]
+        # The tensor leaves, those exactly as their slot declares on the fast path (a step has
+        # thousands); anything else goes through the full validation, which raises its error.
+        for i, slot, t in zip(range(n_s, c.n_leaves), _slot_table(c), leaves[n_s:]):
+            h, kind = slot.header, slot.kind
+            if not (isinstance(t, torch.Tensor) and t.dtype is slot.dtype and
+                    t.shape == slot.shape and t.is_cuda and t.is_contiguous() and
+                    h is not None and kind is not None):
+                tag, t = _checked_tensor(c, i, t)
+                if not t.is_cuda:
+                    raise ValueError(f"leaf {i} is not on the GPU")
+                h, kind = tensor_leaf_header(tag, t), native.FINITE_KIND[t.dtype]
+                if not t.is_contiguous():
+                    raise ValueError(f"payload {i} must be a contiguous GPU tensor")
+            idx.append(uniq.setdefault(h, len(uniq)))
+            ptr.append(t.data_ptr())
+            nbytes.append(t.nbytes)
+            kinds.append(kind)
+            payloads.append(t)
+        hdr_len = np.array([len(h) for h in uniq], dtype=np.uint32)
+        hdr_off = np.zeros(len(uniq), dtype=np.uint64)
+        hdr_off[1:] = np.cumsum(hdr_len[:-1], dtype=np.uint64)
         self.c = c
         # With `fuse` (a native.FvPlan over this step's products), the product leaves' P-pass
         # sums are taken while they are hashed.
-        self.plan = native.get().leaf_plan(headers, payloads, kinds, fuse)
+        self.plan = native.LeafPlan.from_arrays(
+            native.get(), b"".join(uniq), hdr_off, hdr_len, np.array(idx, dtype=np.uint32),
+            np.array(ptr, dtype=np.uint64), np.array(nbytes, dtype=np.uint64),
+            np.array(kinds, dtype=np.uint8), payloads[0].device, fuse)
+        self.plan._keep = payloads
         self.n = len(leaves)
         self.bytes = self.plan.bytes
 
