@@ -936,10 +936,13 @@ static bool fuse_shape(uint64_t msg_bytes, uint32_t row_bytes, uint32_t lrun, ui
 //   1 GiB 382 / 385 / 551;  4 GiB 1444 / 1410 / 2069
 // A chunk is sixteen compressions, each needing the last one's output, so below a wave for
 // every SIMD (64 Ki lanes) the time is one lane's serial chain: short runs, and lanes in
-// quads while those still find idle SIMDs. Once every SIMD has eight waves the runs cost
-// nothing and save the second read of the lines between chunks.
-constexpr uint64_t kQuadMost = 32768;      // chunks hashed by four lanes each, at most
-constexpr uint64_t kRunLeast = 512 << 10;  // chunks from which a lane takes kRun of them
+// quads while those still find idle SIMDs. Runs of four save the second read of the lines
+// between chunks but quarter the blocks: the GPU holds 1024 of them, each 0.4 ms long, and the
+// last round of a few is part empty (a two-layer step's 6.4 M fused and 2.8 M plain chunks, 6.1
+// and 2.6 rounds: 2755 and 1015 us in runs of four, 2490 and 913 singly; 8.7 M chunks in one
+// plan 3010 and 2935). From kRunLeast on, sixteen rounds and more, the last one costs little.
+constexpr uint64_t kQuadMost = 32768;     // chunks hashed by four lanes each, at most
+constexpr uint64_t kRunLeast = 16 << 20;  // chunks from which a lane takes kRun of them
 static uint32_t run_for(uint64_t chunks) { return chunks >= kRunLeast ? kRun : 1; }
 
 // Pinned memory of the synchronous entry point, per direction: a plan's metadata on the way up,

@@ -1,5 +1,6 @@
 """The leaf hasher's ways of cutting work, each against the CPU oracle bit for bit: chunks on
-four lanes, one lane per chunk, and runs of chunks per lane, chosen by a plan's chunk count."""
+four lanes and one lane per chunk, chosen by a plan's chunk count (runs of chunks per lane take
+16 GiB of leaves: the full-size configurations' tests)."""
 
 from __future__ import annotations
 
@@ -38,7 +39,7 @@ def _leaves():
     return out + [odd[1:2], odd[1:], odd[3:2000]]  # 2-byte aligned: staged
 
 
-@pytest.mark.parametrize("filler_mib", [0, 33, 513])  # quads; a chunk per lane; runs of chunks
+@pytest.mark.parametrize("filler_mib", [0, 33, 513])  # quads; a chunk per lane, few and many
 def test_chunk_paths_match_oracle(lib, filler_mib):
     from verification.commitment import native
     ts = _leaves()
