@@ -857,6 +857,7 @@ struct LeafPlan {
   uint32_t* d_cv[2] = {nullptr, nullptr};
   uint32_t max_grid = 0;  // chunk kernel's grid limit; 0 = one block per slot
   std::vector<LevelInfo> levels;
+  char* d_result = nullptr;  // of a synchronous call: the first-bad word (n), then the digests
   StageJob* d_stages = nullptr;
   uint32_t n_stages = 0, stage_blocks = 0;
   std::vector<HostCopy> host_copies;  // after the staging kernel
@@ -948,6 +949,7 @@ static uint32_t run_for(uint64_t chunks) { return chunks >= kRunLeast ? kRun : 1
 // Pinned memory of the synchronous entry point, per direction: a plan's metadata on the way up,
 // digests on the way down. Larger ones (some 5000 leaves, 32 thousand) take pageable copies.
 constexpr size_t kPinnedBytes = size_t(1) << 20;
+constexpr size_t kResultHead = 16;  // bytes of a call's results before its digests
 
 static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
                       const uint32_t* hdr_len, const uint32_t* hdr_idx,
@@ -1148,7 +1150,13 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
   const size_t o_lev = place(std::max<size_t>(ents.size(), 1) * sizeof(LevelEntry));
   const size_t o_blk_ent = place(std::max<size_t>(blk_ent.size(), 1) * sizeof(uint32_t));
   const size_t o_stages = place(std::max<size_t>(stages.size(), 1) * sizeof(StageJob));
-  const size_t meta_bytes = at;
+  // A synchronous call's results: the first-bad word, uploaded with the metadata as n, and the
+  // digests behind it, so that one copy brings both back.
+  size_t o_bad = 0, meta_bytes = at;
+  if (pinned) {
+    o_bad = place(kResultHead + 32 * n);
+    meta_bytes = o_bad + kResultHead;
+  }
   const size_t o_cv0 = place(nc * 32);
   const size_t o_cv1 = place(std::max<uint64_t>(cv1_need, 1) * 32);
   const size_t o_stage = place(std::max<uint64_t>(stage_bytes, 16));
@@ -1240,6 +1248,11 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
   if (!ents.empty()) memcpy(img.data() + o_lev, ents.data(), ents.size() * sizeof(LevelEntry));
   if (!blk_ent.empty())
     memcpy(img.data() + o_blk_ent, blk_ent.data(), blk_ent.size() * sizeof(uint32_t));
+  if (pinned) {
+    const uint32_t none = (uint32_t)n;
+    memcpy(img.data() + o_bad, &none, 4);
+    P->d_result = P->base + o_bad;
+  }
   hipError_t e;
   if (pinned && meta_bytes <= kPinnedBytes) {
     memcpy(pinned, img.data(), meta_bytes);
@@ -1368,23 +1381,29 @@ extern "C" size_t pots_hash_leaves(size_t n, const uint8_t* hdr_buf, const uint6
   LeafPlan* P = nullptr;
   void* res = nullptr;
   size_t bad = SIZE_MAX;
-  const size_t res_bytes = 32 * n + 4;
+  const size_t res_bytes = kResultHead + 32 * n;
   if (plan_build(n, hdr_buf, hdr_off, hdr_len, hdr_idx, payload_ptr, payload_len, kind,
                  /*device_only=*/false, /*owned=*/false, nullptr, &P, nullptr, 0, pinned) ==
           POTS_E_OK &&
-      arena_get(1, 32 * n + 16, &res) == POTS_E_OK) {
-    uint32_t* d_dig = static_cast<uint32_t*>(res);
-    uint32_t* d_bad = reinterpret_cast<uint32_t*>(static_cast<char*>(res) + 32 * n);
-    char* back = static_cast<char*>(pinned) + (pinned ? kPinnedBytes : 0);
-    uint32_t h_bad = 0;
-    if (plan_run(P, d_dig, d_bad, 0) == POTS_E_OK) {
+      (P->d_result || arena_get(1, res_bytes, &res) == POTS_E_OK)) {
+    char* d_res = P->d_result ? P->d_result : static_cast<char*>(res);
+    uint32_t* d_bad = reinterpret_cast<uint32_t*>(d_res);
+    uint32_t* d_dig = reinterpret_cast<uint32_t*>(d_res + kResultHead);
+    // the staging stage only where there is something to stage or a first-bad word to reset
+    int rc = POTS_E_OK;
+    for (int stage = P->d_result && P->n_stages == 0 ? 1 : 0;
+         stage < POTS_LEAF_STAGES && rc == POTS_E_OK; stage++)
+      rc = plan_stage(P, stage, d_dig, d_bad, 0);
+    if (rc == POTS_E_OK) {
+      uint32_t h_bad = 0;
       hipError_t e;
       if (pinned && res_bytes <= kPinnedBytes) {
-        e = hipMemcpyAsync(back, res, res_bytes, hipMemcpyDeviceToHost, 0);
+        char* back = static_cast<char*>(pinned) + kPinnedBytes;
+        e = hipMemcpyAsync(back, d_res, res_bytes, hipMemcpyDeviceToHost, 0);
         if (e == hipSuccess) e = hipStreamSynchronize(0);
         if (e == hipSuccess) {
-          memcpy(out, back, 32 * n);
-          memcpy(&h_bad, back + 32 * n, 4);
+          memcpy(&h_bad, back, 4);
+          memcpy(out, back + kResultHead, 32 * n);
         }
       } else {
         e = hipMemcpy(out, d_dig, 32 * n, hipMemcpyDeviceToHost);
