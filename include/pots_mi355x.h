@@ -217,6 +217,9 @@ int pots_set_key_async(uint8_t *d_key, const uint8_t key[32], void *stream);
  * Σ_i (A²(B²1))_i, ‖b‖², residual_1..k. No allocation, no sync. */
 int pots_fv_plan_run(void *plan, const uint8_t *d_key, double *d_rows, void *stream);
 
+/* pots_fv_plan_run keyed on 32 bytes of host memory (read before the call returns). */
+int pots_fv_plan_run_root(void *plan, const uint8_t root[32], double *d_rows, void *stream);
+
 /* pots_fv_plan_run is these stages in order: 0 the challenge matrices, 1 the B pass
  * (b1 = B·R, b2 = (B²)·1), 2 the reduction of B's split-K partials, 3 the A pass (A·b1 and
  * (A²)·b2), 4 the P pass (P·R, Σ|P|, ΣP²), 5 the rows. Enqueued on `stream` one at a time,

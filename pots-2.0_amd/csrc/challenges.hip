@@ -28,7 +28,14 @@
 
 namespace pots {
 
-__global__ __launch_bounds__(256) void xof_kernel(const uint32_t* __restrict__ key,
+// A root given by the host, as the launch's arguments: no copy, nothing to wait for.
+struct Key {
+  uint32_t w[8];
+};
+
+// The challenges of every item under the key at `key` (device memory), or `by_value` where that
+// is null.
+__global__ __launch_bounds__(256) void xof_kernel(const uint32_t* __restrict__ key, Key by_value,
                                                   const ChallengeItem* __restrict__ items,
                                                   uint32_t n_items, uint64_t n_threads,
                                                   uint32_t k, float* __restrict__ out,
@@ -48,7 +55,7 @@ __global__ __launch_bounds__(256) void xof_kernel(const uint32_t* __restrict__ k
   const uint32_t t = (uint32_t)(unit - it.unit_first);
   uint32_t cv[8], m[16], w[16];
 #pragma unroll
-  for (int i = 0; i < 8; i++) cv[i] = key[i];
+  for (int i = 0; i < 8; i++) cv[i] = key ? key[i] : by_value.w[i];
   const uint32_t mm = it.m, jj = j + 1;
   // Label bytes 0x10, m >> 24, m >> 16, m >> 8, m, j, then zero padding.
   m[0] = 0x10u | ((mm >> 24) & 0xFFu) << 8 | ((mm >> 16) & 0xFFu) << 16 | ((mm >> 8) & 0xFFu) << 24;
@@ -97,23 +104,21 @@ __global__ __launch_bounds__(256) void xof_kernel(const uint32_t* __restrict__ k
   }
 }
 
-int challenges_enqueue(const uint32_t* d_key, const ChallengeItem* d_items, uint32_t n_items,
+int challenges_enqueue(const uint32_t* d_key, const uint8_t* h_key,
+                       const ChallengeItem* d_items, uint32_t n_items,
                        uint64_t n_units, uint32_t k, float* d_out, uint16_t* d_b3, float* d_f4,
                        hipStream_t s) {
   if (n_items == 0) return POTS_E_OK;
   const uint64_t threads = n_units * k;
   const uint64_t blocks = (threads + 255) / 256;
   if (blocks >= 0x7FFFFFFFull) return POTS_E_ARG;
-  hipLaunchKernelGGL(xof_kernel, dim3((uint32_t)blocks), dim3(256), 0, s, d_key, d_items,
+  Key key{};
+  if (h_key) memcpy(key.w, h_key, 32);
+  hipLaunchKernelGGL(xof_kernel, dim3((uint32_t)blocks), dim3(256), 0, s, d_key, key, d_items,
                      n_items, threads, k, d_out, d_b3, d_f4);
   POTS_HIP(hipGetLastError());
   return POTS_E_OK;
 }
-
-// A root given by the host, as the launch's arguments: no copy, nothing to wait for.
-struct Key {
-  uint32_t w[8];
-};
 
 __global__ void set_key(uint32_t* __restrict__ dst, Key key) {
   if (threadIdx.x < 8) dst[threadIdx.x] = key.w[threadIdx.x];
@@ -154,11 +159,9 @@ extern "C" int pots_challenges(const uint8_t key[32], uint32_t k, size_t n, cons
   int rc;
   if ((rc = arena_get(5, meta + (dev_out ? 0 : end * 4), &buf)) != POTS_E_OK) return rc;
   char* b = static_cast<char*>(buf);
-  POTS_HIP(hipMemcpy(b, key, 32, hipMemcpyHostToDevice));
   POTS_HIP(hipMemcpy(b + 32, items.data(), n * sizeof(ChallengeItem), hipMemcpyHostToDevice));
   float* d_out = dev_out ? out : reinterpret_cast<float*>(b + meta);
-  if ((rc = challenges_enqueue(reinterpret_cast<const uint32_t*>(b),
-                               reinterpret_cast<const ChallengeItem*>(b + 32), (uint32_t)n,
+  if ((rc = challenges_enqueue(nullptr, key, reinterpret_cast<const ChallengeItem*>(b + 32), (uint32_t)n,
                                units, k, d_out, nullptr, nullptr, 0)) != POTS_E_OK)
     return rc;
   if (!dev_out) {

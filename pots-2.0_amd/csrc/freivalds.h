@@ -28,7 +28,10 @@ static_assert(sizeof(ChallengeItem) == 40, "ChallengeItem layout");
 __host__ __device__ inline uint32_t groups_b3(uint32_t k) { return (k + 4) / 5; }
 __host__ __device__ inline uint32_t groups_f4(uint32_t k) { return (k + 15) / 16; }
 
-int challenges_enqueue(const uint32_t* d_key, const ChallengeItem* d_items, uint32_t n_items,
+// Under the key at d_key (device memory, 4-byte aligned) or, where that is null, the 32 bytes at
+// h_key (host memory, read before the call returns).
+int challenges_enqueue(const uint32_t* d_key, const uint8_t* h_key,
+                       const ChallengeItem* d_items, uint32_t n_items,
                        uint64_t n_units, uint32_t k, float* d_out, uint16_t* d_b3, float* d_f4,
                        hipStream_t s);
 

@@ -2554,7 +2554,8 @@ static int run_stage(FvPlan* P, int stage, const uint8_t* d_key, double* d_rows,
         POTS_HIP(hipMemcpyAsync(P->d_key, d_key, 32, hipMemcpyDeviceToDevice, s));
         d_key = reinterpret_cast<const uint8_t*>(P->d_key);
       }
-      return challenges_enqueue(reinterpret_cast<const uint32_t*>(d_key), P->d_items, P->n_items,
+      return challenges_enqueue(reinterpret_cast<const uint32_t*>(d_key), nullptr, P->d_items,
+                                P->n_items,
                                 P->n_units, P->k, P->d_r, P->need_b3 ? P->d_r_b3 : nullptr,
                                 P->need_f4 ? P->d_r_f4 : nullptr, s);
     case 1:
@@ -2617,16 +2618,34 @@ static int run_stage(FvPlan* P, int stage, const uint8_t* d_key, double* d_rows,
   }
 }
 
+// A whole run but for its challenges.
+static int run_after_challenges(FvPlan* P, const uint8_t* d_key, double* d_rows, hipStream_t s) {
+  int rc;
+  if ((rc = run_b_and_p(P, s)) || (rc = run_stage(P, 2, d_key, d_rows, s)) ||
+      (rc = run_stage(P, 3, d_key, d_rows, s)))
+    return rc;
+  return run_stage(P, 5, d_key, d_rows, s);
+}
+
 extern "C" int pots_fv_plan_run(void* plan, const uint8_t* d_key, double* d_rows, void* stream) {
   if (!plan || !d_key || !d_rows) return POTS_E_ARG;
   FvPlan* P = static_cast<FvPlan*>(plan);
   if (P->fused) return POTS_E_ARG;  // stage 4 needs the leaf plan's chunk stage first
   hipStream_t s = static_cast<hipStream_t>(stream);
-  int rc;
-  if ((rc = run_stage(P, 0, d_key, d_rows, s)) || (rc = run_b_and_p(P, s)) ||
-      (rc = run_stage(P, 2, d_key, d_rows, s)) || (rc = run_stage(P, 3, d_key, d_rows, s)))
-    return rc;
-  return run_stage(P, 5, d_key, d_rows, s);
+  const int rc = run_stage(P, 0, d_key, d_rows, s);
+  return rc != POTS_E_OK ? rc : run_after_challenges(P, d_key, d_rows, s);
+}
+
+extern "C" int pots_fv_plan_run_root(void* plan, const uint8_t root[32], double* d_rows,
+                                     void* stream) {
+  if (!plan || !root || !d_rows) return POTS_E_ARG;
+  FvPlan* P = static_cast<FvPlan*>(plan);
+  if (P->fused) return POTS_E_ARG;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const int rc = challenges_enqueue(nullptr, root, P->d_items, P->n_items, P->n_units, P->k,
+                                    P->d_r, P->need_b3 ? P->d_r_b3 : nullptr,
+                                    P->need_f4 ? P->d_r_f4 : nullptr, s);
+  return rc != POTS_E_OK ? rc : run_after_challenges(P, nullptr, d_rows, s);
 }
 
 extern "C" int pots_fv_plan_run_stage(void* plan, int stage, const uint8_t* d_key,

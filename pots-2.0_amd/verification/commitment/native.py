@@ -135,6 +135,7 @@ class Native:
             "pots_set_key_async": ([_vp, ctypes.c_char_p, _vp], _int),
             "pots_fv_plan_create": ([_sz, _vp, _u32, _u32, ctypes.POINTER(_vp)], _int),
             "pots_fv_plan_run": ([_vp, _vp, _vp, _vp], _int),
+            "pots_fv_plan_run_root": ([_vp, ctypes.c_char_p, _vp, _vp], _int),
             "pots_fv_plan_run_stage": ([_vp, _int, _vp, _vp, _vp], _int),
             "pots_fv_plan_copy_challenges": ([_vp, _vp, _vp], _int),
             "pots_fv_plan_set_grid": ([_vp, _int, _u32], _int),
@@ -666,23 +667,21 @@ class FvPlan:
         self.bytes = int(lib._lib.pots_fv_plan_bytes(h))
         # pairs of products whose shared operand (A and Aᵀ) the twin pass reads once
         self.twins = int(lib._lib.pots_fv_plan_twins(h))
-        self._key = torch.empty(32, dtype=torch.uint8, device=self.device)
 
     def rows(self, h: bytes | torch.Tensor, out: torch.Tensor | None = None,
              stream: torch.cuda.Stream | None = None) -> torch.Tensor:
         """fp64 ``[n, 5 + k]`` rows (``freivalds.ROW``), challenges keyed on ``h`` (32 bytes,
         host bytes or a GPU uint8 tensor). Stream-ordered, no sync."""
+        if out is None:
+            out = torch.empty(self.n, 5 + self.k, dtype=torch.float64, device=self.device)
+        lib = self._lib._lib
         if isinstance(h, torch.Tensor):
-            key = h
+            rc = lib.pots_fv_plan_run(self._h, h.data_ptr(), out.data_ptr(), _stream(stream))
         else:
             if len(h) != 32:
                 raise ValueError("h must be 32 bytes")
-            key = self._key
-            self._lib.set_key(key, h, stream)
-        if out is None:
-            out = torch.empty(self.n, 5 + self.k, dtype=torch.float64, device=self.device)
-        self._lib._check(self._lib._lib.pots_fv_plan_run(self._h, key.data_ptr(), out.data_ptr(),
-                                                         _stream(stream)), "pots_fv_plan_run")
+            rc = lib.pots_fv_plan_run_root(self._h, bytes(h), out.data_ptr(), _stream(stream))
+        self._lib._check(rc, "pots_fv_plan_run")
         return out
 
     STAGES = ("challenges", "b_pass", "reduce", "a_pass", "p_pass", "rows")

@@ -48,3 +48,19 @@ def test_root_from_host_memory(lib):
             lib.set_key(key[0], bad)
     with pytest.raises(ValueError):
         lib.set_key(key, roots[0])
+
+
+def test_rows_under_a_host_root_or_a_device_one(lib):
+    from verification.commitment.native import FvProduct
+    a, b = torch.randn(40, 33, device=DEV), torch.randn(33, 50, device=DEV)
+    x, y = a.bfloat16(), b.bfloat16()
+    plan = lib.fv_plan([FvProduct(a, b, a @ b, 1), FvProduct(x, y, x @ y, 2)], 3)
+    root = bytes(range(100, 132))
+    store = torch.zeros(40, dtype=torch.uint8, device=DEV)
+    want = plan.rows(root)
+    for skip in (0, 1, 4):  # a device root at any alignment
+        store[skip:skip + 32] = torch.tensor(list(root), dtype=torch.uint8)
+        assert torch.equal(plan.rows(store[skip:skip + 32]), want)
+    with pytest.raises(ValueError):
+        plan.rows(root[:31])
+    plan.close()
