@@ -448,7 +448,7 @@ __device__ __forceinline__ void stage_weight(uint64_t w, uint32_t c0, uint32_t c
 // One tile: job blk_job[bidx], 64-row group, column chunk and column-group block decoded
 // from its index within the job (row group fastest). Every wave of the block calls it with the
 // same tile and reaches its barrier.
-// A B-pass job of one column chunk writes what the reduction (reduce_b) would make of its one
+// A B-pass job of one column chunk writes what the reduction (reduce_rows) would make of its one
 // chunk of partials, the same values bit for bit: for each 8-row group and challenge j, B·R's
 // three exact bf16 terms in slots 3(j mod 5) .. of the group's column group j / 5 (rows past
 // the matrix zero; groups wholly past it are never written, and the plan zeroed them when it

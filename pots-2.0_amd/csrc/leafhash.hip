@@ -503,14 +503,20 @@ __global__ __launch_bounds__(kThreads) void chunk_kernel(
   }
 }
 
+// Orders LDS accesses within a wave: what its lanes wrote before is what its lanes read after.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // The chunks of the unfused leaves on four lanes each (b3_quad_compress), for plans of few
 // chunks, where a chunk's sixteen serial compressions are the call's latency and most of the
 // GPU would idle. A wave hashes kQuadChunks chunks. The quad's lanes load the chunk's sixteen
 // blocks 16 bytes a lane, all in flight at once, into the wave's LDS: groups wholly inside the
 // payload (past the header) as they lie, at word alignment, the loads of the others clamped
 // into the payload and their words then rewritten one by one (header words, zeros past the
-// end). No other wave touches that LDS, so the wave's own program order is the only ordering
-// it needs.
+// end). No other wave touches that LDS, so a wave's own order, which it keeps by itself, is
+// enough: wave_sync() only holds the compiler to it.
 __global__ __launch_bounds__(64) void chunk_kernel_quad(
     const LeafDesc* __restrict__ leaves, Order od, const uint32_t* __restrict__ head,
     uint32_t* __restrict__ cv_out, uint32_t* __restrict__ digests,
@@ -568,6 +574,7 @@ __global__ __launch_bounds__(64) void chunk_kernel_quad(
         }
       }
     }
+    wave_sync();
     const bool root = d.n_chunks == 1;
     uint32_t lo, hi;
     b3_quad_iv(q, lo, hi);
@@ -583,6 +590,7 @@ __global__ __launch_bounds__(64) void chunk_kernel_quad(
     gstore<uint32_t>(out + q, lo);
     gstore<uint32_t>(out + 4 + q, hi);
     if (fin.bad()) atomicMin(first_bad, i);
+    wave_sync();  // the next chunk's words go where these were read
   }
 }
 
