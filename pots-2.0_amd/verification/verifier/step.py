@@ -12,12 +12,12 @@ What runs where. Check 2's hashing (leaf digests, then the Merkle tree) and chec
 measuring (challenges, the three Freivalds passes, rows) depend only on the leaves and the
 claimed root, so they run on two streams at once: hashing is integer-VALU bound and uses a
 fraction of HBM bandwidth, the Freivalds passes are memory bound and leave the VALUs mostly
-idle. Each product's P is a leaf, so by default the leaf plan is fused with the Freivalds plan
-(``pots_leaf_plan_create_fused``): the chunk kernel takes the P-pass sums of the product leaves
-it streams and P is read once. The challenges then go first, the chunk kernel waits for them,
-and the P stage (which adds up the chunk kernel's run records) waits for the chunk kernel. The
-verdicts follow on the main stream. One host read at the end returns the root, the first
-non-finite leaf and the first rejected product.
+idle. Each product's P is a leaf, so by default the leaf plan of all but small steps is fused
+with the Freivalds plan (``pots_leaf_plan_create_fused``): the chunk kernel takes the P-pass sums
+of the product leaves it streams and P is read once. The challenges then go first, the chunk
+kernel waits for them, and the P stage (which adds up the chunk kernel's run records) waits for
+the chunk kernel. The verdicts follow on the main stream. One host read at the end returns the
+root, the first non-finite leaf and the first rejected product.
 """
 
 from __future__ import annotations
@@ -142,6 +142,28 @@ def enqueue_measure_and_hash(plan: native.FvPlan, hp: native.LeafPlan, fused: in
     return c_begin, c_end, a_begin, a_end
 
 
+# Chunks (1 KiB) from which a step's leaf plan is fused with its Freivalds plan. Below, an unfused
+# plan hashes every chunk on four lanes (leafhash.hip, kQuadMost), starts with the step and waits
+# for nothing, where a fused chunk kernel waits for the challenges and the B pass and then takes a
+# lane's sixteen serial compressions with their P sums, 57 us whatever the size; reading P a second
+# time costs a step of 32 MiB under 7 us. Fused / unfused, a step with its host read, us: 9.6 Ki
+# chunks 270 / 209, 15 Ki 283 / 208, 21 Ki 277 / 213, 28 Ki 268 / 210. The unfused order stays
+# ahead up to some 300 Ki (102 Ki 335 / 268, 135 Ki 378 / 260, 290 Ki 608 / 454) and level beyond
+# (506 Ki 608 / 606, 1.4 Mi 1273 / 1251, 1.7 Mi 1350 / 1366); the line lies where the hashing
+# leaves the four-lane kernel, and steps above it keep the fused plan that `fused` promises.
+FUSE_LEAST = 32768
+
+
+def _fuses(c: DeclaredComputation, leaves: Sequence[Any]) -> bool:
+    """Whether the step's tensor leaves hold FUSE_LEAST chunks."""
+    chunks = 0
+    for t in leaves[c.n_s:]:
+        chunks += getattr(t, "nbytes", 0) // 1024 + 1
+        if chunks >= FUSE_LEAST:
+            return True
+    return False
+
+
 class DeviceStepVerifier:
     """Plans for one step's transcript, built once: the leaf-hashing plan, the Freivalds plan
     over every product (operands served by ``operands(spec)``), and the verdict table. Call
@@ -169,6 +191,7 @@ class DeviceStepVerifier:
         self.hash_after_b, self.plain_early = hash_after_b, plain_early
         # Fused: the chunk kernel takes the P-pass sums of the product leaves it hashes, so
         # each P is read from HBM once (pots_leaf_plan_create_fused).
+        fuse = fuse and _fuses(c, leaves)
         self.hasher = StepHasher(c, leaves, fuse=self.plan if fuse else None)
         self.fused = self.hasher.plan.fused
         self.plan.set_grid(1, b_grid)
