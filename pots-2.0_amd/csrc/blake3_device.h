@@ -135,7 +135,15 @@ __device__ __forceinline__ void b3_parent_cv(const uint32_t l[8], const uint32_t
 // in total, so wide work keeps a lane each.
 //
 // The quad's 16 message words lie in LDS; each lane reads the four of a round it needs through
-// its offsets into the block (b3_quad_schedule, made once per kernel).
+// its offsets into the block (b3_quad_schedule, made once per kernel). Where the quad's own lanes
+// write them, wave_sync() stands between those writes and the compression, and again before the
+// words are written over.
+
+// Orders LDS accesses within a wave: what its lanes wrote before is what its lanes read after.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
 
 struct B3Quad {
   uint32_t off[28];  // word of the block for round r: off[4r], off[4r+1] columns, +2, +3 diagonals

@@ -503,12 +503,6 @@ __global__ __launch_bounds__(kThreads) void chunk_kernel(
   }
 }
 
-// Orders LDS accesses within a wave: what its lanes wrote before is what its lanes read after.
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 // The chunks of the unfused leaves on four lanes each (b3_quad_compress), for plans of few
 // chunks, where a chunk's sixteen serial compressions are the call's latency and most of the
 // GPU would idle. A wave hashes kQuadChunks chunks. The quad's lanes load the chunk's sixteen

@@ -96,6 +96,7 @@ __global__ __launch_bounds__(256) void tree_kernel(const uint8_t* __restrict__ l
         msg[i] = (i == 0 ? 0x01u : s[max(i, 1u) - 1] >> 24) | s[i] << 8;
         msg[16 + i] = i == 0 ? s[15] >> 24 : 0u;
       }
+      wave_sync();  // a lane reads words that its quad's other lanes wrote
       uint32_t lo, hi;
       b3_quad_iv(q, lo, hi);
       b3_quad_compress(sched, msg, q, q == 2 ? 64u : q == 3 ? B3_CHUNK_START : 0u, lo, hi);
@@ -104,6 +105,7 @@ __global__ __launch_bounds__(256) void tree_kernel(const uint8_t* __restrict__ l
                        : q == 3 ? (uint32_t)(B3_CHUNK_END | B3_ROOT)
                                 : 0u,
                        lo, hi);
+      wave_sync();  // the quad's next message goes where this one was read
       dst[q] = lo;
       dst[4 + q] = hi;
       uint32_t* node = reinterpret_cast<uint32_t*>(
