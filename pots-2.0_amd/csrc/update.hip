@@ -94,8 +94,9 @@ struct UpdAcc {
     const float ri = fabsf(w1 - (w - eg));
     const float si = eps_w * (fabsf(w) + fabsf(eg));
     const double rd = (double)ri, sd = (double)si;
-    // false for a NaN or infinite r, a NaN s and a NaN or negative tau_lo; an infinite s passes
-    // with any finite r, so it is tested on its own
+    // false for a NaN r, a NaN s and a NaN or negative tau_lo; false for an infinite r too, since
+    // tau_lo is bounded so that no finite s takes tau_lo·s to infinity; an infinite s passes with
+    // any r but a NaN, so it is tested on its own
     if (rd <= tau_lo * sd && si < INFINITY) {
       if (rd * (double)s > (double)r * sd) {
         r = ri;
@@ -137,9 +138,11 @@ __global__ __launch_bounds__(kUpdThreads) void update_kernel(const UpdJob* __res
   const float* wt = reinterpret_cast<const float*>(J.w_t);
   const float* wn = reinterpret_cast<const float*>(J.w_next);
   // (relative error of tau_lo·s under 2^-51: r <= tau_lo·s means r/s < tau_w exactly, and a
-  // product too small to be normal is below every nonzero r)
+  // product too small to be normal is below every nonzero r. A band past 2^800 tests as 2^800: no
+  // ratio of finite fp32 values but r/0 comes near it, and 2^800 times an fp32 s is finite, so an
+  // infinite r is never within it, whatever the band.)
   const double tau_w = J.tau_w;
-  const double tau_lo = tau_w >= 0 ? tau_w * (1.0 - 0x1p-50) : __builtin_nan("");
+  const double tau_lo = tau_w >= 0 ? fmin(tau_w, 0x1p800) * (1.0 - 0x1p-50) : __builtin_nan("");
   UpdAcc acc;
 #pragma unroll 1
   for (uint32_t st = 0; st < STEPS; st++) {

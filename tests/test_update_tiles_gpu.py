@@ -63,17 +63,25 @@ def test_sizes_and_bands(lib, dtypes, skip):
         _check(lib, [*cases, (w, wn, parts, 4.0)], skip)
 
 
-def test_special_values(lib):
-    inf, nan, big, tiny = math.inf, math.nan, 3.4e38, 1e-45
+INF, NAN, BIG, TINY = math.inf, math.nan, 3.4e38, 1e-45
+# (entry, its W_t, W_{t+1} and gradient)
+SPECIAL = [(5, 0.0, 0.0, 0.0), (5, 0.0, 1.0, 0.0), (5, 0.0, TINY, 0.0), (5, 1.0, INF, 0.0),
+           (5, INF, 1.0, 0.0), (5, INF, INF, 0.0), (5, NAN, 1.0, 0.0), (5, 1.0, NAN, 0.0),
+           (5, 1.0, 1.0, NAN), (5, 1.0, 1.0, INF), (5, BIG, -BIG, 0.0), (5, TINY, -TINY, 0.0),
+           (4100, 0.0, 1.0, 0.0), (4100, NAN, NAN, NAN), (20000, 1.0, 2.0, 1.0)]
+
+
+def _special(taus):
     cases = []
-    for seed, (at, w_v, wn_v, g_v) in enumerate([
-            (5, 0.0, 0.0, 0.0), (5, 0.0, 1.0, 0.0), (5, 0.0, tiny, 0.0), (5, 1.0, inf, 0.0),
-            (5, inf, 1.0, 0.0), (5, inf, inf, 0.0), (5, nan, 1.0, 0.0), (5, 1.0, nan, 0.0),
-            (5, 1.0, 1.0, nan), (5, 1.0, 1.0, inf), (5, big, -big, 0.0), (5, tiny, -tiny, 0.0),
-            (4100, 0.0, 1.0, 0.0), (4100, nan, nan, nan), (20000, 1.0, 2.0, 1.0)]):
+    for seed, (at, w_v, wn_v, g_v) in enumerate(SPECIAL):
         w, wn, parts = _case(20001, 50 + seed, [torch.float32])
         w[at], wn[at], parts[0][at] = w_v, wn_v, g_v
-        cases += [(w, wn, parts, tau) for tau in (4.0, 1e30, 0.0)]
+        cases += [(w, wn, parts, tau) for tau in taus]
+    return cases
+
+
+def test_special_values(lib):
+    cases = _special((4.0, 1e30, 0.0))
     zero = torch.zeros(300)
     cases += [(zero, zero, [zero], tau) for tau in (4.0, 0.0, -1.0, math.nan)]
     w, wn, parts = _case(300, 99, [torch.float32])
@@ -82,3 +90,16 @@ def test_special_values(lib):
     for n in (1 << 20, 8 << 20):  # with these, the plan's wider blocks
         w, wn, parts = _case(n, 78, [torch.float32])
         _check(lib, [*cases, (w, wn, parts, 4.0)])
+
+
+@pytest.mark.parametrize("tau", [math.inf, 1e308, 1e300, 1e270, -math.inf])
+def test_special_values_under_bands_past_fp64s_products(lib, tau):
+    """tau·scale overflows fp64 (or, at 1e270, nearly): an infinite residual lies within it."""
+    cases = _special((tau,))
+    # the large scales that overflow under a finite band
+    for w_v, wn_v in ((BIG, -BIG), (BIG, INF), (-BIG, 0.5 * BIG), (1e31, -INF)):
+        w, wn, parts = _case(20001, 70, [torch.float32])
+        w[7], wn[7] = w_v, wn_v
+        cases.append((w, wn, parts, tau))
+    _check(lib, cases)
+    _check(lib, cases, skip=1)
