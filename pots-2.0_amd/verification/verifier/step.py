@@ -12,12 +12,13 @@ What runs where. Check 2's hashing (leaf digests, then the Merkle tree) and chec
 measuring (challenges, the three Freivalds passes, rows) depend only on the leaves and the
 claimed root, so they run on two streams at once: hashing is integer-VALU bound and uses a
 fraction of HBM bandwidth, the Freivalds passes are memory bound and leave the VALUs mostly
-idle. Each product's P is a leaf, so by default the leaf plan of all but small steps is fused
-with the Freivalds plan (``pots_leaf_plan_create_fused``): the chunk kernel takes the P-pass sums
-of the product leaves it streams and P is read once. The challenges then go first, the chunk
-kernel waits for them, and the P stage (which adds up the chunk kernel's run records) waits for
-the chunk kernel. The verdicts follow on the main stream. One host read at the end returns the
-root, the first non-finite leaf and the first rejected product.
+idle. Each product's P is a leaf, so by default (``fuse=None``) the leaf plan of all but small
+steps (``FUSE_LEAST``) is fused with the Freivalds plan (``pots_leaf_plan_create_fused``): the
+chunk kernel takes the P-pass sums of the product leaves it streams and P is read once. The
+challenges then go first, the chunk kernel waits for them, and the P stage (which adds up the
+chunk kernel's run records) waits for the chunk kernel. The verdicts follow on the main stream.
+One host read at the end returns the root, the first non-finite leaf and the first rejected
+product.
 """
 
 from __future__ import annotations
@@ -142,15 +143,19 @@ def enqueue_measure_and_hash(plan: native.FvPlan, hp: native.LeafPlan, fused: in
     return c_begin, c_end, a_begin, a_end
 
 
-# Chunks (1 KiB) from which a step's leaf plan is fused with its Freivalds plan. Below, an unfused
-# plan hashes every chunk on four lanes (leafhash.hip, kQuadMost), starts with the step and waits
-# for nothing, where a fused chunk kernel waits for the challenges and the B pass and then takes a
-# lane's sixteen serial compressions with their P sums, 57 us whatever the size; reading P a second
-# time costs a step of 32 MiB under 7 us. Fused / unfused, a step with its host read, us: 9.6 Ki
-# chunks 270 / 209, 15 Ki 283 / 208, 21 Ki 277 / 213, 28 Ki 268 / 210. The unfused order stays
-# ahead up to some 300 Ki (102 Ki 335 / 268, 135 Ki 378 / 260, 290 Ki 608 / 454) and level beyond
-# (506 Ki 608 / 606, 1.4 Mi 1273 / 1251, 1.7 Mi 1350 / 1366); the line lies where the hashing
-# leaves the four-lane kernel, and steps above it keep the fused plan that `fused` promises.
+# Chunks (1 KiB) from which a step's leaf plan is by default fused with its Freivalds plan. Below,
+# an unfused plan hashes every chunk on four lanes (leafhash.hip, kQuadMost), starts with the step
+# and waits for nothing, where a fused chunk kernel waits for the challenges and the B pass and then
+# takes a lane's sixteen serial compressions with their P sums, 57 us whatever the size; reading P a
+# second time costs a step of 32 MiB under 7 us. Fused / unfused, a bf16 step at k = 4 with its host
+# read, us, by chunks:
+#   9.5 Ki 281 / 215;  31 Ki 282 / 215;  41 Ki 285 / 256;  78 Ki 420 / 296;  128 Ki 401 / 354;
+#   215 Ki 550 / 413;  428 Ki 556 / 517;  834 Ki 748 / 736;  980 Ki 1101 / 985;
+#   1.7 Mi 1536 / 1423;  2.0 Mi 1392 / 1360;  3.1 Mi 2233 / 2115;  5.3 Mi 3844 / 4182
+# So the orders cross between 3 and 5 Mi chunks, not at this line, which is where the hashing leaves
+# the four-lane kernel: above it the default stays the fused plan, one read of every P, and a caller
+# who wants the other order on either side passes `fuse`. (The overlapped path of
+# Verifier.verify_step fuses steps of every size.)
 FUSE_LEAST = 32768
 
 
@@ -167,10 +172,11 @@ def _fuses(c: DeclaredComputation, leaves: Sequence[Any]) -> bool:
 class DeviceStepVerifier:
     """Plans for one step's transcript, built once: the leaf-hashing plan, the Freivalds plan
     over every product (operands served by ``operands(spec)``), and the verdict table. Call
-    :meth:`run` with the claimed root."""
+    :meth:`run` with the claimed root. ``fuse``: whether the leaf plan is fused with the
+    Freivalds plan; by default, for steps of FUSE_LEAST chunks and more."""
 
     def __init__(self, c: DeclaredComputation, leaves: Sequence[Any], operands: Any, *, k: int,
-                 bands: Bands | None = None, guard: bool = True, fuse: bool = True,
+                 bands: Bands | None = None, guard: bool = True, fuse: bool | None = None,
                  a_grid: int | None = None, b_grid: int = 0, hash_after_b: bool = True,
                  plain_early: bool = False) -> None:
         self.c, self.k, self.guard = c, k, guard
@@ -191,7 +197,8 @@ class DeviceStepVerifier:
         self.hash_after_b, self.plain_early = hash_after_b, plain_early
         # Fused: the chunk kernel takes the P-pass sums of the product leaves it hashes, so
         # each P is read from HBM once (pots_leaf_plan_create_fused).
-        fuse = fuse and _fuses(c, leaves)
+        if fuse is None:
+            fuse = _fuses(c, leaves)
         self.hasher = StepHasher(c, leaves, fuse=self.plan if fuse else None)
         self.fused = self.hasher.plan.fused
         self.plan.set_grid(1, b_grid)
