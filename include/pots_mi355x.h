@@ -148,6 +148,15 @@ int pots_leaf_plan_create_fused(size_t n, const uint8_t *hdr_buf, const uint64_t
                                 const uint64_t *payload_ptr, const uint64_t *payload_len,
                                 const uint8_t *kind, void *fv_plan, void **plan);
 
+/* As pots_leaf_plan_create (fv_plan null) or pots_leaf_plan_create_fused, with the consecutive
+ * chunks that a lane of the chunk kernels hashes given: run 1 to 4, or 0 for the plan's own
+ * choice, which the other two take (by the number of chunks; few chunks take four lanes each, a
+ * run given never does). Results do not depend on it. No counterpart in the reference. */
+int pots_leaf_plan_create_runs(size_t n, const uint8_t *hdr_buf, const uint64_t *hdr_off,
+                               const uint32_t *hdr_len, const uint32_t *hdr_idx,
+                               const uint64_t *payload_ptr, const uint64_t *payload_len,
+                               const uint8_t *kind, void *fv_plan, uint32_t run, void **plan);
+
 /* Leaves of the plan whose product's P-pass sums its chunk stage takes (0 for an unfused
  * plan). */
 uint32_t pots_leaf_plan_fused(const void *plan);

@@ -958,8 +958,8 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
                       const uint64_t* payload_ptr, const uint64_t* payload_len,
                       const uint8_t* kind, bool device_only, bool owned, void* fv,
                       LeafPlan** out, char* ext_base = nullptr, size_t ext_cap = 0,
-                      void* pinned = nullptr) {
-  if (n == 0 || n >= 0xFFFFFFFFull) return POTS_E_ARG;
+                      void* pinned = nullptr, uint32_t run_asked = 0) {
+  if (n == 0 || n >= 0xFFFFFFFFull || run_asked > kRun) return POTS_E_ARG;
   for (size_t i = 0; i < n; i++)
     if (kind[i] > POTS_KIND_F16) return POTS_E_ARG;
   LeafPlan* P = new (std::nothrow) LeafPlan;
@@ -982,7 +982,7 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
   uint64_t plain_chunks = 0, all_chunks = 0;
   for (size_t i = 0; i < n; i++)
     all_chunks += (payload_len[i] >> 10) + 1;
-  const uint32_t lrun = run_for(all_chunks);
+  const uint32_t lrun = run_asked ? run_asked : run_for(all_chunks);
   uint64_t nc = 0;
   for (size_t i = 0; i < n; i++) {
     const uint32_t u = hdr_idx[i];
@@ -1078,7 +1078,7 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
     return POTS_E_ARG;
   }
 
-  P->quad = plain_chunks <= kQuadMost;
+  P->quad = !run_asked && plain_chunks <= kQuadMost;
   plain.run = P->quad ? 1 : lrun;
   for (uint32_t i : plain_leaves) plain.add(i, (desc[i].n_chunks + plain.run - 1) / plain.run);
   if (!plain.finish(P->quad ? kQuadChunks : kThreads) || !fused.finish(kThreads)) {
@@ -1509,6 +1509,19 @@ extern "C" int pots_leaf_plan_create_fused(size_t n, const uint8_t* hdr_buf,
   LeafPlan* P = nullptr;
   int rc = plan_build(n, hdr_buf, hdr_off, hdr_len, hdr_idx, payload_ptr, payload_len, kind,
                       /*device_only=*/true, /*owned=*/true, fv_plan, &P);
+  if (rc == POTS_E_OK) *plan = P;
+  return rc;
+}
+
+extern "C" int pots_leaf_plan_create_runs(size_t n, const uint8_t* hdr_buf,
+                                          const uint64_t* hdr_off, const uint32_t* hdr_len,
+                                          const uint32_t* hdr_idx, const uint64_t* payload_ptr,
+                                          const uint64_t* payload_len, const uint8_t* kind,
+                                          void* fv_plan, uint32_t run, void** plan) {
+  if (!plan) return POTS_E_ARG;
+  LeafPlan* P = nullptr;
+  int rc = plan_build(n, hdr_buf, hdr_off, hdr_len, hdr_idx, payload_ptr, payload_len, kind,
+                      /*device_only=*/true, /*owned=*/true, fv_plan, &P, nullptr, 0, nullptr, run);
   if (rc == POTS_E_OK) *plan = P;
   return rc;
 }

@@ -127,6 +127,8 @@ class Native:
             "pots_leaf_plan_destroy": ([_vp], None),
             "pots_leaf_plan_create_fused": ([_sz, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                              ctypes.POINTER(_vp)], _int),
+            "pots_leaf_plan_create_runs": ([_sz, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _u32,
+                                            ctypes.POINTER(_vp)], _int),
             "pots_leaf_plan_fused": ([_vp], _u32),
             "pots_leaf_plan_fused_stats": ([_vp, _vp, _vp, _vp], _int),
             "pots_step_run": ([_vp, _vp, _vp, _vp, _vp, _vp, _vp], _int),
@@ -312,12 +314,13 @@ class Native:
         return UpdatePlan(self, weights, eta, eps_w)
 
     def leaf_plan(self, headers: Sequence[bytes], payloads: Sequence[torch.Tensor],
-                  kinds: Sequence[int], fuse: FvPlan | None = None) -> LeafPlan:
+                  kinds: Sequence[int], fuse: FvPlan | None = None, run: int = 0) -> LeafPlan:
         """A reusable hashing plan over GPU-resident payloads: leaf ``i`` is
         ``BLAKE3(0x00 ‖ headers[i] ‖ payload bytes of payloads[i])``. With ``fuse``, the
         leaves that are the P of a product of that Freivalds plan also have its P-pass sums
-        taken by the chunk stage (``pots_leaf_plan_create_fused``)."""
-        return LeafPlan(self, headers, payloads, kinds, fuse)
+        taken by the chunk stage (``pots_leaf_plan_create_fused``). ``run``: the consecutive
+        chunks a lane hashes, 1 to 4 (0: the plan's choice); results do not depend on it."""
+        return LeafPlan(self, headers, payloads, kinds, fuse, run)
 
     def step_run(self, leaf: LeafPlan, fv: FvPlan, key: torch.Tensor, digests: torch.Tensor,
                  bad: torch.Tensor, rows: torch.Tensor,
@@ -337,7 +340,7 @@ class LeafPlan:
     every leaf on a stream with no allocation and no host sync."""
 
     def __init__(self, lib: Native, headers: Sequence[bytes], payloads: Sequence[torch.Tensor],
-                 kinds: Sequence[int], fuse: FvPlan | None = None) -> None:
+                 kinds: Sequence[int], fuse: FvPlan | None = None, run: int = 0) -> None:
         n = len(payloads)
         if not (len(headers) == len(kinds) == n) or n == 0:
             raise ValueError("one header and one kind per payload, at least one leaf")
@@ -358,7 +361,7 @@ class LeafPlan:
             ptr[i], ln[i] = t.data_ptr(), t.nbytes
         self._create(lib, b"".join(hdrs), hdr_off, hdr_len, idx, ptr, ln,
                      np.asarray(kinds, dtype=np.uint8), fuse, list(payloads),
-                     payloads[0].device)
+                     payloads[0].device, run)
 
     @classmethod
     def from_arrays(cls, lib: Native, hdr_buf: bytes, hdr_off: np.ndarray, hdr_len: np.ndarray,
@@ -375,7 +378,8 @@ class LeafPlan:
 
     def _create(self, lib: Native, hdr_buf: bytes, hdr_off: np.ndarray, hdr_len: np.ndarray,
                 idx: np.ndarray, ptr: np.ndarray, ln: np.ndarray, kd: np.ndarray,
-                fuse: FvPlan | None, keep: list[Any], device: torch.device) -> None:
+                fuse: FvPlan | None, keep: list[Any], device: torch.device,
+                run: int = 0) -> None:
         n = len(idx)
         if not (len(ptr) == len(ln) == len(kd) == n) or n == 0:
             raise ValueError("one header index, payload and kind per leaf, at least one leaf")
@@ -388,17 +392,16 @@ class LeafPlan:
         ptr = np.ascontiguousarray(ptr, dtype=np.uint64)
         ln = np.ascontiguousarray(ln, dtype=np.uint64)
         kd = np.ascontiguousarray(kd, dtype=np.uint8)
+        if not 0 <= run <= 4:
+            raise ValueError(f"run must be in [0, 4], got {run}")
+        if fuse is not None and fuse._fused_leaf is not None:
+            raise ValueError("this Freivalds plan is already fused with a leaf plan")
         h = ctypes.c_void_p()
-        if fuse is None:
-            _create(lib, lambda: lib._lib.pots_leaf_plan_create(
-                n, _addr(hb), _addr(hdr_off), _addr(hdr_len), _addr(idx), _addr(ptr), _addr(ln),
-                _addr(kd), ctypes.byref(h)), "pots_leaf_plan_create")
-        else:
-            if fuse._fused_leaf is not None:
-                raise ValueError("this Freivalds plan is already fused with a leaf plan")
-            _create(lib, lambda: lib._lib.pots_leaf_plan_create_fused(
-                n, _addr(hb), _addr(hdr_off), _addr(hdr_len), _addr(idx), _addr(ptr), _addr(ln),
-                _addr(kd), fuse._h, ctypes.byref(h)), "pots_leaf_plan_create_fused")
+        _create(lib, lambda: lib._lib.pots_leaf_plan_create_runs(
+            n, _addr(hb), _addr(hdr_off), _addr(hdr_len), _addr(idx), _addr(ptr), _addr(ln),
+            _addr(kd), None if fuse is None else fuse._h, run, ctypes.byref(h)),
+            "pots_leaf_plan_create")
+        if fuse is not None:
             fuse._fused_leaf = weakref.ref(self)
         self._h = h
         _LIVE_PLANS.add(self)
