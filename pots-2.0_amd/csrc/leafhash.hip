@@ -83,7 +83,7 @@ static_assert(sizeof(FuseDesc) == 48, "FuseDesc layout");
 struct LevelEntry {     // one leaf with >= 2 nodes at the input level of one fold
   uint64_t in_off;      // its first node in the level's input buffer
   uint64_t out_off;     // its first node in the fold's output buffer
-  uint64_t out_first;   // its first output (and block), counted over the fold's entries
+  uint64_t out_first;   // its first output, counted over the fold's entries
   uint32_t n_in;        // its nodes at this level
   uint32_t leaf;
 };
@@ -99,6 +99,8 @@ constexpr uint32_t kRun = 4;
 constexpr uint32_t kQuadChunks = 16, kQuadStride = 260;
 // Tree levels one launch of level_kernel reduces, and the nodes a block takes to reduce them.
 constexpr uint32_t kFold = 10, kTile = 1u << kFold;
+// The same of level_lanes, of which a lane takes the nodes.
+constexpr uint32_t kLaneFold = 3, kLaneTile = 1u << kLaneFold;
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4w __attribute__((ext_vector_type(4), aligned(4)));  // word aligned
@@ -766,6 +768,56 @@ __global__ __launch_bounds__(kThreads) void level_kernel(
                      cur[tid]);
 }
 
+// Levels kLaneFold at a time, for many short leaves (kShortLeast): lane t makes output t of the
+// fold, node o of its leaf at level l + kLaneFold, from the (at most kLaneTile) nodes o·kLaneTile ..
+// of level l, level by level in registers. The outputs of block b's lanes lie in entries blk_ent[b]
+// .. blk_ent[b + 1]. Latency: seven compressions in a row and a search for the leaf, some 12 us a
+// launch up to half a million nodes.
+__global__ __launch_bounds__(kThreads) void level_lanes(
+    const LevelEntry* __restrict__ ents, const uint32_t* __restrict__ blk_ent, uint64_t n_out,
+    const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
+    uint32_t* __restrict__ digests) {
+  const uint64_t t = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
+  if (t >= n_out) return;
+  uint32_t lo = blk_ent[blockIdx.x], hi = blk_ent[blockIdx.x + 1];
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi + 1) >> 1;
+    if (ents[mid].out_first <= t) lo = mid;
+    else hi = mid - 1;
+  }
+  const LevelEntry e = ents[lo];
+  const uint64_t o = t - e.out_first, first = o * kLaneTile;
+  // m: the lane's nodes at the current level; n: the leaf's
+  uint32_t m = (uint32_t)min<uint64_t>(kLaneTile, e.n_in - first), n = e.n_in;
+  const u32x4* src = reinterpret_cast<const u32x4*>(in + 8ull * (e.in_off + first));
+  uint32_t cv[kLaneTile][8];
+#pragma unroll
+  for (uint32_t a = 0; a < kLaneTile; a++) {
+    u32x4 x = {0, 0, 0, 0}, y = {0, 0, 0, 0};
+    if (a < m) {
+      x = gload<u32x4>(src + 2 * a);
+      y = gload<u32x4>(src + 2 * a + 1);
+    }
+    get8(x, y, cv[a]);
+  }
+#pragma unroll
+  for (uint32_t lvl = 0; lvl < kLaneFold; lvl++) {
+    n = (n + 1) / 2;
+    const uint32_t flags = n == 1 ? B3_ROOT : 0u;
+#pragma unroll
+    for (uint32_t a = 0; a < (kLaneTile >> (lvl + 1)); a++) {
+      if (2 * a + 1 < m) {
+        b3_parent_cv(cv[2 * a], cv[2 * a + 1], flags, cv[a]);
+      } else if (2 * a < m) {
+#pragma unroll
+        for (int q = 0; q < 8; q++) cv[a][q] = cv[2 * a][q];
+      }
+    }
+    m = (m + 1) / 2;
+  }
+  store_cv(e.n_in <= kLaneTile ? digests + 8ull * e.leaf : out + 8ull * (e.out_off + o), cv[0]);
+}
+
 // Messages that are not word aligned where they lie (a record, a view at an odd element) are
 // staged: 0x00 || header || payload in one aligned buffer. One launch writes them all, 16 bytes
 // a thread, and resets the first-bad word; a payload in host memory (to == head) is copied in
@@ -837,6 +889,7 @@ struct LevelInfo {
   uint64_t n_out;
   uint64_t blk_first;  // index of the fold's block -> entry table in blk_ent
   int in_buf, out_buf;  // 0 = cv0, 1 = cv1
+  bool lanes;           // level_lanes' fold, not level_kernel's
 };
 
 struct LeafPlan {
@@ -947,6 +1000,16 @@ static bool fuse_shape(uint64_t msg_bytes, uint32_t row_bytes, uint32_t lrun, ui
 constexpr uint64_t kQuadMost = 32768;     // chunks hashed by four lanes each, at most
 constexpr uint64_t kRunLeast = 16 << 20;  // chunks from which a lane takes kRun of them
 static uint32_t run_for(uint64_t chunks) { return chunks >= kRunLeast ? kRun : 1; }
+
+// Leaves of up to kShortNodes chunks have their trees reduced a lane per eight nodes (level_lanes)
+// where a plan holds more than kShortLeast of them, else a block per leaf (level_kernel), whose
+// latency is shorter but which spends a block's start and the few lanes of its last levels on each.
+// Lanes / blocks, us, for 2, 9, 64, 300 and 600 chunks a leaf:
+//   1000 leaves 11 / 12, 22 / 12, 31 / 14, 40 / 24, 60 / 31;  4000: 12 / 13, 23 / 21, 32 / 27,
+//   63 / 55, 91 / 78;  8000: 12 / 17, 23 / 32, 35 / 43, 83 / 93, 142 / 136;  16000: 12 / 26,
+//   23 / 52, 46 / 76, 132 / 165;  64000: 12 / 73, 37 / 186, 106 / 267
+constexpr uint64_t kShortLeast = 5000;
+constexpr uint32_t kShortNodes = 512;
 
 // Pinned memory of the synchronous entry point, per direction: a plan's metadata on the way up,
 // digests on the way down. Larger ones (some 5000 leaves, 32 thousand) take pageable copies.
@@ -1086,9 +1149,10 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
     return POTS_E_ARG;
   }
 
-  // Reduction folds of kFold levels each. Level 0 nodes of leaf i sit at desc[i].cv_first in
-  // cv0; a fold takes a leaf's n nodes to ceil(n / kTile) (BLAKE3's halving with a promoted
-  // odd node, kFold times, composes to that ceiling), a block each.
+  // Reduction folds of kFold levels each, or kLaneFold. Level 0 nodes of leaf i sit at
+  // desc[i].cv_first in cv0; a fold takes a leaf's n nodes to ceil(n / kTile) (BLAKE3's halving
+  // with a promoted odd node, kFold times, composes to that ceiling), a block each, or to
+  // ceil(n / kLaneTile), a lane each.
   std::vector<LevelEntry> ents;
   std::vector<uint32_t> blk_ent;
   std::vector<uint64_t> n_nodes(n), off(n);
@@ -1096,39 +1160,49 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
     n_nodes[i] = desc[i].n_chunks;
     off[i] = desc[i].cv_first;
   }
+  uint64_t n_short = 0;
+  for (size_t i = 0; i < n; i++) n_short += n_nodes[i] >= 2 && n_nodes[i] <= kShortNodes;
+  const uint32_t short_most = n_short > kShortLeast ? kShortNodes : 0;
   uint64_t cv1_need = 0;
   int in_buf = 0;
-  for (;;) {
-    LevelInfo li{ents.size(), 0, 0, blk_ent.size(), in_buf, 1 - in_buf};
+  for (bool more = true; more;) {
     uint64_t out_next = 0;
-    for (size_t i = 0; i < n; i++) {
-      if (n_nodes[i] < 2) continue;
-      const uint64_t nout = (n_nodes[i] + kTile - 1) >> kFold;
-      LevelEntry e;
-      e.in_off = off[i];
-      e.out_off = out_next;
-      e.out_first = li.n_out;
-      e.n_in = (uint32_t)n_nodes[i];
-      e.leaf = (uint32_t)i;
-      ents.push_back(e);
-      li.n_out += nout;
-      li.n_ents++;
-      off[i] = out_next;
-      n_nodes[i] = nout;
-      out_next += nout;
+    more = false;
+    for (const bool lanes : {false, true}) {
+      const uint32_t fold = lanes ? kLaneFold : kFold;
+      LevelInfo li{ents.size(), 0, 0, blk_ent.size(), in_buf, 1 - in_buf, lanes};
+      for (size_t i = 0; i < n; i++) {
+        if (n_nodes[i] < 2 || (desc[i].n_chunks <= short_most) != lanes) continue;
+        const uint64_t nout = (n_nodes[i] + (1u << fold) - 1) >> fold;
+        LevelEntry e;
+        e.in_off = off[i];
+        e.out_off = out_next;
+        e.out_first = li.n_out;
+        e.n_in = (uint32_t)n_nodes[i];
+        e.leaf = (uint32_t)i;
+        ents.push_back(e);
+        li.n_out += nout;
+        li.n_ents++;
+        off[i] = out_next;
+        n_nodes[i] = nout;
+        out_next += nout;
+      }
+      if (li.n_ents == 0) continue;
+      if (li.n_out >= 0x7FFFFFFFull) {
+        delete P;
+        return POTS_E_ARG;
+      }
+      // Per block (level_kernel: one output each; level_lanes: kThreads), the fold-relative index
+      // of its first output's entry; of level_lanes' a closing bound too.
+      for (uint32_t k = 0; k < li.n_ents; k++) {
+        const uint64_t end = k + 1 < li.n_ents ? ents[li.ent_first + k + 1].out_first : li.n_out;
+        blk_ent.resize(li.blk_first + (lanes ? (end + kThreads - 1) / kThreads : end), k);
+      }
+      if (lanes) blk_ent.push_back(li.n_ents - 1);
+      P->levels.push_back(li);
+      more = true;
     }
-    if (li.n_ents == 0) break;
-    if (li.n_out >= 0x7FFFFFFFull) {
-      delete P;
-      return POTS_E_ARG;
-    }
-    // Per block (one output each): the fold-relative index of its entry.
-    for (uint32_t k = 0; k < li.n_ents; k++) {
-      const uint64_t end = k + 1 < li.n_ents ? ents[li.ent_first + k + 1].out_first : li.n_out;
-      blk_ent.resize(li.blk_first + end, k);
-    }
-    if (li.out_buf == 1) cv1_need = std::max(cv1_need, out_next);
-    P->levels.push_back(li);
+    if (in_buf == 0) cv1_need = std::max(cv1_need, out_next);
     in_buf = 1 - in_buf;
   }
 
@@ -1337,9 +1411,15 @@ static int plan_stage(LeafPlan* P, int stage, uint32_t* d_digests, uint32_t* d_f
       return POTS_E_OK;
     case 2:
       for (const LevelInfo& li : P->levels) {
-        hipLaunchKernelGGL(level_kernel, dim3((uint32_t)li.n_out), dim3(kThreads), 0, stream,
-                           P->d_levels + li.ent_first, P->d_blk_ent + li.blk_first,
-                           P->d_cv[li.in_buf], P->d_cv[li.out_buf], d_digests);
+        if (li.lanes)
+          hipLaunchKernelGGL(level_lanes, dim3((uint32_t)((li.n_out + kThreads - 1) / kThreads)),
+                             dim3(kThreads), 0, stream, P->d_levels + li.ent_first,
+                             P->d_blk_ent + li.blk_first, li.n_out, P->d_cv[li.in_buf],
+                             P->d_cv[li.out_buf], d_digests);
+        else
+          hipLaunchKernelGGL(level_kernel, dim3((uint32_t)li.n_out), dim3(kThreads), 0, stream,
+                             P->d_levels + li.ent_first, P->d_blk_ent + li.blk_first,
+                             P->d_cv[li.in_buf], P->d_cv[li.out_buf], d_digests);
         POTS_HIP(hipGetLastError());
       }
       return POTS_E_OK;

@@ -105,3 +105,31 @@ def test_outer_tree_at_tile_edges(lib, n):
     d = torch.randint(0, 256, (n, 32), device=DEV, dtype=torch.uint8)
     want = O.merkle_tree([bytes(x) for x in d.cpu().numpy()])
     assert lib.merkle_tree_device(d).cpu().numpy().tobytes() == want
+
+
+@pytest.mark.parametrize("short", [5000, 5001])  # a block a leaf, a lane per eight nodes
+def test_leaf_trees_of_many_short_leaves(lib, short):
+    """Short leaves of every shape around a lane's eight nodes and its folds, up to 512 chunks, and
+    longer ones and single chunks among them."""
+    from verification.commitment import native
+    edges = [2, 3, 7, 8, 9, 10, 15, 16, 17, 63, 64, 65, 72, 73, 511, 512]
+    chunks = edges + [2 + i % 9 for i in range(short - len(edges))]
+    for at, c in ((0, 513), (7, 1), (100, 1025), (len(chunks) // 2, 2049), (len(chunks), 1)):
+        chunks.insert(at, c)
+    flat = torch.randint(0, 2**31 - 1, (sum(chunks) * 256,), device=DEV, dtype=torch.int32)
+    ts, at = [], 0
+    for i, c in enumerate(chunks):
+        n = (1024 * c - 8 - 4 * (i % 200)) // 4
+        ts.append(flat[at:at + n])
+        at += n
+    heads = [O.tensor_leaf_header(2, t) for t in ts]
+    host, at, items = flat.cpu(), 0, []
+    for h, t in zip(heads, ts):
+        items.append((h, host[at:at + t.numel()], 0))
+        at += t.numel()
+    want, _ = O.hash_leaves(items, simd=O.simd_degree() > 1)
+    plan = lib.leaf_plan(heads, ts, [native.KIND_NONE] * len(ts))
+    assert plan.chunks == sum(chunks)
+    for _ in range(2):
+        assert [bytes(x) for x in plan.run()[0].cpu().numpy()] == want
+    plan.close()
