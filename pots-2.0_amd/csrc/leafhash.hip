@@ -1002,13 +1002,15 @@ constexpr uint64_t kRunLeast = 16 << 20;  // chunks from which a lane takes kRun
 static uint32_t run_for(uint64_t chunks) { return chunks >= kRunLeast ? kRun : 1; }
 
 // Leaves of up to kShortNodes chunks have their trees reduced a lane per eight nodes (level_lanes)
-// where a plan holds more than kShortLeast of them, else a block per leaf (level_kernel), whose
+// where a plan holds kShortLeast of them or more, else a block per leaf (level_kernel), whose
 // latency is shorter but which spends a block's start and the few lanes of its last levels on each.
 // Lanes / blocks, us, for 2, 9, 64, 300 and 600 chunks a leaf:
 //   1000 leaves 11 / 12, 22 / 12, 31 / 14, 40 / 24, 60 / 31;  4000: 12 / 13, 23 / 21, 32 / 27,
 //   63 / 55, 91 / 78;  8000: 12 / 17, 23 / 32, 35 / 43, 83 / 93, 142 / 136;  16000: 12 / 26,
 //   23 / 52, 46 / 76, 132 / 165;  64000: 12 / 73, 37 / 186, 106 / 267
-constexpr uint64_t kShortLeast = 5000;
+// and for 6782 of 3 to 433 chunks among longer ones (a 135M-parameter step) 163 / 155: the line
+// lies where lanes are ahead at every length up to kShortNodes.
+constexpr uint64_t kShortLeast = 8000;
 constexpr uint32_t kShortNodes = 512;
 
 // Pinned memory of the synchronous entry point, per direction: a plan's metadata on the way up,
@@ -1162,7 +1164,7 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
   }
   uint64_t n_short = 0;
   for (size_t i = 0; i < n; i++) n_short += n_nodes[i] >= 2 && n_nodes[i] <= kShortNodes;
-  const uint32_t short_most = n_short > kShortLeast ? kShortNodes : 0;
+  const uint32_t short_most = n_short >= kShortLeast ? kShortNodes : 0;
   uint64_t cv1_need = 0;
   int in_buf = 0;
   for (bool more = true; more;) {

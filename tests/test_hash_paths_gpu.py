@@ -107,7 +107,7 @@ def test_outer_tree_at_tile_edges(lib, n):
     assert lib.merkle_tree_device(d).cpu().numpy().tobytes() == want
 
 
-@pytest.mark.parametrize("short", [5000, 5001])  # a block a leaf, a lane per eight nodes
+@pytest.mark.parametrize("short", [7999, 8000])  # a block a leaf, a lane per eight nodes
 def test_leaf_trees_of_many_short_leaves(lib, short):
     """Short leaves of every shape around a lane's eight nodes and its folds, up to 512 chunks, and
     longer ones and single chunks among them."""
