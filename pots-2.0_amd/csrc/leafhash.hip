@@ -439,8 +439,17 @@ struct Order {
   const uint32_t* __restrict__ blk_ent;
   uint64_t n_slots;   // slots of the order
   uint32_t n_blocks;  // ceil(n_slots / slots per block)
-  uint32_t run;       // chunks per slot (the plain order)
+  uint32_t run;       // chunks per slot (the plain order: lane_run)
+  uint32_t short_most;
 };
+
+// Chunks per slot of a leaf of n chunks, in a plain order of runs of `run`: a leaf of up to
+// short_most chunks takes runs of kRun, where those leave no more than 1/16 of their chunks empty
+// (a leaf of up to kRun chunks is one run, whatever its length).
+__host__ __device__ constexpr uint32_t lane_run(uint32_t n, uint32_t run, uint32_t short_most) {
+  return n <= short_most && (n <= kRun || (kRun - 1 - (n + kRun - 1) % kRun) * 16 <= n) ? kRun
+                                                                                        : run;
+}
 
 __device__ __forceinline__ uint32_t order_entry(const Order& od, uint64_t g, uint32_t blk) {
   uint32_t lo = od.blk_ent[blk], hi = od.blk_ent[blk + 1];
@@ -478,7 +487,8 @@ __device__ __forceinline__ void hash_run(const LeafDesc& d, const uint32_t* __re
 }
 
 // Every chunk of the unfused leaves: slot g of the plain order is run g − first[e] of leaf
-// leaf[e], its chunks run·(g − first[e]) onwards (slots past a leaf's runs are idle). Block b
+// leaf[e], its chunks run·(g − first[e]) onwards, run the leaf's lane_run (slots past a leaf's runs
+// are idle). Block b
 // hashes slot blocks b, b + gridDim.x, ... so a grid smaller than the order holds a bounded
 // share of the GPU and leaves the rest to kernels on other streams.
 __global__ __launch_bounds__(kThreads) void chunk_kernel(
@@ -491,9 +501,10 @@ __global__ __launch_bounds__(kThreads) void chunk_kernel(
     const uint32_t e = order_entry(od, g, blk);
     const uint32_t i = od.leaf[e];
     const LeafDesc d = leaves[i];
-    const uint64_t c0 = (g - od.first[e]) * od.run;
+    const uint32_t run = lane_run(d.n_chunks, od.run, od.short_most);
+    const uint64_t c0 = (g - od.first[e]) * run;
     if (c0 >= d.n_chunks) continue;
-    const uint64_t c1 = min<uint64_t>(c0 + od.run, d.n_chunks);
+    const uint64_t c1 = min<uint64_t>(c0 + run, d.n_chunks);
     Fin fin(d.kind);
     switch ((uint32_t)((d.payload - d.head_len) >> 2) & 3u) {
       case 0: hash_run<0>(d, head, i, c0, c1, fin, cv_out, digests); break;
@@ -926,7 +937,7 @@ struct OrderHost {
   std::vector<uint32_t> blk_ent;
   uint64_t n_slots = 0;
   uint32_t n_blocks = 0;
-  uint32_t run = 1;  // chunks per slot (the plain order)
+  uint32_t run = 1, short_most = 0;  // the plain order's (lane_run)
   void add(uint32_t i, uint64_t slots) {
     first.push_back(n_slots);
     leaf.push_back(i);
@@ -1000,6 +1011,49 @@ static bool fuse_shape(uint64_t msg_bytes, uint32_t row_bytes, uint32_t lrun, ui
 constexpr uint64_t kQuadMost = 32768;     // chunks hashed by four lanes each, at most
 constexpr uint64_t kRunLeast = 16 << 20;  // chunks from which a lane takes kRun of them
 static uint32_t run_for(uint64_t chunks) { return chunks >= kRunLeast ? kRun : 1; }
+
+// Many short leaves keep runs of kRun: a wave of single chunks goes through the header's path, the
+// last block's and the whole blocks' for the sake of a few lanes each, a wave of runs once for the
+// whole run. One chunk a lane / four, us, leaves at one word shift (and at all four, whose paths a
+// wave of small leaves takes in turn either way), thousands of them:
+//   2 chunks  64: 77 / 58 (370 / 184), 256: 261 / 175 (976 / 560);  3 chunks  43: 78 / 81
+//   (267 / 278), 87: 136 / 136, 175: 267 / 219 (902 / 691);  4 chunks  64: 125 / 103 (437 / 350);
+//   8 chunks  32: 137 / 136 (472 / 487), 64: 265 / 237 (884 / 814);  9 chunks  58: 262 / 319;
+//   24 chunks  11: 134 / 134 (443 / 452), 44: 503 / 448 (1500 / 1451);  64 chunks  16: 470 / 418
+//   (466 / 1443), 33: 933 / 810 (943 / 2782)
+// So leaves of up to 24 chunks, and of up to 128 where all of them lie at one shift (with several,
+// a wave of longer leaves' single chunks still has one), wherever runs take no more time by the
+// rounds of 64 Ki lanes they fill (a wave on every SIMD): a run takes its blocks, a single chunk
+// sixteen and an eighth more.
+constexpr uint32_t kShortMixed = 24, kShortAlike = 128;
+
+struct RunCount {
+  uint64_t runs = 0, chunks = 0, blocks = 0;
+  void add(uint32_t n_chunks, uint64_t bytes) {
+    runs += (n_chunks + kRun - 1) / kRun;
+    chunks += n_chunks;
+    blocks += (bytes + 63) / 64;
+  }
+  bool pay() const {
+    constexpr uint64_t kRound = 64 << 10;
+    return runs > 0 && (double)((runs + kRound - 1) / kRound) * (double)blocks / (double)runs <=
+                           (double)((chunks + kRound - 1) / kRound) * 18.0;
+  }
+};
+
+static uint32_t short_for(const std::vector<LeafDesc>& desc, const std::vector<uint32_t>& leaves) {
+  RunCount mixed, alike;
+  uint32_t shifts = 0;
+  for (uint32_t i : leaves) {
+    const LeafDesc& d = desc[i];
+    if (d.n_chunks < 2 || lane_run(d.n_chunks, 1, kShortAlike) != kRun) continue;
+    alike.add(d.n_chunks, d.head_len + d.len);
+    if (d.n_chunks <= kShortMixed) mixed.add(d.n_chunks, d.head_len + d.len);
+    shifts |= 1u << ((d.payload - d.head_len) >> 2 & 3);
+  }
+  if ((shifts & (shifts - 1)) == 0 && alike.pay()) return kShortAlike;
+  return mixed.pay() ? kShortMixed : 0;
+}
 
 // Leaves of up to kShortNodes chunks have their trees reduced a lane per eight nodes (level_lanes)
 // where a plan holds kShortLeast of them or more, else a block per leaf (level_kernel), whose
@@ -1145,7 +1199,11 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
 
   P->quad = !run_asked && plain_chunks <= kQuadMost;
   plain.run = P->quad ? 1 : lrun;
-  for (uint32_t i : plain_leaves) plain.add(i, (desc[i].n_chunks + plain.run - 1) / plain.run);
+  if (!P->quad && !run_asked) plain.short_most = short_for(desc, plain_leaves);
+  for (uint32_t i : plain_leaves) {
+    const uint32_t run = lane_run(desc[i].n_chunks, plain.run, plain.short_most);
+    plain.add(i, ((uint64_t)desc[i].n_chunks + run - 1) / run);
+  }
   if (!plain.finish(P->quad ? kQuadChunks : kThreads) || !fused.finish(kThreads)) {
     delete P;
     return POTS_E_ARG;
@@ -1287,6 +1345,7 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
     dords[k]->n_slots = ords[k]->n_slots;
     dords[k]->n_blocks = ords[k]->n_blocks;
     dords[k]->run = ords[k]->run;
+    dords[k]->short_most = ords[k]->short_most;
   }
   P->d_head = reinterpret_cast<uint32_t*>(P->base + o_head);
   P->d_levels = reinterpret_cast<LevelEntry*>(P->base + o_lev);

@@ -133,3 +133,36 @@ def test_leaf_trees_of_many_short_leaves(lib, short):
     for _ in range(2):
         assert [bytes(x) for x in plan.run()[0].cpu().numpy()] == want
     plan.close()
+
+
+@pytest.mark.parametrize("step", [256, 257])  # words between payloads: one word shift, all four
+@pytest.mark.parametrize("kind", ["none", "float"])
+def test_runs_of_many_short_leaves(lib, step, kind):
+    """Leaves of 2 to 5 chunks and around the lengths that take runs of four, past the number from
+    which they do; longer ones and single chunks among them."""
+    from verification.commitment import native
+    edges = [5, 6, 7, 8, 9, 12, 15, 16, 18, 19, 20, 23, 24, 25, 27, 28, 64, 127, 128, 129, 132]
+    chunks = [2 + i % 3 for i in range(65400)] + edges * 8 + [1, 500, 2048]
+    tails = (0, 1, 16, 17, 31, 32, 33, 250)  # words the last chunk lacks
+    flat = torch.randn(1 << 20, device=DEV)
+    host = flat.cpu()
+    ts, items, at = [], [], 0
+    for i, c in enumerate(chunks):
+        n = 256 * c - 2 - tails[i % len(tails)]
+        at = (at + step) % ((1 << 20) - 256 * 2049)
+        ts.append(flat[at:at + n])
+        items.append((at, n))
+    k = native.KIND_NONE if kind == "none" else native.KIND_F32
+    heads = [O.tensor_leaf_header(2, t) for t in ts]
+    want, _ = O.hash_leaves([(h, host[a:a + n], 0) for h, (a, n) in zip(heads, items)],
+                            simd=O.simd_degree() > 1)
+    plan = lib.leaf_plan(heads, ts, [k] * len(ts))
+    d, bad = plan.run()
+    assert int(bad) == len(ts) and [bytes(x) for x in d.cpu().numpy()] == want
+    if kind == "float":  # the second chunk's first word and the last word of one leaf
+        for word in (items[70][0] + 254, items[70][0] + items[70][1] - 1):
+            flat[word] = float("nan")
+            first = next(i for i, (a, n) in enumerate(items) if a <= word < a + n)
+            assert int(plan.run()[1]) == first
+            flat[word] = 1.0
+    plan.close()
