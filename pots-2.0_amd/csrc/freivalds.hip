@@ -1761,8 +1761,19 @@ static uint64_t pad32(uint64_t rows) { return (rows + 31) / 32 * 32; }
 // 12, 14, 12 / 11, 9, 10; of eight 1000 x 2050 x 1537 bf16 ones under sixteen challenges 49, 30,
 // 33 / 45, 24, 24; the B pass of an 8192 x 4096 x 4096 fp32 one 25 / 17. (2048 tiles wanted:
 // its A pass 28 -> 35, each chunk's partials costing more than its block hides.)
+//
+// And no further than pays: a column of a chunk is some 0.01 us of its tile's chain (0.005 in
+// bf16), a chunk 0.06 + 0.011 k us of the finish's, which adds a row's chunks one after another, so
+// halving a chunk to c columns is worth it while 20 c² (10 c²) is at least cols·(60 + 11 k). An fp32
+// product of 100 x 16384 x 64 under 4, 16, 64 and 255 challenges, us, whole chunks / cut to 128
+// columns / this: 56, 69, 146, 1296 / 58, 88, 249, 8014 / 40, 53, 120, 1245; one of 1000 x 4096 x
+// 4096 101, 119, 245, 2463 / 64, 90, 274, 4672 / 56, 77, 169, 873.
 constexpr uint64_t kTilesWanted = 1024;
 constexpr uint32_t kLeastF32 = 128, kLeastBf16 = 512, kLeastBf16B = 1024;
+
+static bool cut_pays(uint32_t dt, uint64_t c, uint64_t cols, uint64_t k) {
+  return (dt == DT_BF16 ? 10 : 20) * c * c >= cols * (60 + 11 * k);
+}
 
 static uint32_t chunk_cols_for(uint32_t cols, uint32_t sstep, uint32_t cmax) {
   // At most cmax columns per chunk, in whole pipeline stages, balanced over the chunks (cmax
@@ -1890,7 +1901,12 @@ extern "C" int pots_fv_plan_create(size_t n, const pots_fv_product* prods, uint3
   // fewer than kTilesWanted tiles. A tile is a chain of stages, each a load's latency, and it
   // takes several blocks on a CU to hide one another's.
   auto chunk_most = [&](uint32_t dt, uint32_t most, uint32_t least, auto&& shape_of) {
-    for (; most > least; most /= 2) {
+    uint32_t widest = 0;
+    for (size_t i = 0; i < n; i++) {
+      const Shape s = shape_of(i);
+      if (s.dt == dt) widest = std::max(widest, s.cols);
+    }
+    for (; most > least && cut_pays(dt, most / 2, widest, k); most /= 2) {
       uint64_t tiles = 0;
       for (size_t i = 0; i < n && tiles < kTilesWanted; i++) {
         const Shape s = shape_of(i);

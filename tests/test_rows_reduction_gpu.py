@@ -78,3 +78,16 @@ def test_fused_records_match_oracle(lib, dtype, n, w, k):
     assert [bytes(x) for x in digests.cpu().numpy()] == \
         [O.tensor_leaf_hash(3, p.cpu()) for p in ps]
     fv.close()
+
+@pytest.mark.parametrize("k", [1, 4, 64, 255])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_wide_products_under_few_and_many_challenges(lib, dtype, k):
+    """Small plans whose chunks are cut as far as their columns and challenges say: a wide A, a
+    wide B and P."""
+    from verification.commitment.native import FvProduct
+    prods = [_product(40, 9001, 70, dtype, False, 7), _product(70, 45, 9001, dtype, True, 8)]
+    plan = lib.fv_plan([FvProduct(a, b, p, m, bv) for m, (a, b, p, bv) in enumerate(prods, 1)], k)
+    rows = plan.rows(ROOT).cpu().tolist()
+    for m, prod in enumerate(prods, 1):
+        _check(rows[m - 1], prod, m, k)
+    plan.close()
