@@ -1569,7 +1569,7 @@ __global__ __launch_bounds__(64) void finish_final(const FinJob* __restrict__ jo
 struct FixJob {
   uint64_t p, r, seg;        // P, R [w][k], run records [J][n]
   uint64_t pdot, pabs, psq;  // the P job's partials: column chunk 0 of [rows_pad]
-  uint64_t row_first;        // prefix of rows over the jobs before it
+  uint64_t row_first;        // prefix of rows over its launch's jobs before it
   uint32_t n, w;
   uint32_t head, esz;
   uint32_t J, pad;           // record slots per row
@@ -1581,24 +1581,30 @@ static_assert(sizeof(FixJob) == 80, "FixJob layout");
 // row), which no chunk's interior pairs took. Rounded to the P job's partial formats as one
 // column chunk.
 //
-// A block takes 64 rows; each of its four waves adds every fourth record of them (a lane a row,
-// so a wave's loads are contiguous), four records' loads in flight, and the first wave adds the
-// waves' sums in wave order. (A thread per row was one chain of loads as long as the row's
-// records, 298 for a 151936-column product: 1017 us beside the hashing in a two-layer step,
-// where this takes 720, 62 alone.)
+// W waves share 64 rows, a lane a row (so a wave's loads are contiguous): each adds every W'th
+// record of them, four records' loads in flight, and the first adds the waves' sums in wave order.
+// Rows of up to kFixShort record slots are a wave's alone, 256 to a block: their few loads are all
+// in flight at once, and a wave that reads every fourth of a dozen only shares its start with
+// three more. 524288 rows of 4, 9 and 11 slots 44, 53 and 55 us (four waves 84, 95, 96), 131072 of
+// 19 and 33 32 and 40 (43, 49). Longer rows are few, as a rule, and a wave's chain of loads the
+// time: 8192 rows of 129 slots 32 / 24, 298 slots (151936 columns) beside the hashing of a two-layer
+// step 1017 / 720; 32768 rows of 49 to 129 slots are equal either way.
 // `blk[b]`: the job of block b's first row (blk[gridDim.x] the last job), so a thread searches
 // only the few jobs its block's rows span instead of all of them (a dozen dependent loads).
-constexpr uint32_t kFixRows = 64;
+constexpr uint32_t kFixShort = 48;
+constexpr uint32_t kFixWaves[2] = {1, 4};  // per 64 rows: up to kFixShort records a row, more
+constexpr uint32_t fix_rows(uint32_t waves) { return 256 / waves; }  // of a block
 
-template <int K>
+template <int K, uint32_t W>
 __global__ __launch_bounds__(256) void fused_rows(const FixJob* __restrict__ jobs,
                                                   const uint32_t* __restrict__ blk,
                                                   uint64_t n_rows) {
-  __shared__ double s_sum[3][K + 2][kFixRows];
-  __shared__ uint32_t s_exact[3][kFixRows];
-  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  constexpr uint32_t kRows = fix_rows(W), kSums = W > 1 ? W - 1 : 1;
+  __shared__ double s_sum[kSums][K + 2][kRows];
+  __shared__ uint32_t s_exact[kSums][kRows];
+  const uint32_t wave = threadIdx.x / kRows, lane = threadIdx.x % kRows;
   // (lanes past the last row take it too and write nothing)
-  const uint64_t g0 = (uint64_t)blockIdx.x * kFixRows + lane, g = min(g0, n_rows - 1);
+  const uint64_t g0 = (uint64_t)blockIdx.x * kRows + lane, g = min(g0, n_rows - 1);
   uint32_t lo = blk[blockIdx.x], hi = blk[blockIdx.x + 1];
   while (lo < hi) {
     const uint32_t mid = (lo + hi + 1) >> 1;
@@ -1625,31 +1631,35 @@ __global__ __launch_bounds__(256) void fused_rows(const FixJob* __restrict__ job
     d[K + 1] += __longlong_as_double((long long)((uint64_t)b.w << 32 | b.z));
   };
   uint32_t c = wave;
-  for (; c + 12 < count; c += 16) {
+  for (; c + 3 * W < count; c += 4 * W) {
     v4f32 a[4];
     u32x4 b[4];
 #pragma unroll
     for (uint32_t u = 0; u < 4; u++) {
-      a[u] = gload<v4f32>(rec + (c + 4 * u) * stride);
-      b[u] = gload<u32x4>(rec + (c + 4 * u) * stride + 16);
+      a[u] = gload<v4f32>(rec + (c + W * u) * stride);
+      b[u] = gload<u32x4>(rec + (c + W * u) * stride + 16);
     }
 #pragma unroll
     for (int u = 0; u < 4; u++) add(a[u], b[u]);
   }
-  for (; c < count; c += 4)
+  for (; c < count; c += W)
     add(gload<v4f32>(rec + c * stride), gload<u32x4>(rec + c * stride + 16));
-  if (wave) {
+  if constexpr (W > 1) {
+    if (wave) {
 #pragma unroll
-    for (int j = 0; j < K + 2; j++) s_sum[wave - 1][j][lane] = d[j];
-    s_exact[wave - 1][lane] = exact ? 1u : 0u;
+      for (int j = 0; j < K + 2; j++) s_sum[wave - 1][j][lane] = d[j];
+      s_exact[wave - 1][lane] = exact ? 1u : 0u;
+    }
+    __syncthreads();
   }
-  __syncthreads();
   if (wave || g0 >= n_rows) return;
+  if constexpr (W > 1) {
 #pragma unroll
-  for (int w = 0; w < 3; w++) {
+    for (uint32_t w = 0; w < W - 1; w++) {
 #pragma unroll
-    for (int j = 0; j < K + 2; j++) d[j] += s_sum[w][j][lane];
-    exact |= s_exact[w][lane] != 0u;
+      for (int j = 0; j < K + 2; j++) d[j] += s_sum[w][j][lane];
+      exact |= s_exact[w][lane] != 0u;
+    }
   }
   const float* R = reinterpret_cast<const float*>(J.r);
   auto elem = [&](uint64_t e) {
@@ -1746,8 +1756,8 @@ struct FvPlan {
   char* fbase = nullptr;
   FixJob* d_fix = nullptr;
   uint32_t n_fix = 0;
-  uint64_t n_fix_rows = 0;
-  uint32_t* d_fix_blk = nullptr;  // block -> first fix-up job (fused_rows)
+  uint64_t n_fix_rows[2] = {0, 0};  // of the jobs of few records a row, of the others
+  uint32_t* d_fix_blk[2] = {nullptr, nullptr};  // block -> first fix-up job (fused_rows)
 };
 
 // Packed operands (R, B·R) hold whole 32-row groups, one bf16 K-step of the row pass; rows past
@@ -2369,11 +2379,30 @@ int fv_fuse_commit(void* fv, const std::vector<uint32_t>& prods,
     at = align_up(at + std::max<size_t>(bytes, 16), 256);
     return a;
   };
+  // Two launches: the products of up to kFixShort records a row, then the others.
+  std::vector<uint32_t> order;  // of `prods`
+  uint64_t fix_rows_of[2] = {0, 0};
+  uint32_t n_short = 0;
+  auto row_slots = [&](uint32_t i) {
+    const pots_fv_product& p = P->h_prods[i];
+    return (uint32_t)(((uint64_t)p.w * (p.p_dtype == DT_BF16 ? 2 : 4) + 1023) / 1024 + 1);
+  };
+  for (const bool lng : {false, true}) {
+    for (uint32_t f = 0; f < prods.size(); f++) {
+      if ((row_slots(prods[f]) > kFixShort) != lng) continue;
+      order.push_back(f);
+      fix_rows_of[lng] += P->h_prods[prods[f]].n;
+    }
+    if (!lng) n_short = (uint32_t)order.size();
+  }
+  uint64_t fix_blocks[2];
+  size_t o_fix_blk[2];
   const size_t o_fix = place(prods.size() * sizeof(FixJob));
-  uint64_t all_rows = 0;
-  for (uint32_t i : prods) all_rows += P->h_prods[i].n;
-  const uint64_t fix_blocks = (all_rows + kFixRows - 1) / kFixRows;
-  const size_t o_fix_blk = place((fix_blocks + 1) * 4);
+  for (int g = 0; g < 2; g++) {
+    const uint32_t per = fix_rows(kFixWaves[g]);
+    fix_blocks[g] = (fix_rows_of[g] + per - 1) / per;
+    o_fix_blk[g] = place((fix_blocks[g] + 1) * 4);
+  }
   std::vector<size_t> o_seg(prods.size());
   for (size_t f = 0; f < prods.size(); f++) {
     const pots_fv_product& p = P->h_prods[prods[f]];
@@ -2390,12 +2419,14 @@ int fv_fuse_commit(void* fv, const std::vector<uint32_t>& prods,
   std::vector<FixJob> fix(prods.size());
   uint64_t rows = 0;
   seg_out->assign(prods.size(), 0);
-  for (size_t f = 0; f < prods.size(); f++) {
+  for (size_t o = 0; o < order.size(); o++) {
+    const size_t f = order[o];
     const uint32_t i = prods[f];
     const pots_fv_product& p = P->h_prods[i];
     const PassJob& J = P->h_jobs[pos[2 * n + i]];
-    FixJob& x = fix[f];
+    FixJob& x = fix[o];
     memset(&x, 0, sizeof x);
+    if (o == n_short) rows = 0;
     x.p = reinterpret_cast<uint64_t>(p.p);
     x.r = reinterpret_cast<uint64_t>(P->d_r) + 4 * P->h_r_off[i];
     x.seg = fb + o_seg[f];
@@ -2407,16 +2438,19 @@ int fv_fuse_commit(void* fv, const std::vector<uint32_t>& prods,
     x.w = p.w;
     x.head = head_len[f];
     x.esz = p.p_dtype == DT_BF16 ? 2 : 4;
-    x.J = (uint32_t)(((uint64_t)p.w * x.esz + 1023) / 1024 + 1);
+    x.J = row_slots(i);
     rows += p.n;
     (*seg_out)[f] = x.seg;
   }
-  std::vector<uint32_t> fix_blk(fix_blocks + 1);
-  for (size_t f = 0, b = 0; b < fix_blocks; b++) {
-    while (f + 1 < fix.size() && fix[f + 1].row_first <= b * kFixRows) f++;
-    fix_blk[b] = (uint32_t)f;
+  std::vector<uint32_t> fix_blk[2];
+  for (int g = 0; g < 2; g++) {
+    const size_t end = g ? fix.size() : n_short;
+    for (size_t f = g ? n_short : 0, b = 0; b < fix_blocks[g]; b++) {
+      while (f + 1 < end && fix[f + 1].row_first <= b * fix_rows(kFixWaves[g])) f++;
+      fix_blk[g].push_back((uint32_t)f);
+    }
+    fix_blk[g].push_back(end ? (uint32_t)(end - 1) : 0u);
   }
-  fix_blk[fix_blocks] = fix.empty() ? 0u : (uint32_t)(fix.size() - 1);
   // The P pass without the fused products: each P launch keeps its other jobs, packed at the
   // front of its ranges of the job array and the block table.
   std::vector<PassLaunch> launches = P->pass_ap;
@@ -2448,7 +2482,8 @@ int fv_fuse_commit(void* fv, const std::vector<uint32_t>& prods,
   };
   int rc;
   if ((rc = up(fbase + o_fix, fix.data(), fix.size() * sizeof(FixJob))) ||
-      (rc = up(fbase + o_fix_blk, fix_blk.data(), fix_blk.size() * 4)) ||
+      (rc = up(fbase + o_fix_blk[0], fix_blk[0].data(), fix_blk[0].size() * 4)) ||
+      (rc = up(fbase + o_fix_blk[1], fix_blk[1].data(), fix_blk[1].size() * 4)) ||
       (rc = up(P->d_jobs, jobs.data(), jobs.size() * sizeof(PassJob))) ||
       (rc = up(P->d_blk, blk.data(), blk.size() * 4)) ||
       (rc = up(P->d_fin, fin.data(), n * sizeof(FinJob)))) {
@@ -2465,9 +2500,11 @@ int fv_fuse_commit(void* fv, const std::vector<uint32_t>& prods,
   P->fused = true;
   P->fbase = fbase;
   P->d_fix = reinterpret_cast<FixJob*>(fbase + o_fix);
-  P->d_fix_blk = reinterpret_cast<uint32_t*>(fbase + o_fix_blk);
   P->n_fix = (uint32_t)prods.size();
-  P->n_fix_rows = rows;
+  for (int g = 0; g < 2; g++) {
+    P->d_fix_blk[g] = reinterpret_cast<uint32_t*>(fbase + o_fix_blk[g]);
+    P->n_fix_rows[g] = fix_rows_of[g];
+  }
   return POTS_E_OK;
 }
 
@@ -2614,10 +2651,19 @@ static int run_stage(FvPlan* P, int stage, const uint8_t* d_key, double* d_rows,
     case POTS_FV_STAGE_P_FUSED:
       if (P->fused) {
         if (P->n_fix == 0) return POTS_E_HIP;  // a fusion that failed half way
-        const auto kernel = P->k == 1 ? fused_rows<1> : P->k == 2 ? fused_rows<2> : fused_rows<4>;
-        hipLaunchKernelGGL(kernel, dim3((uint32_t)((P->n_fix_rows + kFixRows - 1) / kFixRows)),
-                           dim3(256), 0, s, P->d_fix, P->d_fix_blk, P->n_fix_rows);
-        POTS_HIP(hipGetLastError());
+        for (int g = 0; g < 2; g++) {
+          if (P->n_fix_rows[g] == 0) continue;
+          const auto kernel = g == 0 ? (P->k == 1   ? fused_rows<1, kFixWaves[0]>
+                                        : P->k == 2 ? fused_rows<2, kFixWaves[0]>
+                                                    : fused_rows<4, kFixWaves[0]>)
+                                     : (P->k == 1   ? fused_rows<1, kFixWaves[1]>
+                                        : P->k == 2 ? fused_rows<2, kFixWaves[1]>
+                                                    : fused_rows<4, kFixWaves[1]>);
+          const uint32_t per = fix_rows(kFixWaves[g]);
+          hipLaunchKernelGGL(kernel, dim3((uint32_t)((P->n_fix_rows[g] + per - 1) / per)),
+                             dim3(256), 0, s, P->d_fix, P->d_fix_blk[g], P->n_fix_rows[g]);
+          POTS_HIP(hipGetLastError());
+        }
       }
       return POTS_E_OK;
     case 5:

@@ -91,3 +91,26 @@ def test_wide_products_under_few_and_many_challenges(lib, dtype, k):
     for m, prod in enumerate(prods, 1):
         _check(rows[m - 1], prod, m, k)
     plan.close()
+
+@pytest.mark.parametrize("k", [1, 2, 4])
+def test_fused_rows_short_and_long_match_oracle(lib, k):
+    """A plan of rows of few and of many records, either side of the line between them (48 slots),
+    whose products are not in that order."""
+    from verification.commitment import native
+    # (rows in whole waves of a period, so that no class is padded and all are fused)
+    shapes = [(64, 24576), (64, 512), (64, 24064), (192, 2048), (64, 40960), (320, 1024)]
+    prods = [_product(n, 16, w, torch.bfloat16, False, 20 + i) for i, (n, w) in enumerate(shapes)]
+    fv = lib.fv_plan([native.FvProduct(a, b, p, m, bv)
+                      for m, (a, b, p, bv) in enumerate(prods, 1)], k)
+    ps = [prod[2] for prod in prods]
+    leaf = lib.leaf_plan([O.tensor_leaf_header(3, p) for p in ps], ps,
+                         [native.KIND_BF16] * len(ps), fuse=fv)
+    assert leaf.fused == 6
+    key = torch.tensor(list(ROOT), dtype=torch.uint8, device=DEV)
+    digests = torch.empty(len(ps), 32, dtype=torch.uint8, device=DEV)
+    bad = torch.empty(1, dtype=torch.int32, device=DEV)
+    rows = torch.empty(len(ps), 5 + k, dtype=torch.float64, device=DEV)
+    lib.step_run(leaf, fv, key, digests, bad, rows)
+    for m, prod in enumerate(prods, 1):
+        _check(rows.cpu().tolist()[m - 1], prod, m, k)
+    fv.close()
