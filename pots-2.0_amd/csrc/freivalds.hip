@@ -1143,7 +1143,7 @@ struct RedJob {
   uint64_t pdot, pabs, psq;  // the B job's partials
   uint64_t vout;             // packed B·R for the A pass
   uint64_t u, w;             // b1 = |B|·1 and b2 = B²·1, fp32 [q]
-  uint32_t blk_first;        // prefix of kRedRows-row blocks over the jobs before it
+  uint32_t blk_first;        // prefix of red_rows(k)-row blocks over the jobs before it
   uint32_t rows, rows_pad;   // q and its padding
   uint32_t n_chunks, a_dt;   // the A pass's dtype decides the packing
   uint32_t u_slots;          // 1: also pack b1's three bf16 terms into slots 12..14 (a
@@ -1151,16 +1151,21 @@ struct RedJob {
 };
 static_assert(sizeof(RedJob) == 72, "RedJob layout");
 
-constexpr uint32_t kRedRows = 32;  // rows of B a block reduces (a packed K-step of bf16)
+// Rows of B a block reduces: packed K-steps of bf16, as many as leave a thread for each of their
+// k values and one for each row's |B|·1. (8000 biased products of 100 rows, k = 1 and 2, with 32
+// rows a block / these, us: 110, 111 / 74, 88.)
+__host__ __device__ constexpr uint32_t red_rows(uint32_t k) {
+  return k >= 4 ? 32 : 256 / (32 * (k + 1)) * 32;
+}
 
-// A block adds kRedRows rows' partials over the column chunks: a thread per value, so a chunk's
+// A block adds red_rows(k) rows' partials over the column chunks: a thread per value, so a chunk's
 // values of the block's rows are one contiguous read, four chunks' reads in flight, then packs
 // them from LDS eight rows at a time. (A thread per eight-row group and challenge read its rows
 // one by one: 107 us for a 1536 x 151936 B of 38 chunks, k = 4, against 10, and 12 us for a
 // 4096 x 4096 one of four, k = 8, against 5.) Sums in fp64, in chunk order.
 __device__ __forceinline__ void reduce_rows(const RedJob* __restrict__ jobs, uint32_t n_jobs,
                                             uint32_t k, float* s_red) {
-  // s_red: [kRedRows][k], then |B|·1's kRedRows
+  // s_red: [rows][k], then |B|·1's rows
   uint32_t lo = 0, hi = n_jobs - 1;
   while (lo < hi) {
     const uint32_t mid = (lo + hi + 1) >> 1;
@@ -1168,8 +1173,10 @@ __device__ __forceinline__ void reduce_rows(const RedJob* __restrict__ jobs, uin
     else hi = mid - 1;
   }
   const RedJob J = jobs[lo];
-  const uint32_t r0 = (blockIdx.x - J.blk_first) * kRedRows, nv = kRedRows * k;
-  const uint32_t live = min(kRedRows, J.rows - r0);  // rows past the matrix: zero
+  // (the packed outputs end at the next multiple of 32 rows)
+  const uint32_t r0 = (blockIdx.x - J.blk_first) * red_rows(k);
+  const uint32_t rows = min(red_rows(k), (J.rows + 31) / 32 * 32 - r0), nv = rows * k;
+  const uint32_t live = min(rows, J.rows - r0);  // rows past the matrix: zero
   float* const s_abs = s_red + nv;
   const float* pdot = reinterpret_cast<const float*>(J.pdot) + (uint64_t)r0 * k;
   const uint64_t cstride = (uint64_t)J.rows_pad * k;
@@ -1187,8 +1194,8 @@ __device__ __forceinline__ void reduce_rows(const RedJob* __restrict__ jobs, uin
       }
     s_red[t] = (float)sum;
   }
-  if (threadIdx.x >= 256 - kRedRows) {  // the last threads, idle above at small k
-    const uint32_t e = threadIdx.x - (256 - kRedRows);
+  if (threadIdx.x >= 256 - rows) {  // the last threads, idle above at small k
+    const uint32_t e = threadIdx.x - (256 - rows);
     double a = 0.0, q = 0.0;
     if (e < live) {
       const float* pabs = reinterpret_cast<const float*>(J.pabs) + r0 + e;
@@ -1227,7 +1234,7 @@ __device__ __forceinline__ void reduce_rows(const RedJob* __restrict__ jobs, uin
                                        pl[p][4] | (uint32_t)pl[p][5] << 16,
                                        pl[p][6] | (uint32_t)pl[p][7] << 16});
   };
-  for (uint32_t t = threadIdx.x; t < kRedRows / 8 * k; t += 256) {
+  for (uint32_t t = threadIdx.x; t < rows / 8 * k; t += 256) {
     const uint32_t g = t / k, j = t - g * k;
     const uint64_t grp = r0 / 8 + g;
     float v[8];
@@ -1247,7 +1254,7 @@ __device__ __forceinline__ void reduce_rows(const RedJob* __restrict__ jobs, uin
                             __float_as_uint(v[4 * h + 2]), __float_as_uint(v[4 * h + 3])});
     }
   }
-  if (J.u_slots && threadIdx.x < kRedRows / 8) {
+  if (J.u_slots && threadIdx.x < rows / 8) {
     const uint32_t g = threadIdx.x;
     float v[8];
 #pragma unroll
@@ -2248,7 +2255,7 @@ extern "C" int pots_fv_plan_create(size_t n, const pots_fv_product* prods, uint3
     R.n_chunks = J.n_chunks;
     R.a_dt = prods[i].a_dtype;
     R.u_slots = twin_of[i] >= 0;  // a twin's |A|·b1 runs on the matrix cores
-    red_blocks += (uint32_t)(pad32(prods[i].q) / kRedRows);
+    red_blocks += (uint32_t)((pad32(prods[i].q) + red_rows(k) - 1) / red_rows(k));
   }
   P->n_red = (uint32_t)red.size();
   P->n_red_blocks = red_blocks;
@@ -2618,7 +2625,7 @@ static int run_stage(FvPlan* P, int stage, const uint8_t* d_key, double* d_rows,
     case 2:
       if (P->n_red_blocks + P->n_biased == 0) return POTS_E_OK;
       hipLaunchKernelGGL(reduce_bias, dim3(P->n_red_blocks + P->n_biased), dim3(256),
-                         P->n_red_blocks ? (kRedRows * P->k + kRedRows) * sizeof(float) : 0, s,
+                         P->n_red_blocks ? red_rows(P->k) * (P->k + 1) * sizeof(float) : 0, s,
                          P->d_red, P->n_red, P->n_red_blocks, P->d_fin, P->d_biased, P->k,
                          P->d_bout, P->d_br);
       POTS_HIP(hipGetLastError());

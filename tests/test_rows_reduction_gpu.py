@@ -114,3 +114,16 @@ def test_fused_rows_short_and_long_match_oracle(lib, k):
     for m, prod in enumerate(prods, 1):
         _check(rows.cpu().tolist()[m - 1], prod, m, k)
     fv.close()
+
+@pytest.mark.parametrize("k", [1, 2, 3, 4])
+def test_reductions_of_a_few_rows(lib, k):
+    """B of every height around the rows a block reduces at each k (128, 64, 64, 32), side by side."""
+    from verification.commitment.native import FvProduct
+    heights = (1, 31, 32, 33, 63, 64, 65, 96, 97, 127, 128, 129, 160, 257)
+    prods = [_product(9, q, 40, torch.float32, i % 3 == 0, 30 + i) for i, q in enumerate(heights)]
+    prods += [_product(9, q, 5000, torch.bfloat16, False, 50 + q) for q in (33, 65, 129)]
+    plan = lib.fv_plan([FvProduct(a, b, p, m, bv) for m, (a, b, p, bv) in enumerate(prods, 1)], k)
+    rows = plan.rows(ROOT).cpu().tolist()
+    for m, prod in enumerate(prods, 1):
+        _check(rows[m - 1], prod, m, k)
+    plan.close()
