@@ -1780,8 +1780,9 @@ static uint64_t pad32(uint64_t rows) { return (rows + 31) / 32 * 32; }
 // its A pass 28 -> 35, each chunk's partials costing more than its block hides.)
 //
 // And no further than pays: a column of a chunk is some 0.01 us of its tile's chain (0.005 in
-// bf16), a chunk 0.06 + 0.011 k us of the finish's, which adds a row's chunks one after another, so
-// halving a chunk to c columns is worth it while 20 c² (10 c²) is at least cols·(60 + 11 k). An fp32
+// bf16), a chunk 0.06 + 0.011 k us of the finish's, which adds a row's chunks one after another
+// (0.16 + 0.07 k where k is no multiple of four and it loads word by word), so halving a chunk to c
+// columns is worth it while 20 c² (10 c²) is at least cols·(60 + 11 k) (cols·(160 + 70 k)). An fp32
 // product of 100 x 16384 x 64 under 4, 16, 64 and 255 challenges, us, whole chunks / cut to 128
 // columns / this: 56, 69, 146, 1296 / 58, 88, 249, 8014 / 40, 53, 120, 1245; one of 1000 x 4096 x
 // 4096 101, 119, 245, 2463 / 64, 90, 274, 4672 / 56, 77, 169, 873.
@@ -1789,7 +1790,7 @@ constexpr uint64_t kTilesWanted = 1024;
 constexpr uint32_t kLeastF32 = 128, kLeastBf16 = 512, kLeastBf16B = 1024;
 
 static bool cut_pays(uint32_t dt, uint64_t c, uint64_t cols, uint64_t k) {
-  return (dt == DT_BF16 ? 10 : 20) * c * c >= cols * (60 + 11 * k);
+  return (dt == DT_BF16 ? 10 : 20) * c * c >= cols * (k % 4 ? 160 + 70 * k : 60 + 11 * k);
 }
 
 static uint32_t chunk_cols_for(uint32_t cols, uint32_t sstep, uint32_t cmax) {
