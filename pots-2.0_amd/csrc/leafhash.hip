@@ -1223,31 +1223,35 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
   uint64_t n_short = 0;
   for (size_t i = 0; i < n; i++) n_short += n_nodes[i] >= 2 && n_nodes[i] <= kShortNodes;
   const uint32_t short_most = n_short >= kShortLeast ? kShortNodes : 0;
+  std::vector<uint32_t> live[2];  // leaves of two nodes and more: level_kernel's, level_lanes'
+  for (size_t i = 0; i < n; i++)
+    if (n_nodes[i] >= 2) live[n_nodes[i] <= short_most].push_back((uint32_t)i);
   uint64_t cv1_need = 0;
   int in_buf = 0;
-  for (bool more = true; more;) {
+  while (!live[0].empty() || !live[1].empty()) {
     uint64_t out_next = 0;
-    more = false;
     for (const bool lanes : {false, true}) {
+      if (live[lanes].empty()) continue;
       const uint32_t fold = lanes ? kLaneFold : kFold;
-      LevelInfo li{ents.size(), 0, 0, blk_ent.size(), in_buf, 1 - in_buf, lanes};
-      for (size_t i = 0; i < n; i++) {
-        if (n_nodes[i] < 2 || (desc[i].n_chunks <= short_most) != lanes) continue;
+      LevelInfo li{ents.size(), (uint32_t)live[lanes].size(), 0, blk_ent.size(), in_buf,
+                   1 - in_buf, lanes};
+      size_t left = 0;
+      for (uint32_t i : live[lanes]) {
         const uint64_t nout = (n_nodes[i] + (1u << fold) - 1) >> fold;
         LevelEntry e;
         e.in_off = off[i];
         e.out_off = out_next;
         e.out_first = li.n_out;
         e.n_in = (uint32_t)n_nodes[i];
-        e.leaf = (uint32_t)i;
+        e.leaf = i;
         ents.push_back(e);
         li.n_out += nout;
-        li.n_ents++;
         off[i] = out_next;
         n_nodes[i] = nout;
         out_next += nout;
+        if (nout >= 2) live[lanes][left++] = i;
       }
-      if (li.n_ents == 0) continue;
+      live[lanes].resize(left);
       if (li.n_out >= 0x7FFFFFFFull) {
         delete P;
         return POTS_E_ARG;
@@ -1260,7 +1264,6 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
       }
       if (lanes) blk_ent.push_back(li.n_ents - 1);
       P->levels.push_back(li);
-      more = true;
     }
     if (in_buf == 0) cv1_need = std::max(cv1_need, out_next);
     in_buf = 1 - in_buf;
