@@ -8,9 +8,9 @@
 // plan of few chunks, four) compresses one chunk (up to 16 blocks) and writes its chaining
 // value, or the digest itself when the leaf is a single chunk. The chunk CVs of a leaf form
 // BLAKE3's tree, which has the RFC 6962 shape (a run of n > 1 chunks splits at the largest
-// power of two below n), so it is reduced level by level, ten levels a launch: level l+1 node j
-// is the parent of level-l nodes 2j and 2j+1, or node 2j itself when it has no sibling. The
-// node that covers the whole leaf gets the ROOT flag.
+// power of two below n), so it is reduced level by level, ten levels a launch (three, where a plan
+// holds many short leaves): level l+1 node j is the parent of level-l nodes 2j and 2j+1, or node
+// 2j itself when it has no sibling. The node that covers the whole leaf gets the ROOT flag.
 //
 // Message layout in HBM. The 0x00 prefix and the tensor header are 4(1 + ndim) bytes, a whole
 // number of words, so message word w of a leaf is payload word w - H/4 and no byte shifting is
