@@ -835,19 +835,21 @@ __global__ __launch_bounds__(kThreads) void level_lanes(
 // after it. (Two device copies per leaf and the reset, each a launch of its own, were 17 launches
 // and about 80 us for eight records.)
 struct StageJob {
-  uint64_t dst;      // the staged message, 16-byte aligned, with room to a multiple of 16 bytes
-  uint64_t head;     // device address of the head bytes in the metadata region
-  uint64_t payload;  // device address of the payload, at any alignment
-  uint64_t head_bytes;
-  uint64_t to;        // message bytes to write
-  uint64_t blk_first;  // prefix of blocks over the jobs before it
+  uint64_t payload;    // device address of the payload, at any alignment
+  uint32_t leaf;       // whose descriptor holds where the message goes (16-byte aligned, with room
+                       // to a multiple of 16 bytes), its bytes and those of its head
+  uint32_t head_word;  // first word of the head bytes in the head table
+  uint32_t blk_first;  // prefix of blocks over the jobs before it
+  uint32_t host;       // the payload is in host memory: only the head is written
 };
-static_assert(sizeof(StageJob) == 48, "StageJob layout");
+static_assert(sizeof(StageJob) == 24, "StageJob layout");
 constexpr uint32_t kStageBytes = 16 * kThreads;  // of a message, per block
 
 __global__ __launch_bounds__(kThreads) void stage_kernel(const StageJob* __restrict__ jobs,
-                                                         uint32_t n_jobs, uint32_t* first_bad,
-                                                         uint32_t n_leaves) {
+                                                         uint32_t n_jobs,
+                                                         const LeafDesc* __restrict__ leaves,
+                                                         const uint32_t* __restrict__ head_table,
+                                                         uint32_t* first_bad, uint32_t n_leaves) {
   if (blockIdx.x == 0 && threadIdx.x == 0) *first_bad = n_leaves;
   if (n_jobs == 0) return;
   uint32_t lo = 0, hi = n_jobs - 1;
@@ -857,14 +859,16 @@ __global__ __launch_bounds__(kThreads) void stage_kernel(const StageJob* __restr
     else hi = mid - 1;
   }
   const StageJob J = jobs[lo];
-  const uint64_t m0 = (blockIdx.x - J.blk_first) * kStageBytes + 16ull * threadIdx.x;
-  if (m0 >= J.to) return;
-  const char* head = reinterpret_cast<const char*>(J.head);
+  const LeafDesc d = leaves[J.leaf];
+  const uint64_t head_bytes = d.fin_from, to = J.host ? head_bytes : d.len;
+  const uint64_t m0 = (uint64_t)(blockIdx.x - J.blk_first) * kStageBytes + 16ull * threadIdx.x;
+  if (m0 >= to) return;
+  const char* head = reinterpret_cast<const char*>(head_table + J.head_word);
   const char* payload = reinterpret_cast<const char*>(J.payload);
   u32x4 v = {0, 0, 0, 0};
-  if (m0 >= J.head_bytes && m0 + 16 <= J.to) {
+  if (m0 >= head_bytes && m0 + 16 <= to) {
     // the aligned words the sixteen bytes lie in, none of them past the payload's last
-    const uint64_t src = J.payload + (m0 - J.head_bytes);
+    const uint64_t src = J.payload + (m0 - head_bytes);
     const char* at = reinterpret_cast<const char*>(src & ~uint64_t(3));
     const uint32_t sh = 8 * (uint32_t)(src & 3);
     const u32x4 w = gload<u32x4w>(at);
@@ -880,12 +884,12 @@ __global__ __launch_bounds__(kThreads) void stage_kernel(const StageJob* __restr
     for (uint32_t t = 0; t < 16; t++) {
       const uint64_t m = m0 + t;
       uint32_t byte = 0;
-      if (m < J.head_bytes) byte = gload<uint8_t>(head + m);
-      else if (m < J.to) byte = gload<uint8_t>(payload + (m - J.head_bytes));
+      if (m < head_bytes) byte = gload<uint8_t>(head + m);
+      else if (m < to) byte = gload<uint8_t>(payload + (m - head_bytes));
       v[t / 4] |= byte << (8 * (t % 4));
     }
   }
-  gstore<u32x4>(reinterpret_cast<char*>(J.dst) + m0, v);
+  gstore<u32x4>(reinterpret_cast<char*>(d.payload) + m0, v);
 }
 
 // ---- host side ----------------------------------------------------------------------------
@@ -1093,7 +1097,7 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
   std::vector<int64_t> stage_head_at(n, -1);
   uint64_t stage_bytes = 0, stage_blocks = 0;
   std::vector<uint64_t> stage_off(n, 0);
-  std::vector<StageJob> stages;  // offsets until the plan's memory is placed
+  std::vector<StageJob> stages;
   std::vector<FuseDesc> fdesc;                 // per fused leaf
   std::vector<uint32_t> fprod, fhead;          // its product and head bytes
   std::unordered_set<uint32_t> fused_prods;
@@ -1136,7 +1140,8 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
       d.head_word = 0;
       d.head_len = 0;
       const uint64_t to = host ? hl : hl + len;
-      stages.push_back(StageJob{stage_off[i], at, ptr, hl, to, stage_blocks});
+      stages.push_back(StageJob{ptr, (uint32_t)i, (uint32_t)(at / 4), (uint32_t)stage_blocks,
+                                host ? 1u : 0u});
       stage_blocks += (to + kStageBytes - 1) / kStageBytes;
       if (host) P->host_copies.push_back(HostCopy{stage_off[i] + hl, ptr, len});
     }
@@ -1248,8 +1253,10 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
         li.n_out += nout;
         off[i] = out_next;
         n_nodes[i] = nout;
-        out_next += nout;
-        if (nout >= 2) live[lanes][left++] = i;
+        if (nout >= 2) {  // (a leaf that closes writes its digest and nothing else)
+          out_next += nout;
+          live[lanes][left++] = i;
+        }
       }
       live[lanes].resize(left);
       if (li.n_out >= 0x7FFFFFFFull) {
@@ -1288,10 +1295,13 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
   const size_t o_head = place(std::max<size_t>(headbytes.size(), 4));
   const size_t o_lev = place(std::max<size_t>(ents.size(), 1) * sizeof(LevelEntry));
   const size_t o_blk_ent = place(std::max<size_t>(blk_ent.size(), 1) * sizeof(uint32_t));
-  const size_t o_stages = place(std::max<size_t>(stages.size(), 1) * sizeof(StageJob));
+  // The staging jobs last: a call that runs once, in memory it must fit, has them where its chunk
+  // kernels then put the chaining values, which take more (32 bytes a chunk).
+  const size_t o_stages = at, stages_bytes = stages.size() * sizeof(StageJob);
+  if (!ext_base) place(stages_bytes);
   // A synchronous call's results: the first-bad word, uploaded with the metadata as n, and the
   // digests behind it, so that one copy brings both back.
-  size_t o_bad = 0, meta_bytes = at;
+  size_t o_bad = 0, meta_bytes = o_stages + stages_bytes;
   if (pinned) {
     o_bad = place(kResultHead + 32 * n);
     meta_bytes = o_bad + kResultHead;
@@ -1330,10 +1340,6 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
   const uint64_t B = reinterpret_cast<uint64_t>(P->base);
   for (size_t i = 0; i < n; i++)
     if (stage_head_at[i] >= 0) desc[i].payload = B + o_stage + stage_off[i];
-  for (StageJob& j : stages) {
-    j.dst += B + o_stage;
-    j.head += B + o_head;
-  }
   for (HostCopy& c : P->host_copies) c.dst += B + o_stage;
   P->d_stages = reinterpret_cast<StageJob*>(P->base + o_stages);
   P->n_stages = (uint32_t)stages.size();
@@ -1382,8 +1388,7 @@ static int plan_build(size_t n, const uint8_t* hdr_buf, const uint64_t* hdr_off,
     memcpy(img.data() + o_ord[k][2], ords[k]->blk_ent.data(),
            ords[k]->blk_ent.size() * sizeof(uint32_t));
   }
-  if (!stages.empty())
-    memcpy(img.data() + o_stages, stages.data(), stages.size() * sizeof(StageJob));
+  if (!stages.empty()) memcpy(img.data() + o_stages, stages.data(), stages_bytes);
   if (!headbytes.empty()) memcpy(img.data() + o_head, headbytes.data(), headbytes.size());
   if (!ents.empty()) memcpy(img.data() + o_lev, ents.data(), ents.size() * sizeof(LevelEntry));
   if (!blk_ent.empty())
@@ -1418,7 +1423,8 @@ static int plan_stage(LeafPlan* P, int stage, uint32_t* d_digests, uint32_t* d_f
   switch (stage) {
     case 0:
       hipLaunchKernelGGL(stage_kernel, dim3(std::max(1u, P->stage_blocks)), dim3(kThreads), 0,
-                         stream, P->d_stages, P->n_stages, d_first_bad, (uint32_t)P->n);
+                         stream, P->d_stages, P->n_stages, P->d_leaves, P->d_head, d_first_bad,
+                         (uint32_t)P->n);
       for (const HostCopy& c : P->host_copies)
         POTS_HIP(hipMemcpyAsync(reinterpret_cast<void*>(c.dst), reinterpret_cast<const void*>(c.src),
                                 c.bytes, hipMemcpyHostToDevice, stream));
@@ -1613,11 +1619,14 @@ extern "C" size_t pots_hash_leaves_noalloc(size_t n, const uint8_t* hdr_buf,
                std::to_string(kNoallocScratchBytes));
     return SIZE_MAX;
   }
+  // In runs of kRun, whose tables are the smallest, where the plan's own cut does not fit.
   LeafPlan* P = nullptr;
-  if (plan_build(n, hdr_buf, hdr_off, hdr_len, hdr_idx, payload_ptr, payload_len, kind,
-                 /*device_only=*/false, /*owned=*/false, nullptr, &P, base + res_bytes,
-                 kNoallocScratchBytes - res_bytes) != POTS_E_OK)
-    return SIZE_MAX;
+  int rc = POTS_E_ARG;
+  for (uint32_t run = 0; run <= kRun && rc == POTS_E_ARG; run += kRun)
+    rc = plan_build(n, hdr_buf, hdr_off, hdr_len, hdr_idx, payload_ptr, payload_len, kind,
+                    /*device_only=*/false, /*owned=*/false, nullptr, &P, base + res_bytes,
+                    kNoallocScratchBytes - res_bytes, nullptr, run);
+  if (rc != POTS_E_OK) return SIZE_MAX;
   uint32_t* d_dig = reinterpret_cast<uint32_t*>(base);
   uint32_t* d_bad = reinterpret_cast<uint32_t*>(base + 32 * n);
   size_t bad = SIZE_MAX;

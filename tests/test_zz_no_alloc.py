@@ -82,3 +82,31 @@ def test_noalloc_refuses_more_than_its_scratch(lib):
     want, _ = _call(lib, "pots_hash_leaves", leaves, _kinds(leaves))
     got, bad = _call(lib, "pots_hash_leaves_noalloc", leaves, _kinds(leaves))
     assert bad == 2 and np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("n, header, payload", [
+    (453312, 5, 0),      # messages that are headers alone: all staged
+    (34584, 900, 0),
+    (270528, 11, 100),   # host payloads
+    (129024, 11, 9000),  # nine chunks each, in device memory
+    (17580, 11, 102000),
+    (289152, 11, 1500)])
+def test_noalloc_takes_what_fits_its_scratch(lib, n, header, payload):
+    """As many leaves of a kind as the tables of runs of four chunks leave room for, to the plan's
+    alignment: no table for staging or shorter runs may cost a leaf of them."""
+    g = torch.Generator().manual_seed(n)
+    data = torch.randint(0, 256, (max(payload, 1),), generator=g, dtype=torch.uint8)
+    where = data.cuda() if payload > 1000 else data
+    heads = [bytes([i & 255, i >> 8 & 255, i >> 16]) + b"x" * (header - 3) for i in range(3)]
+    hb = np.frombuffer(b"".join(heads), dtype=np.uint8)
+    hlen = np.full(3, header, np.uint32)
+    hoff = np.arange(3, dtype=np.uint64) * header
+    hidx = (np.arange(n) % 3).astype(np.uint32)
+    ptr = np.full(n, where.data_ptr() if payload else 0, np.uint64)
+    ln, kd = np.full(n, payload, np.uint64), np.zeros(n, np.uint8)
+    out = np.zeros((n, 32), dtype=np.uint8)
+    addr = [a.ctypes.data for a in (hb, hoff, hlen, hidx, ptr, ln, kd, out)]
+    assert lib._lib.pots_hash_leaves_noalloc(n, *map(ctypes.c_void_p, addr), 1) == n
+    want = np.array([np.frombuffer(O.hash_leaf(h + bytes(data.numpy())[:payload]), np.uint8)
+                     for h in heads])
+    assert np.array_equal(out, want[hidx])
