@@ -1,5 +1,5 @@
 // A driver for the sanitized CPU build of libpots_mi355x's host code (host_model.cpp stands in
-// for the HIP runtime). Two modes:
+// for the HIP runtime). Three modes:
 //
 //   host_check scan FILE...   pots_store_scan over the files (the untrusted prover files of an
 //                             on-disk transcript); one line per file with what the scan found,
@@ -10,6 +10,8 @@
 //                             twins, k, guard) and leaf plans over their P (fused and not) and
 //                             other leaves, each built and destroyed; the twin count and the
 //                             refusals are checked against what the generator made.
+//   host_check pinned         pots_hash_leaves with and without pinned memory to be had, launches
+//                             succeeding and doing nothing: it returns the number of leaves.
 //
 // Exit status 0 when every result is as expected; the sanitizers abort on any finding.
 
@@ -265,10 +267,36 @@ int plans(uint64_t seed, int count) {
 
 }  // namespace
 
+extern "C" void host_model_set(int pinned, int launches);
+
+namespace {
+
+int pinned() {
+  const uint8_t hdr[] = "abcdefgh";
+  const uint64_t off[] = {0, 3, 0}, zero[] = {0, 0, 0};
+  const uint32_t len[] = {3, 5, 8}, idx[] = {0, 1, 2};
+  const uint8_t kind[] = {0, 0, 0};
+  for (const int have : {0, 0, 1, 1, 0}) {
+    host_model_set(have, 1);
+    uint8_t out[96];
+    const size_t bad = pots_hash_leaves(3, hdr, off, len, idx, zero, zero, kind, out, 1);
+    if (bad != 3) {
+      fprintf(stderr, "pots_hash_leaves %s pinned memory: %zu, %s\n", have ? "with" : "without",
+              bad, pots_last_error());
+      return 1;
+    }
+  }
+  printf("pinned ok\n");
+  return 0;
+}
+
+}  // namespace
+
 int main(int argc, char** argv) {
+  if (argc == 2 && !strcmp(argv[1], "pinned")) return pinned();
   if (argc >= 2 && !strcmp(argv[1], "scan")) return scan(argc, argv);
   if (argc == 4 && !strcmp(argv[1], "plans"))
     return plans(strtoull(argv[2], nullptr, 10), atoi(argv[3]));
-  fprintf(stderr, "usage: host_check scan FILE... | host_check plans SEED COUNT\n");
+  fprintf(stderr, "usage: host_check scan FILE... | plans SEED COUNT | pinned\n");
   return 2;
 }

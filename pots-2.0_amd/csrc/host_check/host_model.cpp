@@ -1,7 +1,8 @@
 // A host model of the HIP runtime calls that libpots_mi355x's host code makes, for a CPU-only
 // build of that code under AddressSanitizer and UndefinedBehaviorSanitizer (no GPU, no HIP
 // runtime): device memory is host memory from malloc, copies and fills are memcpy and memset,
-// streams and events are complete as soon as they are made, and a kernel launch fails. The
+// streams and events are complete as soon as they are made, and a kernel launch fails
+// (host_model_set makes it succeed, doing nothing). The
 // plan builders and the store reader run on it unchanged, every host-side access checked.
 //
 // Pointer attributes report memory from hipMalloc as device memory and anything else as
@@ -31,6 +32,7 @@ State& state() {
 }
 
 thread_local hipError_t g_last = hipSuccess;
+bool g_pinned = true, g_launches = false;
 int g_event_tag, g_stream_tag;
 
 hipError_t set(hipError_t e) {
@@ -76,8 +78,14 @@ hipError_t hipFree(void* ptr) {
 
 hipError_t hipHostMalloc(void** ptr, size_t size, unsigned int) {
   if (!ptr) return set(hipErrorInvalidValue);
-  *ptr = malloc(size ? size : 1);
+  *ptr = g_pinned ? malloc(size ? size : 1) : nullptr;
   return *ptr ? hipSuccess : set(hipErrorOutOfMemory);
+}
+
+// Whether pinned memory is to be had (yes), and whether launches succeed, doing nothing (no).
+void host_model_set(int pinned, int launches) {
+  g_pinned = pinned != 0;
+  g_launches = launches != 0;
 }
 
 hipError_t hipHostFree(void* ptr) {
@@ -160,7 +168,7 @@ hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
 
 hipError_t hipLaunchKernel(const void*, dim3, dim3, void**, size_t, hipStream_t) {
-  return set(hipErrorNoDevice);
+  return g_launches ? hipSuccess : set(hipErrorNoDevice);
 }
 
 hipError_t hipGetSymbolAddress(void** dev_ptr, const void* symbol) {

@@ -1529,7 +1529,10 @@ extern "C" size_t pots_hash_leaves(size_t n, const uint8_t* hdr_buf, const uint6
   static std::mutex mu;
   std::lock_guard<std::mutex> lock(mu);
   void* pinned = nullptr;
-  if (pinned_get(0, 2 * kPinnedBytes, &pinned) != POTS_E_OK) pinned = nullptr;
+  if (pinned_get(0, 2 * kPinnedBytes, &pinned) != POTS_E_OK) {
+    pinned = nullptr;
+    (void)hipGetLastError();  // pageable copies instead: the next launch's check is not to see it
+  }
   LeafPlan* P = nullptr;
   void* res = nullptr;
   size_t bad = SIZE_MAX;

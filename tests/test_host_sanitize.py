@@ -11,6 +11,7 @@ at their first finding:
   changed in the archive and in the pickle of two tensors, 300 files each) and the files the
   scan must leave to torch.load; every file's outcome must equal the production library's,
   and every storage the scan takes must load to the file's own bytes;
+- ``pots_hash_leaves`` where the system has no pinned memory to give;
 - 300 randomized Freivalds plans (shapes, strides, dtypes, biases, twins, k, guard) and the
   leaf plans over their products, fused and not, with the refusals the generator expects.
 """
@@ -144,6 +145,10 @@ def test_plan_builders_are_clean_under_sanitizers(driver):
     assert out.startswith("plans ok: 300")
     twins, fused = (int(x) for x in out.split("(")[1].split()[0:4:2])
     assert twins > 0 and fused > 0  # the generator reached the twin pass and the fusion
+
+
+def test_hash_leaves_without_pinned_memory(driver):
+    assert _run(driver, "pinned") == "pinned ok\n"
 
 
 def test_sanitizers_are_live_in_the_driver(driver):
