@@ -1439,6 +1439,72 @@ __device__ __forceinline__ void chunk_sums(const float* __restrict__ abs_,
   }
 }
 
+// A pass's partials of many column chunks, added up for the rows (which then find one chunk): a
+// block takes 32 values, a row's dot product, Σ|x|u or Σx²w each, eight threads a value adding every
+// eighth chunk, four loads in flight, then the eight in order; all in fp64, rounded to the partials'
+// formats as the finish rounds its own sums. The finish's threads take a row each and its chunks one
+// after another, k values of them: an fp32 product of 100 x 16384 x 64, whose 128 chunks are there
+// for the A pass's sake, took 33, 58, 200 and 8034 us there under 4, 16, 64 and 255 challenges (16
+// whole chunks 19, 29, 85 and 742), and 17, 24, 58 and 361 with this.
+constexpr uint32_t kAddValues = 32, kAddGroups = 256 / kAddValues;
+
+struct AddJob {
+  uint64_t dot, abs, sq;     // the pass's partials, [chunks][rows_pad] (x k)
+  uint64_t odot, oabs, osq;  // their sums, [rows] (x k)
+  uint32_t rows, rows_pad, chunks;
+  uint32_t blk_first;        // prefix of blocks over the jobs before it
+};
+static_assert(sizeof(AddJob) == 64, "AddJob layout");
+
+template <typename T>
+__device__ __forceinline__ double add_every(const T* p, uint64_t stride, uint32_t c,
+                                            uint32_t chunks) {
+  double sum = 0.0;
+  for (; c < chunks; c += 4 * kAddGroups) {
+    T x[4];
+#pragma unroll
+    for (uint32_t t = 0; t < 4; t++)
+      x[t] = gload<T>(p + min(c + t * kAddGroups, chunks - 1) * stride);
+#pragma unroll
+    for (uint32_t t = 0; t < 4; t++)
+      if (c + t * kAddGroups < chunks) sum += (double)x[t];
+  }
+  return sum;
+}
+
+__global__ __launch_bounds__(256) void add_chunks(const AddJob* __restrict__ jobs,
+                                                  uint32_t n_jobs, uint32_t k) {
+  __shared__ double s_sum[kAddGroups][kAddValues];
+  uint32_t lo = 0, hi = n_jobs - 1;
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi + 1) >> 1;
+    if (jobs[mid].blk_first <= blockIdx.x) lo = mid;
+    else hi = mid - 1;
+  }
+  const AddJob J = jobs[lo];
+  const uint32_t lane = threadIdx.x % kAddValues, group = threadIdx.x / kAddValues;
+  const uint64_t v = (uint64_t)(blockIdx.x - J.blk_first) * kAddValues + lane;
+  const uint64_t dots = (uint64_t)J.rows * k, abss = dots + J.rows, end = abss + J.rows;
+  double sum = 0.0;
+  if (v < dots)
+    sum = add_every(reinterpret_cast<const float*>(J.dot) + v, (uint64_t)J.rows_pad * k, group,
+                    J.chunks);
+  else if (v < abss)
+    sum = add_every(reinterpret_cast<const float*>(J.abs) + (v - dots), J.rows_pad, group,
+                    J.chunks);
+  else if (v < end)
+    sum = add_every(reinterpret_cast<const double*>(J.sq) + (v - abss), J.rows_pad, group,
+                    J.chunks);
+  s_sum[group][lane] = sum;
+  __syncthreads();
+  if (group || v >= end) return;
+#pragma unroll
+  for (uint32_t g = 1; g < kAddGroups; g++) sum += s_sum[g][lane];
+  if (v < dots) gstore<float>(reinterpret_cast<float*>(J.odot) + v, (float)sum);
+  else if (v < abss) gstore<float>(reinterpret_cast<float*>(J.oabs) + (v - dots), (float)sum);
+  else gstore<double>(reinterpret_cast<double*>(J.osq) + (v - abss), sum);
+}
+
 // The sum of record column `col` as its column of the row.
 __device__ __forceinline__ void put_column(double* row, uint32_t col, double sum,
                                            uint32_t guard) {
@@ -1734,6 +1800,10 @@ struct FvPlan {
   RedJob* d_red = nullptr;
   uint32_t n_red = 0;
   uint32_t n_red_blocks = 0;
+  AddJob* d_add = nullptr;
+  std::vector<AddJob> h_add;
+  std::vector<uint32_t> add_src;  // of each: n + product (A) or 2 n + product (P)
+  uint32_t n_add_blocks = 0;
   FinJob* d_fin = nullptr;
   SliceJob* d_slices = nullptr;
   uint32_t n_slices = 0;
@@ -1778,19 +1848,14 @@ static uint64_t pad32(uint64_t rows) { return (rows + 31) / 32 * 32; }
 // 12, 14, 12 / 11, 9, 10; of eight 1000 x 2050 x 1537 bf16 ones under sixteen challenges 49, 30,
 // 33 / 45, 24, 24; the B pass of an 8192 x 4096 x 4096 fp32 one 25 / 17. (2048 tiles wanted:
 // its A pass 28 -> 35, each chunk's partials costing more than its block hides.)
-//
-// And no further than pays: a column of a chunk is some 0.01 us of its tile's chain (0.005 in
-// bf16), a chunk 0.06 + 0.011 k us of the finish's, which adds a row's chunks one after another
-// (0.16 + 0.07 k where k is no multiple of four and it loads word by word), so halving a chunk to c
-// columns is worth it while 20 c² (10 c²) is at least cols·(60 + 11 k) (cols·(160 + 70 k)). An fp32
-// product of 100 x 16384 x 64 under 4, 16, 64 and 255 challenges, us, whole chunks / cut to 128
-// columns / this: 56, 69, 146, 1296 / 58, 88, 249, 8014 / 40, 53, 120, 1245; one of 1000 x 4096 x
-// 4096 101, 119, 245, 2463 / 64, 90, 274, 4672 / 56, 77, 169, 873.
 constexpr uint64_t kTilesWanted = 1024;
 constexpr uint32_t kLeastF32 = 128, kLeastBf16 = 512, kLeastBf16B = 1024;
 
-static bool cut_pays(uint32_t dt, uint64_t c, uint64_t cols, uint64_t k) {
-  return (dt == DT_BF16 ? 10 : 20) * c * c >= cols * (k % 4 ? 160 + 70 * k : 60 + 11 * k);
+// Whether a pass's chunks are added up ahead of the rows (add_chunks): by the time that a row's
+// chain over them would take there, 0.06 + 0.011 k us a chunk, or 0.16 + 0.07 k where k is no
+// multiple of four and the finish loads word by word, against a launch and the chunks' eighth.
+static bool adds_chunks(uint64_t chunks, uint64_t k) {
+  return chunks >= 3 && chunks * (k % 4 ? 160 + 70 * k : 60 + 11 * k) > 10000;
 }
 
 static uint32_t chunk_cols_for(uint32_t cols, uint32_t sstep, uint32_t cmax) {
@@ -1919,12 +1984,7 @@ extern "C" int pots_fv_plan_create(size_t n, const pots_fv_product* prods, uint3
   // fewer than kTilesWanted tiles. A tile is a chain of stages, each a load's latency, and it
   // takes several blocks on a CU to hide one another's.
   auto chunk_most = [&](uint32_t dt, uint32_t most, uint32_t least, auto&& shape_of) {
-    uint32_t widest = 0;
-    for (size_t i = 0; i < n; i++) {
-      const Shape s = shape_of(i);
-      if (s.dt == dt) widest = std::max(widest, s.cols);
-    }
-    for (; most > least && cut_pays(dt, most / 2, widest, k); most /= 2) {
+    for (; most > least; most /= 2) {
       uint64_t tiles = 0;
       for (size_t i = 0; i < n && tiles < kTilesWanted; i++) {
         const Shape s = shape_of(i);
@@ -2137,8 +2197,35 @@ extern "C" int pots_fv_plan_create(size_t n, const pots_fv_product* prods, uint3
   // record of 4 + k sums per slice.
   // A thread of a slice adds each of its rows' partials over the chunks in order, so a
   // product with many chunks (a wide A, or a twin's many tiles) gets smaller slices.
-  std::vector<uint32_t> a_chunks(n);
-  for (size_t i = 0; i < n; i++) a_chunks[i] = jobs[n + i].n_chunks;
+  std::vector<uint32_t> a_chunks(n), p_chunks(n);
+  for (size_t i = 0; i < n; i++) {
+    a_chunks[i] = jobs[n + i].n_chunks;
+    p_chunks[i] = jobs[2 * n + i].n_chunks;
+  }
+  // The passes whose chunks are added up ahead of the rows: their sums, and one chunk for these.
+  std::vector<size_t> off_add;
+  for (size_t src = n; src < 3 * n; src++) {
+    const PassJob& J = jobs[src];
+    const uint64_t blocks =
+        ((uint64_t)J.rows * (k + 2) + kAddValues - 1) / kAddValues + P->n_add_blocks;
+    if ((src < 2 * n && twin_of[src - n] >= 0) || !adds_chunks(J.n_chunks, k) ||
+        blocks >= 0x7FFFFFFFull)
+      continue;
+    AddJob a;
+    memset(&a, 0, sizeof a);
+    a.rows = J.rows;
+    a.rows_pad = J.rows_pad;
+    a.chunks = J.n_chunks;
+    a.blk_first = P->n_add_blocks;
+    P->n_add_blocks = (uint32_t)blocks;
+    P->h_add.push_back(a);
+    P->add_src.push_back((uint32_t)src);
+    off_add.push_back(place((uint64_t)J.rows * k * 4));
+    off_add.push_back(place((uint64_t)J.rows * 4));
+    off_add.push_back(place((uint64_t)J.rows * 8));
+    (src < 2 * n ? a_chunks[src - n] : p_chunks[src - 2 * n]) = 1;
+  }
+  const size_t o_add = place(std::max<size_t>(P->h_add.size(), 1) * sizeof(AddJob));
   for (size_t t = 0; t < twins.size(); t++) {
     a_chunks[twins[t].first] = tw[t].n_ct;
     a_chunks[twins[t].second] = tw[t].n_rt;
@@ -2150,7 +2237,7 @@ extern "C" int pots_fv_plan_create(size_t n, const pots_fv_product* prods, uint3
   std::vector<SliceJob> slices;
   std::vector<uint32_t> slice_first(n), slice_rows(n), biased;
   for (size_t i = 0; i < n; i++) {
-    const uint32_t chunks = std::max(a_chunks[i], jobs[2 * n + i].n_chunks);
+    const uint32_t chunks = std::max(a_chunks[i], p_chunks[i]);
     uint32_t sr = slice_most;
     while (sr > 64 && (uint64_t)sr * chunks > 8ull * kSliceRows) sr /= 2;
     slice_rows[i] = sr;
@@ -2191,6 +2278,7 @@ extern "C" int pots_fv_plan_create(size_t n, const pots_fv_product* prods, uint3
   P->d_jobs = reinterpret_cast<PassJob*>(P->base + o_jobs);
   P->d_blk = reinterpret_cast<uint32_t*>(P->base + o_blk);
   P->d_red = reinterpret_cast<RedJob*>(P->base + o_red);
+  P->d_add = reinterpret_cast<AddJob*>(P->base + o_add);
   P->d_fin = reinterpret_cast<FinJob*>(P->base + o_fin);
   P->d_slices = reinterpret_cast<SliceJob*>(P->base + o_slices);
   P->n_slices = (uint32_t)slices.size();
@@ -2282,6 +2370,25 @@ extern "C" int pots_fv_plan_create(size_t n, const pots_fv_product* prods, uint3
     F.slice_first = slice_first[i];
     F.n_slices = (uint32_t)((prods[i].n + slice_rows[i] - 1) / slice_rows[i]);
   }
+  for (size_t a = 0; a < P->h_add.size(); a++) {
+    AddJob& D = P->h_add[a];
+    const uint32_t src = P->add_src[a];
+    const PassJob& J = ordered[pos[src]];
+    D.dot = J.pdot;
+    D.abs = J.pabs;
+    D.sq = J.psq;
+    D.odot = base + off_add[3 * a];
+    D.oabs = base + off_add[3 * a + 1];
+    D.osq = base + off_add[3 * a + 2];
+    FinJob& F = fin[src % n];
+    if (src < 2 * n) {
+      F.a_dot = D.odot, F.a_abs = D.oabs, F.a_sq = D.osq;
+      F.a_rows_pad = J.rows, F.a_chunks = 1;
+    } else {
+      F.p_dot = D.odot, F.p_abs = D.oabs, F.p_sq = D.osq;
+      F.p_rows_pad = J.rows, F.p_chunks = 1;
+    }
+  }
   std::vector<uint32_t> twin_tile(twin_tiles);
   for (size_t t = 0; t < tw.size(); t++) {
     TwinJob& T = tw[t];
@@ -2313,6 +2420,7 @@ extern "C" int pots_fv_plan_create(size_t n, const pots_fv_product* prods, uint3
   if ((rc = up(o_items, items.data(), n * sizeof(ChallengeItem))) ||
       (rc = up(o_jobs, ordered.data(), ordered.size() * sizeof(PassJob))) ||
       (rc = up(o_blk, blk_table.data(), blk_table.size() * 4)) ||
+      (rc = up(o_add, P->h_add.data(), P->h_add.size() * sizeof(AddJob))) ||
       (rc = up(o_red, red.data(), red.size() * sizeof(RedJob))) ||
       (rc = up(o_fin, fin.data(), n * sizeof(FinJob))) ||
       (rc = up(o_slices, slices.data(), slices.size() * sizeof(SliceJob))) ||
@@ -2482,7 +2590,24 @@ int fv_fuse_commit(void* fv, const std::vector<uint32_t>& prods,
     L.n_blocks = (uint32_t)blocks;
   }
   std::vector<FinJob> fin = P->h_fin;
-  for (uint32_t i : prods) fin[i].p_chunks = 1;
+  // A fused product's P has one chunk of partials, in its P job's place, and no others to add up.
+  std::vector<AddJob> add;
+  std::vector<uint32_t> add_src;
+  uint32_t add_blocks = 0;
+  for (size_t a = 0; a < P->h_add.size(); a++) {
+    const uint32_t src = P->add_src[a];
+    if (src >= 2 * n && fused[src - 2 * n]) continue;
+    const AddJob& D = P->h_add[a];
+    add.push_back(D);
+    add.back().blk_first = add_blocks;
+    add_blocks += (uint32_t)(((uint64_t)D.rows * (P->k + 2) + kAddValues - 1) / kAddValues);
+    add_src.push_back(src);
+  }
+  for (uint32_t i : prods) {
+    const PassJob& J = P->h_jobs[pos[2 * n + i]];
+    fin[i].p_dot = J.pdot, fin[i].p_abs = J.pabs, fin[i].p_sq = J.psq;
+    fin[i].p_rows_pad = J.rows_pad, fin[i].p_chunks = 1;
+  }
   auto up = [&](void* dst, const void* src, size_t bytes) -> int {
     if (!bytes) return POTS_E_OK;
     POTS_HIP(hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice));
@@ -2494,6 +2619,7 @@ int fv_fuse_commit(void* fv, const std::vector<uint32_t>& prods,
       (rc = up(fbase + o_fix_blk[1], fix_blk[1].data(), fix_blk[1].size() * 4)) ||
       (rc = up(P->d_jobs, jobs.data(), jobs.size() * sizeof(PassJob))) ||
       (rc = up(P->d_blk, blk.data(), blk.size() * 4)) ||
+      (rc = up(P->d_add, add.data(), add.size() * sizeof(AddJob))) ||
       (rc = up(P->d_fin, fin.data(), n * sizeof(FinJob)))) {
     // The device tables may be half rewritten: the plan is unusable, and says so.
     P->fused = true;
@@ -2505,6 +2631,9 @@ int fv_fuse_commit(void* fv, const std::vector<uint32_t>& prods,
   P->h_jobs = std::move(jobs);
   P->h_blk = std::move(blk);
   P->h_fin = std::move(fin);
+  P->h_add = std::move(add);
+  P->add_src = std::move(add_src);
+  P->n_add_blocks = add_blocks;
   P->fused = true;
   P->fbase = fbase;
   P->d_fix = reinterpret_cast<FixJob*>(fbase + o_fix);
@@ -2675,6 +2804,11 @@ static int run_stage(FvPlan* P, int stage, const uint8_t* d_key, double* d_rows,
       }
       return POTS_E_OK;
     case 5:
+      if (P->n_add_blocks) {
+        hipLaunchKernelGGL(add_chunks, dim3(P->n_add_blocks), dim3(256), 0, s, P->d_add,
+                           (uint32_t)P->h_add.size(), P->k);
+        POTS_HIP(hipGetLastError());
+      }
       hipLaunchKernelGGL(finish_slices, dim3(P->n_slices), dim3(256), 0, s, P->d_fin,
                          P->d_slices, P->k, P->d_bout, P->d_br, P->guard, P->d_recs, d_rows);
       POTS_HIP(hipGetLastError());

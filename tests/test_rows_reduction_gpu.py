@@ -97,8 +97,10 @@ def test_fused_rows_short_and_long_match_oracle(lib, k):
     """A plan of rows of few and of many records, either side of the line between them (48 slots),
     whose products are not in that order."""
     from verification.commitment import native
-    # (rows in whole waves of a period, so that no class is padded and all are fused)
-    shapes = [(64, 24576), (64, 512), (64, 24064), (192, 2048), (64, 40960), (320, 1024)]
+    # (rows in whole waves of a period, so that no class is padded and all are fused,
+    # but the last, whose rows fit no period); the two widest have chunks enough to be added up ahead
+    # of the rows, unless they are fused
+    shapes = [(64, 24576), (64, 512), (64, 24064), (192, 2048), (64, 65536), (320, 1024), (33, 65537)]
     prods = [_product(n, 16, w, torch.bfloat16, False, 20 + i) for i, (n, w) in enumerate(shapes)]
     fv = lib.fv_plan([native.FvProduct(a, b, p, m, bv)
                       for m, (a, b, p, bv) in enumerate(prods, 1)], k)
